@@ -5,8 +5,9 @@
 // reads 16-byte vectors (8 bf16 / 4 fp32) so a 2 KiB bf16 row is exactly two
 // dwordx4 loads per lane and every HBM line is fully used.  Cross-lane
 // combination is a 6-step butterfly.  Rows never interact, so the grid is
-// rows/4 workgroups of 4 waves — tens of thousands of waves for the C2
-// shapes, enough to keep all 256 CUs streaming.
+// rows/4 workgroups of 4 waves — tens of thousands of waves for 65536 rows,
+// enough to keep all 256 CUs streaming.  Few or long rows take 4 or 16 waves
+// each (team_waves).
 #include "mk_common.h"
 
 #include <algorithm>
@@ -54,167 +55,121 @@ template <int OP> __device__ inline float identity() {
   else return 1.f;
 }
 
+// A row of any length at any element-aligned address, shared by the W waves
+// of a team (W = 1: four rows per 256-thread workgroup; W = 4, 16: one row
+// per workgroup): 16-byte vectors t, t + 64 W, ... for team lane t, then the
+// up to N - 1 elements past the last whole vector, one per lane.  A row of
+// odd length starts off the 16-byte grid; the vector loads need element
+// alignment only (global accesses of any alignment are one instruction on
+// gfx950), so such rows keep the full load width.
+template <typename T> struct __attribute__((packed, aligned(sizeof(T)))) Unaligned16 { u32x4_t v; };
+template <typename T> __device__ inline u32x4_t ld_row(const T* p) { return reinterpret_cast<const Unaligned16<T>*>(p)->v; }
+template <typename T> __device__ inline void st_row(T* p, u32x4_t v) { reinterpret_cast<Unaligned16<T>*>(p)->v = v; }
+
+template <int W> constexpr int kTeamBlock = W > kWavesPerBlock ? W * kWave : kBlock;
+
+template <int W>
+struct Team {
+  static constexpr int kRows = kTeamBlock<W> / (W * kWave);  // rows per workgroup
+  static constexpr int kLanes = W * kWave;
+  int wave, t;
+  int64_t row;
+  __device__ inline Team() {
+    wave = int(threadIdx.x) / kWave;
+    t = int(threadIdx.x) % kLanes;
+    row = int64_t(blockIdx.x) * kRows + int(threadIdx.x) / kLanes;
+  }
+  // v, already combined over each wave, over the team's waves in wave order
+  template <typename V, class F>
+  __device__ inline V combine(V v, V* lds, F f) const {
+    if constexpr (W == 1) return v;
+    if ((threadIdx.x & (kWave - 1)) == 0) lds[wave] = v;
+    __syncthreads();
+    V r = lds[0];
+#pragma unroll
+    for (int w = 1; w < W; ++w) r = f(r, lds[w]);
+    return r;
+  }
+};
+
+// f(i, vector i) for the lane's vectors of a row, up to 4 loads in flight
+template <int W, typename T, class F>
+__device__ inline void for_vectors(const T* xr, int64_t nv, int t, F f) {
+  constexpr int S = W * kWave, N = Vec<T>::N;
+  int64_t i = t;
+  for (; i + 3 * S < nv; i += 4 * S) {
+    const u32x4_t a = ld_row(xr + i * N), b = ld_row(xr + (i + S) * N);
+    const u32x4_t c = ld_row(xr + (i + 2 * S) * N), d = ld_row(xr + (i + 3 * S) * N);
+    f(i, a);
+    f(i + S, b);
+    f(i + 2 * S, c);
+    f(i + 3 * S, d);
+  }
+  if (i + S < nv) {
+    const u32x4_t a = ld_row(xr + i * N), b = ld_row(xr + (i + S) * N);
+    f(i, a);
+    f(i + S, b);
+    i += 2 * S;
+  }
+  if (i < nv) f(i, ld_row(xr + i * N));
+}
+
+// element j of a 16-byte vector as fp32
+template <typename T, bool IS_F16>
+__device__ inline float elem(const u32x4_t& v, int j) {
+  if constexpr (sizeof(T) == 4) {
+    const uint32_t w = v[j];
+    return __builtin_bit_cast(float, w);
+  } else {
+    const uint32_t w = v[j / 2];
+    return ld<T, IS_F16>(uint16_t(j % 2 ? w >> 16 : w));
+  }
+}
+
 // StableHLO max/min propagate NaN; fmaxf/fminf drop it, so NaN is tracked
 // separately for OP 1/2.
-template <typename T, bool IS_F16, int OP>
-__global__ __launch_bounds__(kBlock) void row_reduce_kernel(const T* __restrict__ x, int64_t rows,
-                                                            int64_t cols, float init, void* y,
-                                                            int out_type, bool vec_ok) {
-  const int lane = threadIdx.x & (kWave - 1);
-  const int64_t row = int64_t(blockIdx.x) * kWavesPerBlock + (threadIdx.x >> 6);
-  if (row >= rows) return;
-  const T* xr = x + row * cols;
+template <typename T, bool IS_F16, int OP, int W>
+__global__ __launch_bounds__(kTeamBlock<W>) void row_reduce_kernel(const T* __restrict__ x, int64_t rows,
+                                                                   int64_t cols, float init, void* y,
+                                                                   int out_type) {
+  __shared__ float red[W];
+  __shared__ int red_nan[W];
+  const Team<W> tm;
+  if (W == 1 && tm.row >= rows) return;
+  const T* xr = x + tm.row * cols;
+  constexpr int N = Vec<T>::N;
+  const int64_t nv = cols / N;
   float acc = identity<OP>();
   bool nan = false;
-  constexpr int N = Vec<T>::N;
-  if (vec_ok) {
-    using V = typename Vec<T>::V;
-    const V* xv = reinterpret_cast<const V*>(xr);
-    const int64_t nv = cols / N;
-    int64_t i = lane;
-    // two vectors in flight per iteration
-    for (; i + kWave < nv; i += 2 * kWave) {
-      V a = xv[i], b = xv[i + kWave];
+  auto take = [&](float f) {
+    nan |= (f != f);
+    acc = combine<OP>(acc, f);
+  };
+  for_vectors<W>(xr, nv, tm.t, [&](int64_t, const u32x4_t& v) {
 #pragma unroll
-      for (int j = 0; j < N; ++j) {
-        float fa = ld<T, IS_F16>(a.v[j]);
-        nan |= (fa != fa);
-        acc = combine<OP>(acc, fa);
-      }
-#pragma unroll
-      for (int j = 0; j < N; ++j) {
-        float fb = ld<T, IS_F16>(b.v[j]);
-        nan |= (fb != fb);
-        acc = combine<OP>(acc, fb);
-      }
-    }
-    for (; i < nv; i += kWave) {
-      V a = xv[i];
-#pragma unroll
-      for (int j = 0; j < N; ++j) {
-        float fa = ld<T, IS_F16>(a.v[j]);
-        nan |= (fa != fa);
-        acc = combine<OP>(acc, fa);
-      }
-    }
-  } else {
-    for (int64_t c = lane; c < cols; c += kWave) {
-      float f = ld<T, IS_F16>(xr[c]);
-      nan |= (f != f);
-      acc = combine<OP>(acc, f);
-    }
-  }
-  acc = wave_combine<OP>(acc);
+    for (int j = 0; j < N; ++j) take(elem<T, IS_F16>(v, j));
+  });
+  if (nv * N + tm.t < cols) take(ld<T, IS_F16>(xr[nv * N + tm.t]));
+  acc = tm.combine(wave_combine<OP>(acc), red, [](float a, float b) { return combine<OP>(a, b); });
   // the vote must run with the whole wave active, before the lane-0 branch
-  const bool any_nan = __any(nan);
-  if (lane == 0) {
+  const int any_nan = tm.combine(int(__any(nan)), red_nan, [](int a, int b) { return a | b; });
+  if (tm.t == 0) {
     float r = combine<OP>(acc, init);
     if constexpr (OP == 1 || OP == 2) {
       if (any_nan || init != init) r = __builtin_nanf("");
     }
-    store_from_f32(y, row, out_type, r);
+    store_from_f32(y, tm.row, out_type, r);
   }
 }
 
-// (value, index) pair compare for argmax/argmin with XLA semantics.
-template <bool IS_MIN>
-__device__ inline bool better(float a, int64_t ia, float b, int64_t ib) {
-  const bool an = a != a, bn = b != b;
-  if (an || bn) {
-    if (an && bn) return ia < ib;
-    return an;
-  }
-  if (a == b) return ia < ib;
-  return IS_MIN ? (a < b) : (a > b);
-}
-
-template <typename T> __device__ inline uint32_t raw_bits(T v) {
-  if constexpr (sizeof(T) == 4) {
-    uint32_t u;
-    __builtin_memcpy(&u, &v, 4);
-    return u;
-  } else {
-    return uint32_t(v);
-  }
-}
-template <typename T> __device__ inline T from_bits(uint32_t u) {
-  if constexpr (sizeof(T) == 4) {
-    T v;
-    __builtin_memcpy(&v, &u, 4);
-    return v;
-  } else {
-    return T(u);
-  }
-}
-
-template <typename T, bool IS_F16, bool IS_MIN, typename IdxT>
-__global__ __launch_bounds__(kBlock) void row_argmax_kernel(const T* __restrict__ x, int64_t rows,
-                                                            int64_t cols, T* __restrict__ values,
-                                                            IdxT* __restrict__ indices, bool vec_ok) {
-  const int lane = threadIdx.x & (kWave - 1);
-  const int64_t row = int64_t(blockIdx.x) * kWavesPerBlock + (threadIdx.x >> 6);
-  if (row >= rows) return;
-  const T* xr = x + row * cols;
-  float best = 0.f;
-  int64_t bi = INT64_MAX;  // "no element yet": loses to any real element
-  uint32_t braw = 0;
-  constexpr int N = Vec<T>::N;
-  // Elements are visited in increasing index within a lane, so only a
-  // strictly better element may replace the current one.
-  auto consider = [&](T raw, int64_t idx) {
-    float f = ld<T, IS_F16>(raw);
-    if (bi == INT64_MAX || better<IS_MIN>(f, idx, best, bi)) {
-      best = f;
-      bi = idx;
-      braw = raw_bits<T>(raw);
-    }
-  };
-  if (vec_ok) {
-    using V = typename Vec<T>::V;
-    const V* xv = reinterpret_cast<const V*>(xr);
-    const int64_t nv = cols / N;
-    int64_t i = lane;
-    for (; i + kWave < nv; i += 2 * kWave) {
-      V a = xv[i], b = xv[i + kWave];
-#pragma unroll
-      for (int j = 0; j < N; ++j) consider(a.v[j], i * N + j);
-#pragma unroll
-      for (int j = 0; j < N; ++j) consider(b.v[j], (i + kWave) * N + j);
-    }
-    for (; i < nv; i += kWave) {
-      V a = xv[i];
-#pragma unroll
-      for (int j = 0; j < N; ++j) consider(a.v[j], i * N + j);
-    }
-  } else {
-    for (int64_t c = lane; c < cols; c += kWave) consider(xr[c], c);
-  }
-  // butterfly: every lane ends with the row winner
-#pragma unroll
-  for (int m = 32; m >= 1; m >>= 1) {
-    const float ob = __shfl_xor(best, m, kWave);
-    const int64_t oi = __shfl_xor(bi, m, kWave);
-    const uint32_t oraw = __shfl_xor(braw, m, kWave);
-    if (oi != INT64_MAX && (bi == INT64_MAX || better<IS_MIN>(ob, oi, best, bi))) {
-      best = ob;
-      bi = oi;
-      braw = oraw;
-    }
-  }
-  if (lane == 0) {
-    if (values) values[row] = from_bits<T>(braw);
-    indices[row] = IdxT(bi == INT64_MAX ? 0 : bi);
-  }
-}
-
-// Argmax / argmin of 16-bit floats (bf16, f16) with a row of at most 65536
-// elements: each element becomes the 32-bit word (key << 16) | (0xFFFF - i),
-// where key orders the values as the XLA reducer does (larger value wins for
-// argmax, smaller for argmin, every NaN beats every number, -0 == +0), so
-// the row winner -- ties going to the lower index -- is the unsigned max of
-// the words.  Two elements are keyed at once with packed 16-bit integer ops.
+// Argmax / argmin with XLA's variadic-reduce semantics: larger value wins for
+// argmax (smaller for argmin), every NaN beats every number, -0 == +0, ties
+// go to the lower index.  Each element becomes an unsigned key that orders
+// the values that way.
 typedef unsigned short u16x2_t __attribute__((ext_vector_type(2)));
 
+// two 16-bit floats (bf16, f16; INF the infinity's bits) at once with packed
+// 16-bit integer ops
 template <bool IS_MIN, uint32_t INF>
 __device__ inline uint32_t order_keys(uint32_t w) {
   constexpr unsigned short kNan = INF + 1;  // smallest NaN magnitude
@@ -233,36 +188,86 @@ __device__ inline uint32_t order_keys(uint32_t w) {
   const uint32_t kn = __builtin_bit_cast(uint32_t, u16x2_t{0x8000, 0x8000} - magc);
   return (mask & kn) | (~mask & kp);
 }
+// one fp32
+template <bool IS_MIN>
+__device__ inline uint32_t order_key32(uint32_t w) {
+  const uint32_t mag = w & 0x7FFFFFFFu;
+  if (mag > 0x7F800000u) return 0xFFFFFFFFu;
+  return ((w >> 31) != 0) != IS_MIN ? 0x80000000u - mag : 0x80000000u + mag;
+}
 
-template <bool IS_F16, bool IS_MIN, typename IdxT>
-__global__ __launch_bounds__(kBlock) void row_argmax16_kernel(const uint16_t* __restrict__ x, int64_t rows,
-                                                              int cols, uint16_t* __restrict__ values,
-                                                              IdxT* __restrict__ indices) {
+// Rows of at most 65536 16-bit floats (NARROW): an element is the word
+// (key << 16) | (0xFFFF - index), so the row winner is the unsigned max of
+// the words.  Otherwise key and index are kept apart; a lane visits its
+// elements in increasing index, so only a larger key replaces its winner.
+template <typename T, bool IS_F16, bool IS_MIN, typename IdxT, bool NARROW, int W>
+__global__ __launch_bounds__(kTeamBlock<W>) void row_argmax_kernel(const T* __restrict__ x, int64_t rows,
+                                                                   int64_t cols, T* __restrict__ values,
+                                                                   IdxT* __restrict__ indices) {
   constexpr uint32_t kInf = IS_F16 ? 0x7C00u : 0x7F80u;
-  const int lane = threadIdx.x & (kWave - 1);
-  const int64_t row = int64_t(blockIdx.x) * kWavesPerBlock + (threadIdx.x >> 6);
-  if (row >= rows) return;
-  const uint16_t* xr = x + row * cols;
-  const u32x4_t* xv = reinterpret_cast<const u32x4_t*>(xr);
-  const int nv = cols / 8;
-  uint32_t best = 0;  // below every element's word
-#pragma unroll 2
-  for (int i = lane; i < nv; i += kWave) {
-    const u32x4_t a = xv[i];
+  constexpr int N = Vec<T>::N;
+  __shared__ uint32_t red_key[W];
+  __shared__ int64_t red_at[W];
+  const Team<W> tm;
+  if (W == 1 && tm.row >= rows) return;
+  const T* xr = x + tm.row * cols;
+  const int64_t nv = cols / N, tail = nv * N + tm.t;
+  uint32_t best = 0;  // below every element's word; at or below every key
+  int64_t at = INT64_MAX;
+  if constexpr (NARROW) {
+    static_assert(sizeof(T) == 2, "16-bit floats");
+    for_vectors<W>(xr, nv, tm.t, [&](int64_t i, const u32x4_t& v) {
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const uint32_t k = order_keys<IS_MIN, kInf>(a[j]);
-      const uint32_t e = 0xFFFFu - uint32_t(8 * i + 2 * j);  // complement of the low half's index
-      const uint32_t p0 = (k << 16) | e, p1 = (k & 0xFFFF0000u) | (e - 1u);
-      best = max(best, max(p0, p1));
+      for (int j = 0; j < 4; ++j) {
+        const uint32_t k = order_keys<IS_MIN, kInf>(v[j]);
+        const uint32_t e = 0xFFFFu - (8u * uint32_t(i) + 2 * j);  // complement of the low half's index
+        const uint32_t p0 = (k << 16) | e, p1 = (k & 0xFFFF0000u) | (e - 1u);
+        best = max(best, max(p0, p1));
+      }
+    });
+    if (tail < cols) best = max(best, (order_keys<IS_MIN, kInf>(xr[tail]) << 16) | (0xFFFFu - uint32_t(tail)));
+#pragma unroll
+    for (int m = 32; m >= 1; m >>= 1) best = max(best, uint32_t(__shfl_xor(int(best), m, kWave)));
+    best = tm.combine(best, red_key, [](uint32_t a, uint32_t b) { return max(a, b); });
+    at = int64_t(0xFFFFu - (best & 0xFFFFu));
+  } else {
+    auto take = [&](uint32_t key, int64_t i) {
+      if (key > best || at == INT64_MAX) best = key, at = i;
+    };
+    for_vectors<W>(xr, nv, tm.t, [&](int64_t i, const u32x4_t& v) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        if constexpr (sizeof(T) == 2) {
+          const uint32_t k = order_keys<IS_MIN, kInf>(v[j]);
+          take(k & 0xFFFFu, i * N + 2 * j);
+          take(k >> 16, i * N + 2 * j + 1);
+        } else {
+          take(order_key32<IS_MIN>(v[j]), i * N + j);
+        }
+      }
+    });
+    if (tail < cols) {
+      if constexpr (sizeof(T) == 2) take(order_keys<IS_MIN, kInf>(xr[tail]) & 0xFFFFu, tail);
+      else take(order_key32<IS_MIN>(__builtin_bit_cast(uint32_t, xr[tail])), tail);
+    }
+    // lanes without an element hold (0, INT64_MAX) and lose every tie
+#pragma unroll
+    for (int m = 32; m >= 1; m >>= 1) {
+      const uint32_t ok = __shfl_xor(best, m, kWave);
+      const int64_t oi = __shfl_xor(at, m, kWave);
+      if (ok > best || (ok == best && oi < at)) best = ok, at = oi;
+    }
+    if constexpr (W > 1) {
+      if ((threadIdx.x & (kWave - 1)) == 0) red_key[tm.wave] = best, red_at[tm.wave] = at;
+      __syncthreads();
+      if (tm.t != 0) return;
+      for (int w = 1; w < W; ++w)
+        if (red_key[w] > best || (red_key[w] == best && red_at[w] < at)) best = red_key[w], at = red_at[w];
     }
   }
-#pragma unroll
-  for (int m = 32; m >= 1; m >>= 1) best = max(best, uint32_t(__shfl_xor(int(best), m, kWave)));
-  if (lane == 0) {
-    const int idx = int(0xFFFFu - (best & 0xFFFFu));
-    if (values) values[row] = xr[idx];  // the winner's own bits (NaN payloads included)
-    indices[row] = IdxT(idx);
+  if (tm.t == 0) {
+    if (values) values[tm.row] = xr[at];  // the winner's own bits (NaN payloads included)
+    indices[tm.row] = IdxT(at);
   }
 }
 
@@ -453,66 +458,249 @@ __global__ __launch_bounds__(kBlock) void layernorm_bf16_split_kernel(
   }
 }
 
-// Fallback LayerNorm for any width: three streaming passes over the row.
-// With x2 (fp32 rows): the row is x + x2, written to xsum first (the passes
-// then read that row back; each lane reads only what it wrote).
-template <typename T, typename TO = T>
-__global__ __launch_bounds__(kBlock) void layernorm_loop_kernel(const T* __restrict__ x,
-                                                                const T* __restrict__ gamma,
-                                                                const T* __restrict__ beta,
-                                                                int64_t rows, int64_t cols,
-                                                                float eps, TO* __restrict__ y,
-                                                                const T* x2 = nullptr, T* xsum = nullptr) {
-  const int lane = threadIdx.x & (kWave - 1);
-  const int64_t row = int64_t(blockIdx.x) * kWavesPerBlock + (threadIdx.x >> 6);
-  if (row >= rows) return;
-  const T* xr = x + row * cols;
-  if constexpr (sizeof(T) == 4) {
-    if (x2) {
-      for (int64_t c = lane; c < cols; c += kWave) xsum[row * cols + c] = xr[c] + x2[row * cols + c];
-      xr = xsum + row * cols;
+// A lane's share of a team's row: KV 16-byte vectors (vector t + 64 W k; nv
+// whole ones in the row) and the row's element nv N + t past them.  The loads
+// are unconditional (vector 0 where the row has no such vector), so all of
+// them are in flight together.
+template <typename T, int W, int KV>
+struct RowShare {
+  static constexpr int N = Vec<T>::N, S = W * kWave;
+  u32x4_t v[KV];
+  float tail;
+  int64_t nv;
+  int t;
+  bool has_tail;
+  __device__ inline RowShare(const T* xr, int64_t cols, int t_) : t(t_) {
+    nv = cols / N;
+    has_tail = nv * N + t < cols;
+    if (nv > 0) {
+#pragma unroll
+      for (int k = 0; k < KV; ++k) v[k] = ld_row(xr + (has(k) ? t + k * S : 0) * int64_t(N));
     }
+    tail = has_tail ? to_f32<T>(xr[nv * N + t]) : 0.f;
   }
-  float s = 0.f;
-  for (int64_t c = lane; c < cols; c += kWave) s += to_f32<T>(xr[c]);
-  const float mean = wave_sum(s) / float(cols);
-  float q = 0.f;
-  for (int64_t c = lane; c < cols; c += kWave) {
-    float d = to_f32<T>(xr[c]) - mean;
-    q += d * d;
-  }
-  const float rstd = 1.f / sqrtf(wave_sum(q) / float(cols) + eps);
-  TO* yr = y + row * cols;
-  for (int64_t c = lane; c < cols; c += kWave) {
-    float gj = gamma ? to_f32<T>(gamma[c]) : 1.f;
-    float bj = beta ? to_f32<T>(beta[c]) : 0.f;
-    float v = (to_f32<T>(xr[c]) - mean) * rstd * gj + bj;
-    if constexpr (sizeof(TO) == 2) yr[c] = f32_to_bf16(v);
-    else yr[c] = v;
-  }
+  __device__ inline bool has(int k) const { return t + k * S < nv; }
+  __device__ inline float at(int k, int j) const { return elem<T, false>(v[k], j); }
+};
+
+template <typename T>
+__device__ inline T narrow(float f) {
+  if constexpr (sizeof(T) == 2) return f32_to_bf16(f);
+  else return f;
+}
+// N fp32 values to TO elements at an element-aligned address
+template <typename TO, int N>
+__device__ inline void st_values(TO* p, const float (&o)[N]) {
+  struct __attribute__((packed, aligned(sizeof(TO)))) Pack { TO e[N]; };
+  Pack q;
+#pragma unroll
+  for (int j = 0; j < N; ++j) q.e[j] = narrow<TO>(o[j]);
+  *reinterpret_cast<Pack*>(p) = q;
 }
 
-// Softmax over a row: max pass, sum-of-exp pass, normalise pass.
-template <typename T>
-__global__ __launch_bounds__(kBlock) void softmax_kernel(const T* __restrict__ x, int64_t rows,
-                                                         int64_t cols, T* __restrict__ y) {
-  const int lane = threadIdx.x & (kWave - 1);
-  const int64_t row = int64_t(blockIdx.x) * kWavesPerBlock + (threadIdx.x >> 6);
-  if (row >= rows) return;
-  const T* xr = x + row * cols;
-  float m = -INFINITY;
-  for (int64_t c = lane; c < cols; c += kWave) m = fmaxf(m, to_f32<T>(xr[c]));
-  m = wave_max(m);
-  float s = 0.f;
-  for (int64_t c = lane; c < cols; c += kWave) s += __expf(to_f32<T>(xr[c]) - m);
-  s = wave_sum(s);
-  const float inv = 1.f / s;
-  T* yr = y + row * cols;
-  for (int64_t c = lane; c < cols; c += kWave) {
-    float v = __expf(to_f32<T>(xr[c]) - m) * inv;
-    if constexpr (sizeof(T) == 2) yr[c] = f32_to_bf16(v);
-    else yr[c] = v;
+// LayerNorm of rows off the 16-byte grid or wider than the kernels above
+// hold: the row in the registers of a team of W waves (KV vectors per lane),
+// one read of x, the same two-pass statistics.  With x2 (fp32 rows) the row
+// is x + x2, written to xsum.  Against three element-wise passes over the
+// row: 8192 x 4095 bf16 114 -> 29.9 us, 8192 x 4096 fp32 114 -> 50.5 us (5.3
+// TB/s), 30000 x 300 bf16 26.3 -> 12.8 us.
+template <typename T, typename TO, int W, int KV>
+__global__ __launch_bounds__(kTeamBlock<W>) void layernorm_team_kernel(
+    const T* __restrict__ x, const T* __restrict__ gamma, const T* __restrict__ beta, int64_t rows, int64_t cols,
+    float eps, TO* __restrict__ y, const T* __restrict__ x2, T* __restrict__ xsum) {
+  using R = RowShare<T, W, KV>;
+  constexpr int N = R::N;
+  __shared__ float red[2][W];
+  const Team<W> tm;
+  if (W == 1 && tm.row >= rows) return;
+  R r(x + tm.row * cols, cols, tm.t);
+  const int64_t tail = r.nv * N + tm.t;
+  if constexpr (sizeof(T) == 4) {
+    if (x2) {
+      const R r2(x2 + tm.row * cols, cols, tm.t);
+      T* sr = xsum + tm.row * cols;
+#pragma unroll
+      for (int k = 0; k < KV; ++k) {
+        float o[N];
+#pragma unroll
+        for (int j = 0; j < N; ++j) {
+          o[j] = r.at(k, j) + r2.at(k, j);
+          r.v[k][j] = __builtin_bit_cast(uint32_t, o[j]);
+        }
+        if (r.has(k)) st_values<T, N>(sr + int64_t(tm.t + k * R::S) * N, o);
+      }
+      r.tail += r2.tail;
+      if (r.has_tail) sr[tail] = r.tail;
+    }
   }
+  auto add = [](float a, float b) { return a + b; };
+  const float inv_n = 1.f / float(cols);
+  float s = r.tail;
+#pragma unroll
+  for (int k = 0; k < KV; ++k)
+    if (r.has(k))
+#pragma unroll
+      for (int j = 0; j < N; ++j) s += r.at(k, j);
+  const float mean = tm.combine(wave_sum(s), red[0], add) * inv_n;
+  float q = r.has_tail ? (r.tail - mean) * (r.tail - mean) : 0.f;
+#pragma unroll
+  for (int k = 0; k < KV; ++k)
+    if (r.has(k))
+#pragma unroll
+      for (int j = 0; j < N; ++j) {
+        const float d = r.at(k, j) - mean;
+        q += d * d;
+      }
+  const float rstd = 1.f / sqrtf(tm.combine(wave_sum(q), red[1], add) * inv_n + eps);
+  TO* yr = y + tm.row * cols;
+#pragma unroll
+  for (int k = 0; k < KV; ++k) {
+    if (!r.has(k)) continue;
+    const int64_t c = int64_t(tm.t + k * R::S) * N;
+    const u32x4_t g = gamma ? ld_row(gamma + c) : u32x4_t{0u, 0u, 0u, 0u};
+    const u32x4_t b = beta ? ld_row(beta + c) : u32x4_t{0u, 0u, 0u, 0u};
+    float o[N];
+#pragma unroll
+    for (int j = 0; j < N; ++j)
+      o[j] = (r.at(k, j) - mean) * rstd * (gamma ? elem<T, false>(g, j) : 1.f) + elem<T, false>(b, j);
+    st_values<TO, N>(yr + c, o);
+  }
+  if (r.has_tail)
+    yr[tail] = narrow<TO>((r.tail - mean) * rstd * (gamma ? to_f32<T>(gamma[tail]) : 1.f) +
+                          (beta ? to_f32<T>(beta[tail]) : 0.f));
+}
+
+// LayerNorm of rows longer than a 16-wave team holds: three passes over the
+// row.  With x2: as above; each lane reads back only what it wrote to xsum.
+template <typename T, typename TO = T>
+__global__ __launch_bounds__(kTeamBlock<16>) void layernorm_loop_kernel(
+    const T* __restrict__ x, const T* __restrict__ gamma, const T* __restrict__ beta, int64_t rows, int64_t cols,
+    float eps, TO* __restrict__ y, const T* x2, T* xsum) {
+  constexpr int N = Vec<T>::N;
+  __shared__ float red[2][16];
+  const Team<16> tm;
+  const T* xr = x + tm.row * cols;
+  const int64_t nv = cols / N, tail = nv * N + tm.t;
+  const bool has_tail = tail < cols;
+  if constexpr (sizeof(T) == 4) {
+    if (x2) {
+      T* sr = xsum + tm.row * cols;
+      for_vectors<16>(xr, nv, tm.t, [&](int64_t i, const u32x4_t& v) {
+        const u32x4_t v2 = ld_row(x2 + tm.row * cols + i * N);
+        float o[N];
+#pragma unroll
+        for (int j = 0; j < N; ++j) o[j] = elem<T, false>(v, j) + elem<T, false>(v2, j);
+        st_values<T, N>(sr + i * N, o);
+      });
+      if (has_tail) sr[tail] = xr[tail] + x2[tm.row * cols + tail];
+      xr = sr;
+    }
+  }
+  auto add = [](float a, float b) { return a + b; };
+  float s = has_tail ? to_f32<T>(xr[tail]) : 0.f;
+  for_vectors<16>(xr, nv, tm.t, [&](int64_t, const u32x4_t& v) {
+#pragma unroll
+    for (int j = 0; j < N; ++j) s += elem<T, false>(v, j);
+  });
+  const float mean = tm.combine(wave_sum(s), red[0], add) / float(cols);
+  float q = has_tail ? (to_f32<T>(xr[tail]) - mean) * (to_f32<T>(xr[tail]) - mean) : 0.f;
+  for_vectors<16>(xr, nv, tm.t, [&](int64_t, const u32x4_t& v) {
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+      const float d = elem<T, false>(v, j) - mean;
+      q += d * d;
+    }
+  });
+  const float rstd = 1.f / sqrtf(tm.combine(wave_sum(q), red[1], add) / float(cols) + eps);
+  TO* yr = y + tm.row * cols;
+  for_vectors<16>(xr, nv, tm.t, [&](int64_t i, const u32x4_t& v) {
+    const u32x4_t g = gamma ? ld_row(gamma + i * N) : u32x4_t{0u, 0u, 0u, 0u};
+    const u32x4_t b = beta ? ld_row(beta + i * N) : u32x4_t{0u, 0u, 0u, 0u};
+    float o[N];
+#pragma unroll
+    for (int j = 0; j < N; ++j)
+      o[j] = (elem<T, false>(v, j) - mean) * rstd * (gamma ? elem<T, false>(g, j) : 1.f) + elem<T, false>(b, j);
+    st_values<TO, N>(yr + i * N, o);
+  });
+  if (has_tail)
+    yr[tail] = narrow<TO>((to_f32<T>(xr[tail]) - mean) * rstd * (gamma ? to_f32<T>(gamma[tail]) : 1.f) +
+                          (beta ? to_f32<T>(beta[tail]) : 0.f));
+}
+
+// Softmax with the row in a team's registers: one read of x, the exponentials
+// kept for the division.  Against three element-wise passes over the row:
+// 65536 x 1024 bf16 171 -> 46.5 us (5.8 TB/s), 2048 x 50257 921 -> 118 us.
+template <typename T, int W, int KV>
+__global__ __launch_bounds__(kTeamBlock<W>) void softmax_team_kernel(const T* __restrict__ x, int64_t rows,
+                                                                     int64_t cols, T* __restrict__ y) {
+  using R = RowShare<T, W, KV>;
+  constexpr int N = R::N;
+  __shared__ float red[2][W];
+  const Team<W> tm;
+  if (W == 1 && tm.row >= rows) return;
+  const R r(x + tm.row * cols, cols, tm.t);
+  float m = r.has_tail ? r.tail : -INFINITY;
+#pragma unroll
+  for (int k = 0; k < KV; ++k)
+    if (r.has(k))
+#pragma unroll
+      for (int j = 0; j < N; ++j) m = fmaxf(m, r.at(k, j));
+  m = tm.combine(wave_max(m), red[0], [](float a, float b) { return fmaxf(a, b); });
+  float e[KV][N], s = 0.f;
+#pragma unroll
+  for (int k = 0; k < KV; ++k)
+    if (r.has(k))
+#pragma unroll
+      for (int j = 0; j < N; ++j) {
+        e[k][j] = __expf(r.at(k, j) - m);
+        s += e[k][j];
+      }
+  const float et = __expf(r.tail - m);
+  if (r.has_tail) s += et;
+  const float inv = 1.f / tm.combine(wave_sum(s), red[1], [](float a, float b) { return a + b; });
+  T* yr = y + tm.row * cols;
+#pragma unroll
+  for (int k = 0; k < KV; ++k) {
+    if (!r.has(k)) continue;
+#pragma unroll
+    for (int j = 0; j < N; ++j) e[k][j] *= inv;
+    st_values<T, N>(yr + int64_t(tm.t + k * R::S) * N, e[k]);
+  }
+  if (r.has_tail) yr[r.nv * N + tm.t] = narrow<T>(et * inv);
+}
+
+// Softmax of rows longer than a 16-wave team holds: max pass, sum-of-exp
+// pass, normalise pass.
+template <typename T>
+__global__ __launch_bounds__(kTeamBlock<16>) void softmax_loop_kernel(const T* __restrict__ x, int64_t rows,
+                                                                      int64_t cols, T* __restrict__ y) {
+  constexpr int N = Vec<T>::N;
+  __shared__ float red[2][16];
+  const Team<16> tm;
+  const T* xr = x + tm.row * cols;
+  const int64_t nv = cols / N, tail = nv * N + tm.t;
+  const bool has_tail = tail < cols;
+  const float xt = has_tail ? to_f32<T>(xr[tail]) : -INFINITY;
+  float m = xt;
+  for_vectors<16>(xr, nv, tm.t, [&](int64_t, const u32x4_t& v) {
+#pragma unroll
+    for (int j = 0; j < N; ++j) m = fmaxf(m, elem<T, false>(v, j));
+  });
+  m = tm.combine(wave_max(m), red[0], [](float a, float b) { return fmaxf(a, b); });
+  float s = has_tail ? __expf(xt - m) : 0.f;
+  for_vectors<16>(xr, nv, tm.t, [&](int64_t, const u32x4_t& v) {
+#pragma unroll
+    for (int j = 0; j < N; ++j) s += __expf(elem<T, false>(v, j) - m);
+  });
+  const float inv = 1.f / tm.combine(wave_sum(s), red[1], [](float a, float b) { return a + b; });
+  T* yr = y + tm.row * cols;
+  for_vectors<16>(xr, nv, tm.t, [&](int64_t i, const u32x4_t& v) {
+    float o[N];
+#pragma unroll
+    for (int j = 0; j < N; ++j) o[j] = __expf(elem<T, false>(v, j) - m) * inv;
+    st_values<T, N>(yr + i * N, o);
+  });
+  if (has_tail) yr[tail] = narrow<T>(__expf(xt - m) * inv);
 }
 
 inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
@@ -521,47 +709,116 @@ inline unsigned grid_for_rows(int64_t rows) {
   return unsigned((rows + kWavesPerBlock - 1) / kWavesPerBlock);
 }
 
+// Waves per row.  A wave per row when there are rows enough to fill the chip
+// and a lane's share is at most 8 vectors; four or sixteen waves for longer
+// rows, and for few rows, whose time is one wave's serial chain of loads
+// (argmax of 32 rows of 50257 bf16: 161 us a call with a wave per row and
+// 2-byte loads, 11.8 us with sixteen, most of that the call itself).
+inline int team_waves(int64_t rows, int64_t vecs) {
+  if (vecs > 2048 || (rows < 512 && vecs > 512)) return 16;
+  if (vecs > 512 || (rows < 2048 && vecs > 64)) return 4;
+  return 1;
+}
+template <int W> using Waves = std::integral_constant<int, W>;
+// f(Waves<W>{}) with the team of rows x vecs 16-byte vectors
+template <class F>
+void with_team(int64_t rows, int64_t vecs, F f) {
+  switch (team_waves(rows, vecs)) {
+    case 1: f(Waves<1>{}); break;
+    case 4: f(Waves<4>{}); break;
+    default: f(Waves<16>{}); break;
+  }
+}
+template <int W> dim3 team_grid(int64_t rows) { return dim3(unsigned((rows + Team<W>::kRows - 1) / Team<W>::kRows)); }
+
+template <typename T, bool IS_F16, int OP>
+void launch_reduce_op(hipStream_t s, int64_t rows, int64_t cols, const void* x, float init, void* y, int out_type) {
+  with_team(rows, cols / Vec<T>::N, [&](auto w) {
+    constexpr int W = decltype(w)::value;
+    hipLaunchKernelGGL((row_reduce_kernel<T, IS_F16, OP, W>), team_grid<W>(rows), dim3(kTeamBlock<W>), 0, s,
+                       reinterpret_cast<const T*>(x), rows, cols, init, y, out_type);
+  });
+}
+
 template <typename T, bool IS_F16>
 int launch_reduce(hipStream_t s, int op, int64_t rows, int64_t cols, const void* x, float init,
                   void* y, int out_type) {
-  const bool vec_ok = aligned16(x) && (cols % Vec<T>::N) == 0;
-  const T* xp = reinterpret_cast<const T*>(x);
-  dim3 g(grid_for_rows(rows)), b(kBlock);
   switch (op) {
-    case 0: hipLaunchKernelGGL((row_reduce_kernel<T, IS_F16, 0>), g, b, 0, s, xp, rows, cols, init, y, out_type, vec_ok); break;
-    case 1: hipLaunchKernelGGL((row_reduce_kernel<T, IS_F16, 1>), g, b, 0, s, xp, rows, cols, init, y, out_type, vec_ok); break;
-    case 2: hipLaunchKernelGGL((row_reduce_kernel<T, IS_F16, 2>), g, b, 0, s, xp, rows, cols, init, y, out_type, vec_ok); break;
-    case 3: hipLaunchKernelGGL((row_reduce_kernel<T, IS_F16, 3>), g, b, 0, s, xp, rows, cols, init, y, out_type, vec_ok); break;
+    case 0: launch_reduce_op<T, IS_F16, 0>(s, rows, cols, x, init, y, out_type); break;
+    case 1: launch_reduce_op<T, IS_F16, 1>(s, rows, cols, x, init, y, out_type); break;
+    case 2: launch_reduce_op<T, IS_F16, 2>(s, rows, cols, x, init, y, out_type); break;
+    case 3: launch_reduce_op<T, IS_F16, 3>(s, rows, cols, x, init, y, out_type); break;
     default: return fail(MK_ERR_INVALID, "mk_row_reduce: op must be 0..3");
   }
   return check_launch("mk_row_reduce");
 }
 
+template <typename T, bool IS_F16, bool IS_MIN, typename IdxT>
+int launch_argmax_as(hipStream_t s, int64_t rows, int64_t cols, const void* x, void* values, void* indices) {
+  with_team(rows, cols / Vec<T>::N, [&](auto w) {
+    constexpr int W = decltype(w)::value;
+    auto go = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, team_grid<W>(rows), dim3(kTeamBlock<W>), 0, s, reinterpret_cast<const T*>(x), rows,
+                         cols, reinterpret_cast<T*>(values), reinterpret_cast<IdxT*>(indices));
+    };
+    if constexpr (sizeof(T) == 2) {
+      if (cols <= 65536) return go(row_argmax_kernel<T, IS_F16, IS_MIN, IdxT, true, W>);
+    }
+    go(row_argmax_kernel<T, IS_F16, IS_MIN, IdxT, false, W>);
+  });
+  return check_launch("mk_row_argmax");
+}
+
 template <typename T, bool IS_F16, bool IS_MIN>
 int launch_argmax(hipStream_t s, int64_t rows, int64_t cols, const void* x, void* values,
                   int index_type, void* indices) {
-  const bool vec_ok = aligned16(x) && (cols % Vec<T>::N) == 0;
-  dim3 g(grid_for_rows(rows)), b(kBlock);
-  const T* xp = reinterpret_cast<const T*>(x);
-  T* vp = reinterpret_cast<T*>(values);
-  if constexpr (sizeof(T) == 2) {
-    if (vec_ok && cols <= 65536) {
-      if (index_type == MK_S32)
-        hipLaunchKernelGGL((row_argmax16_kernel<IS_F16, IS_MIN, int32_t>), g, b, 0, s, xp, rows, int(cols), vp,
-                           reinterpret_cast<int32_t*>(indices));
-      else
-        hipLaunchKernelGGL((row_argmax16_kernel<IS_F16, IS_MIN, int64_t>), g, b, 0, s, xp, rows, int(cols), vp,
-                           reinterpret_cast<int64_t*>(indices));
-      return check_launch("mk_row_argmax");
-    }
+  return index_type == MK_S32 ? launch_argmax_as<T, IS_F16, IS_MIN, int32_t>(s, rows, cols, x, values, indices)
+                              : launch_argmax_as<T, IS_F16, IS_MIN, int64_t>(s, rows, cols, x, values, indices);
+}
+
+// f(Waves<KV>{}) with the vectors per lane of a team of W waves
+template <class F>
+void with_share(int64_t vecs, int waves, F f) {
+  const int64_t per = (vecs + 64 * waves - 1) / (64 * waves);
+  if (per <= 2) f(Waves<2>{});
+  else if (per <= 4) f(Waves<4>{});
+  else f(Waves<8>{});
+}
+constexpr int64_t kTeamMaxVecs = 16 * kWave * 8;  // vectors a 16-wave team's registers hold
+
+// LayerNorm on the kernels that take any width and alignment
+template <typename T, typename TO>
+void launch_layernorm_any(hipStream_t s, int64_t rows, int64_t cols, const T* x, const T* gamma, const T* beta,
+                          float eps, TO* y, const T* x2 = nullptr, T* xsum = nullptr) {
+  const int64_t vecs = cols / Vec<T>::N;
+  if (vecs > kTeamMaxVecs) {
+    hipLaunchKernelGGL((layernorm_loop_kernel<T, TO>), team_grid<16>(rows), dim3(kTeamBlock<16>), 0, s, x, gamma,
+                       beta, rows, cols, eps, y, x2, xsum);
+    return;
   }
-  if (index_type == MK_S32)
-    hipLaunchKernelGGL((row_argmax_kernel<T, IS_F16, IS_MIN, int32_t>), g, b, 0, s, xp, rows, cols,
-                       vp, reinterpret_cast<int32_t*>(indices), vec_ok);
-  else
-    hipLaunchKernelGGL((row_argmax_kernel<T, IS_F16, IS_MIN, int64_t>), g, b, 0, s, xp, rows, cols,
-                       vp, reinterpret_cast<int64_t*>(indices), vec_ok);
-  return check_launch("mk_row_argmax");
+  with_team(rows, vecs, [&](auto w) {
+    constexpr int W = decltype(w)::value;
+    with_share(vecs, W, [&](auto kv) {
+      hipLaunchKernelGGL((layernorm_team_kernel<T, TO, W, decltype(kv)::value>), team_grid<W>(rows),
+                         dim3(kTeamBlock<W>), 0, s, x, gamma, beta, rows, cols, eps, y, x2, xsum);
+    });
+  });
+}
+
+template <typename T>
+void launch_softmax(hipStream_t s, int64_t rows, int64_t cols, const T* x, T* y) {
+  const int64_t vecs = cols / Vec<T>::N;
+  if (vecs > kTeamMaxVecs) {
+    hipLaunchKernelGGL((softmax_loop_kernel<T>), team_grid<16>(rows), dim3(kTeamBlock<16>), 0, s, x, rows, cols, y);
+    return;
+  }
+  with_team(rows, vecs, [&](auto w) {
+    constexpr int W = decltype(w)::value;
+    with_share(vecs, W, [&](auto kv) {
+      hipLaunchKernelGGL((softmax_team_kernel<T, W, decltype(kv)::value>), team_grid<W>(rows), dim3(kTeamBlock<W>), 0,
+                         s, x, rows, cols, y);
+    });
+  });
 }
 
 }  // namespace
@@ -637,14 +894,14 @@ extern "C" int mk_layernorm(void* stream, int io_type, int64_t rows, int64_t col
       hipLaunchKernelGGL((layernorm_bf16_split_kernel<4, 8>), dim3(unsigned(rows)), b, 0, s, xp, gp, bp, rows,
                          int(cols), eps, (T*)y);
     else
-      hipLaunchKernelGGL(layernorm_loop_kernel<T>, g, b, 0, s, xp, gp, bp, rows, cols, eps, (T*)y);
+      launch_layernorm_any<T, T>(s, rows, cols, xp, gp, bp, eps, (T*)y);
   } else if (io_type == MK_F32) {
     using T = float;
     const T *xp = (const T*)x, *gp = (const T*)gamma, *bp = (const T*)beta;
     if (vec_ok(4))
       hipLaunchKernelGGL(layernorm_reg_kernel<T>, g, b, 0, s, xp, gp, bp, rows, int(cols), eps, (T*)y);
     else
-      hipLaunchKernelGGL(layernorm_loop_kernel<T>, g, b, 0, s, xp, gp, bp, rows, cols, eps, (T*)y);
+      launch_layernorm_any<T, T>(s, rows, cols, xp, gp, bp, eps, (T*)y);
   } else {
     return fail(MK_ERR_UNSUPPORTED, "mk_layernorm: io_type must be bf16/f32");
   }
@@ -670,8 +927,7 @@ extern "C" int mk_layernorm_typed(void* stream, int in_type, int out_type, int64
     hipLaunchKernelGGL((layernorm_reg_kernel<float, uint16_t>), g, b, 0, s, xp, gp, bp, rows, int(cols), eps,
                        (uint16_t*)y);
   else
-    hipLaunchKernelGGL((layernorm_loop_kernel<float, uint16_t>), g, b, 0, s, xp, gp, bp, rows, cols, eps,
-                       (uint16_t*)y);
+    launch_layernorm_any<float, uint16_t>(s, rows, cols, xp, gp, bp, eps, (uint16_t*)y);
   return check_launch("mk_layernorm_typed");
 }
 
@@ -700,15 +956,13 @@ extern "C" int mk_add_layernorm_typed(void* stream, int in_type, int out_type, i
       hipLaunchKernelGGL((layernorm_reg_kernel<float, uint16_t, true>), g, blk, 0, s, ap, gp, tp, rows, int(cols), eps,
                          (uint16_t*)y, bp, sp);
     else
-      hipLaunchKernelGGL((layernorm_loop_kernel<float, uint16_t>), g, blk, 0, s, ap, gp, tp, rows, cols, eps,
-                         (uint16_t*)y, bp, sp);
+      launch_layernorm_any<float, uint16_t>(s, rows, cols, ap, gp, tp, eps, (uint16_t*)y, bp, sp);
   } else {
     if (vec)
       hipLaunchKernelGGL((layernorm_reg_kernel<float, float, true>), g, blk, 0, s, ap, gp, tp, rows, int(cols), eps,
                          (float*)y, bp, sp);
     else
-      hipLaunchKernelGGL((layernorm_loop_kernel<float, float>), g, blk, 0, s, ap, gp, tp, rows, cols, eps, (float*)y,
-                         bp, sp);
+      launch_layernorm_any<float, float>(s, rows, cols, ap, gp, tp, eps, (float*)y, bp, sp);
   }
   return check_launch("mk_add_layernorm_typed");
 }
@@ -720,11 +974,10 @@ extern "C" int mk_softmax_rows(void* stream, int io_type, int64_t rows, int64_t 
   if (rows == 0) return MK_OK;
   if (!x || !y) return fail(MK_ERR_INVALID, "mk_softmax_rows: null pointer");
   hipStream_t s = as_stream(stream);
-  dim3 g(grid_for_rows(rows)), b(kBlock);
   if (io_type == MK_BF16)
-    hipLaunchKernelGGL(softmax_kernel<uint16_t>, g, b, 0, s, (const uint16_t*)x, rows, cols, (uint16_t*)y);
+    launch_softmax(s, rows, cols, (const uint16_t*)x, (uint16_t*)y);
   else if (io_type == MK_F32)
-    hipLaunchKernelGGL(softmax_kernel<float>, g, b, 0, s, (const float*)x, rows, cols, (float*)y);
+    launch_softmax(s, rows, cols, (const float*)x, (float*)y);
   else
     return fail(MK_ERR_UNSUPPORTED, "mk_softmax_rows: io_type must be bf16/f32");
   return check_launch("mk_softmax_rows");

@@ -1,0 +1,93 @@
+"""Kernels chosen by a size rule, at the sizes where the rule changes: edges of
+tiles and teams, remainders, unaligned rows, the smallest and largest of each
+range.  References are the oracle, or torch on the CPU in float64."""
+
+import numpy as np
+import pytest
+import torch
+
+from oracle import bf16, ops
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def K(cuda):
+    from mi355x_pjrt import kernels
+
+    kernels.lib()
+    return kernels
+
+
+def shifted(t, off):
+    """t on the GPU, off elements past a 16-byte boundary."""
+    buf = torch.empty(t.numel() + off, dtype=t.dtype, device="cuda")
+    view = buf[off:].view(t.shape)
+    view.copy_(t)
+    return view
+
+
+# rows x columns around a wave's, a 4-wave and a 16-wave team's shares (64, 512, 2048 and 8192
+# vectors), tails of every kind, and past the registers (65536 bf16, 32768 fp32)
+ROW_SHAPES = [(1, 1, 0), (3, 7, 1), (2050, 511, 1), (700, 4097, 0), (511, 4105, 3), (2, 16384, 1), (33, 16391, 0),
+              (5, 50257, 0), (3, 65529, 1), (2, 65551, 0), (2, 140003, 1)]
+
+
+@pytest.mark.parametrize("rows,cols,off", ROW_SHAPES)
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_row_kernels_any_width(K, rows, cols, off, dtype):
+    """Sum, max, argmax, softmax and LayerNorm of odd rows: argmax exact, the
+    rest within fp32 summation error (2^-24 sqrt(cols) of the magnitudes, with
+    a factor of 16) and one rounding to the stored type."""
+    print(f"case: rows [{rows},{cols}] off={off} {dtype}", flush=True)
+    g = torch.Generator().manual_seed(rows * 7 + cols)
+    x = torch.randn(rows, cols, generator=g).to(dtype)
+    x[0, cols // 2] = x[0].max() + 1 if cols > 1 else 1.0
+    x[0, cols - 1] = x[0, cols // 2]  # a tie: the lower index wins
+    if rows > 2:
+        x[1, cols // 3] = float("nan")
+        x[2] = -float("inf")
+    xd, xf = shifted(x, off), x.double().numpy()
+    index, value = K.row_argmax(xd)
+    want, _ = ops.argmax_rows(x.float().numpy())
+    np.testing.assert_array_equal(index.cpu().numpy(), want)
+    bits = torch.int16 if dtype == torch.bfloat16 else torch.int32
+    picked = x[torch.arange(rows), torch.from_numpy(want.astype(np.int64))]
+    assert torch.equal(value.cpu().view(bits), picked.view(bits))
+    low, _ = K.row_argmax(xd, is_min=True, index_dtype=torch.int64)
+    np.testing.assert_array_equal(low.cpu().numpy(), ops.argmax_rows(x.float().numpy(), True)[0])
+    np.testing.assert_array_equal(K.row_reduce(xd, "max").cpu().numpy().astype(np.float64), xf.max(-1))
+
+    ok = slice(3, None) if rows > 2 else slice(None)  # the finite rows
+    xs, xf = shifted(x[ok], off) if x[ok].numel() else None, xf[ok]
+    if xs is None:
+        return
+    # unit roundoff of the stored type: bf16 has 8 significant bits, so half an ulp is up to 2^-8 of the value
+    eps, out = 16 * 2.0 ** -24 * np.sqrt(cols), 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -24
+    got = K.row_reduce(xs, "sum").cpu().double().numpy()
+    assert np.all(np.abs(got - xf.sum(-1)) <= eps * np.abs(xf).sum(-1) / np.sqrt(cols))
+    want = ops.softmax_rows(xf)
+    got = K.softmax_rows(xs).cpu().double().numpy()
+    # __expf: 2 ulp plus the rounding of its argument, |x - max| * 2^-24
+    assert np.all(np.abs(got - want) <= (out + eps + 32 * 2.0 ** -24) * want + 1e-38)
+    gamma, beta = (1 + 0.1 * torch.randn(cols, generator=g)).to(dtype), torch.randn(cols, generator=g).to(dtype)
+    want = ops.layernorm(xf, gamma.double().numpy(), beta.double().numpy())
+    got = K.layernorm(xs, shifted(gamma, off), shifted(beta, 0)).cpu().double().numpy()
+    scale = np.abs(gamma.double().numpy()) * 8 + np.abs(beta.double().numpy())
+    assert np.all(np.abs(got - want) <= out * np.abs(want) + 1e-5 * scale)
+
+
+@pytest.mark.parametrize("rows,cols", [(5, 2052), (3, 4099), (2, 33000)])
+def test_add_layernorm_f32_wide(K, rows, cols):
+    """The fp32 residual add inside the LayerNorm of rows the one-wave kernel
+    does not hold: the stored sum is the one fp32 add, bit for bit."""
+    g = torch.Generator().manual_seed(cols)
+    a, b = torch.randn(rows, cols, generator=g), torch.randn(rows, cols, generator=g)
+    gamma, beta = torch.randn(cols, generator=g), torch.randn(cols, generator=g)
+    s, y = K.add_layernorm(a.cuda(), b.cuda(), None, gamma.cuda(), beta.cuda())
+    assert torch.equal(s.cpu(), a + b)
+    want = ops.layernorm((a + b).double().numpy(), gamma.double().numpy(), beta.double().numpy())
+    scale = gamma.abs().double().numpy() * 8 + beta.abs().double().numpy()
+    assert np.all(np.abs(y.cpu().double().numpy() - want) <= 1e-5 * scale)
+    _, y16 = K.add_layernorm(a.cuda(), b.cuda(), None, gamma.cuda(), beta.cuda(), out_dtype=torch.bfloat16)
+    assert torch.equal(y16.cpu(), y.cpu().bfloat16())

@@ -81,6 +81,20 @@ def sdpa_fwd(q, k, v, scale: float, causal: bool = True, out=None, lse=None, str
 
 
 # ------------------------------------------------------------------ a4 GEMM
+def _few_row_slices(a, b, out):
+    """Slices of the contraction for a product of few rows and too few
+    columns to fill the chip's 256 CUs with 64-column workgroups (1: none).
+    16 x 16384 x 4096 bf16 (M x K x N): 72 us in one launch, 32 in 4 slices and
+    their sum; below 4096 bf16 deep the second launch costs what it saves."""
+    M, Kd = a.shape
+    N = b.shape[1]
+    tiles = (N + 63) // 64
+    if (M > 64 or N < 16 or tiles >= 192 or Kd * a.element_size() < 8192 or a.stride(1) != 1 or N % 4
+            or out.stride(0) % 4 or out.data_ptr() % 16 or out.dtype == torch.float16):
+        return 1
+    return min(16, 256 // tiles, Kd // 512)
+
+
 def gemm(a, b, out_dtype=None, bias=None, relu=False, out=None, stream=None):
     """C[b] = A[b] @ B[b] (+bias)(relu) for 2-D or 3-D views with a unit
     stride along one dim of each operand (transposed views are free)."""
@@ -102,6 +116,15 @@ def gemm(a, b, out_dtype=None, bias=None, relu=False, out=None, stream=None):
     epi = 0 if bias is None else (2 if relu else 1)
     if bias is not None and bias.dtype == torch.float32 and out_dtype != torch.float32:
         epi |= 4  # an fp32 bias added before the narrowing store
+    if squeeze and b.dim() == 2 and stream is None:
+        slices = _few_row_slices(a, b, o3[0])
+        if slices > 1:
+            ws = torch.empty(slices * M * N, dtype=torch.float32, device=a.device)
+            rc = lib().mk_gemm_splitk_typed(
+                _stream(None), mk_dtype(a.dtype), mk_dtype(out_dtype), M, N, K, _ptr(a), a.stride(0), 1,
+                _ptr(b), b.stride(0), b.stride(1), _ptr(o3), o3.stride(1), slices, _ptr(ws), _ptr(bias), epi)
+            _check(rc, "mk_gemm_splitk_typed")
+            return out[0] if out.dim() == 3 else out
     rc = lib().mk_gemm(
         _stream(stream), mk_dtype(a.dtype), mk_dtype(out_dtype), batch, M, N, K,
         _ptr(a3), a3.stride(0), a3.stride(1), a3.stride(2),

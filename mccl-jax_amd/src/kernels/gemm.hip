@@ -392,6 +392,11 @@ extern "C" int mk_gemm(void* stream, int ab_type, int c_type, int64_t batch, int
   a.vec_a = al16(A) && (a_bs % vec == 0) && ((a_kc ? a.a_ms : a.a_ks) % vec == 0);
   a.vec_b = al16(B) && (b_bs % vec == 0) && ((b_kc ? a.b_ns : a.b_ks) % vec == 0);
   hipStream_t s = as_stream(stream);
+  // few rows: one pass over B whatever its size, strides and alignment
+  if (const int r = gemm_skinny(s, ab_type, c_type, batch, M, N, K, A, a_bs, a.a_ms, a.a_ks, B, b_bs, a.b_ks, a.b_ns,
+                                C, c_bs, c_ms, bias, epilogue);
+      r >= 0)
+    return r;
   if (ab_type == MK_BF16) {
     const int r = gemm_tiled(s, c_type, batch, M, N, K, A, a_bs, a_ms, a_ks, B, b_bs, b_ks, b_ns, C, c_bs,
                              c_ms, bias, epilogue);
@@ -423,6 +428,21 @@ extern "C" int mk_gemm_splitk_typed(void* stream, int ab_type, int c_type, int64
   if ((N % 4) != 0 || (c_ms % 4) != 0 || (reinterpret_cast<uintptr_t>(C) & cal) ||
       (reinterpret_cast<uintptr_t>(workspace) & 15u))
     return fail(MK_ERR_UNSUPPORTED, "mk_gemm_splitk: N and c_ms multiples of 4, aligned C and workspace");
+  // few rows: the kernel that takes them splits k inside the workgroup, and
+  // over workgroups only where the columns alone leave the chip idle
+  if (gemm_skinny_fits(M, N, K, a_ks, b_ks, b_ns)) {
+    const int64_t slices = gemm_skinny_slices(ab_type, N, K, splits);
+    if (slices == 1 || !A || !B)
+      return mk_gemm(stream, ab_type, c_type, 1, M, N, K, A, 0, a_ms, a_ks, B, 0, b_ks, b_ns, C, 0, c_ms, bias,
+                     epilogue);
+    if (ab_type != MK_BF16 && ab_type != MK_F32)
+      return fail(MK_ERR_UNSUPPORTED, "mk_gemm: ab_type must be bf16 or f32");
+    if (int rc = gemm_skinny(as_stream(stream), ab_type, MK_F32, 1, M, N, K, A, 0, a_ms, a_ks, B, 0, b_ks, b_ns,
+                             workspace, M * N, N, nullptr, 0, slices))
+      return rc;
+    return splitk_sum(as_stream(stream), static_cast<const float*>(workspace), slices, M, N, C, c_ms, "mk_gemm_splitk",
+                      c_type, bias, epilogue);
+  }
   float* W = static_cast<float*>(workspace);
   hipStream_t s = as_stream(stream);
   if (K % splits == 0) {

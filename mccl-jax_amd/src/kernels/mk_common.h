@@ -51,6 +51,18 @@ int gemm_tiled(hipStream_t s, int c_type, int64_t batch, int64_t M, int64_t N, i
                int64_t b_ns, void* C, int64_t c_bs, int64_t c_ms, const void* bias, int epilogue,
                int64_t k_rem = 0, void* Y = nullptr, int64_t y_ms = 0, float* colpart = nullptr);
 
+// GEMM with at most 64 rows behind mk_gemm (gemm_skinny.hip), same operand
+// convention, A k-contiguous; returns -1 without launching when the shape or
+// strides do not fit it (gemm_skinny_fits), else MK_OK or an MK_ERR_* code.
+// slices > 1 (batch 1): slice i of k writes its partial product at C + i c_bs;
+// gemm_skinny_slices: how many of at most `most` slices pay.
+bool gemm_skinny_fits(int64_t M, int64_t N, int64_t K, int64_t a_ks, int64_t b_ks, int64_t b_ns);
+int gemm_skinny(hipStream_t s, int ab_type, int c_type, int64_t batch, int64_t M, int64_t N, int64_t K,
+                const void* A, int64_t a_bs, int64_t a_ms, int64_t a_ks, const void* B, int64_t b_bs, int64_t b_ks,
+                int64_t b_ns, void* C, int64_t c_bs, int64_t c_ms, const void* bias, int epilogue,
+                int64_t slices = 1);
+int64_t gemm_skinny_slices(int ab_type, int64_t N, int64_t K, int64_t most);
+
 // Flash attention backward behind mk_sdpa_bwd for head_dim 64 / 128
 // (attention_bwd.hip); workspace: the per-row statistics.
 size_t sdpa_bwd_flash_workspace(int64_t B, int64_t H, int64_t Sq);

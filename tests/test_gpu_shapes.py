@@ -91,3 +91,48 @@ def test_add_layernorm_f32_wide(K, rows, cols):
     assert np.all(np.abs(y.cpu().double().numpy() - want) <= 1e-5 * scale)
     _, y16 = K.add_layernorm(a.cuda(), b.cuda(), None, gamma.cuda(), beta.cuda(), out_dtype=torch.bfloat16)
     assert torch.equal(y16.cpu(), y.cpu().bfloat16())
+
+
+# few-row products: rows around the 16-row blocks, columns around the 16/32/64-column tiles, k
+# around the 32-deep steps and the waves' shares, both orientations of B, rows off alignment
+SKINNY = [(1, 16, 1), (1, 17, 31), (5, 63, 33), (16, 100, 96), (17, 64, 1000), (33, 129, 515), (64, 4096, 256),
+          (64, 33, 40), (3, 12352, 130), (49, 12301, 64)]
+
+
+@pytest.mark.parametrize("M,N,K_", SKINNY)
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("b_kc", [False, True])
+def test_gemm_few_rows(K, M, N, K_, dtype, b_kc):
+    """C = relu(A B + bias) with NaN past every row end in memory: fp32 sums
+    within 2^-23 sqrt(K) of the magnitudes (factor 8), one rounding to C."""
+    print(f"case: gemm {M}x{N}x{K_} {dtype} b_kc={b_kc}", flush=True)
+    g = torch.Generator().manual_seed(M * 1000 + N + K_)
+    a, b, bias = torch.randn(M, K_, generator=g), torch.randn(K_, N, generator=g), torch.randn(N, generator=g)
+    a, b, bias = a.to(dtype), b.to(dtype), bias.to(dtype)
+    nan = float("nan")
+    ad = torch.full((M, K_ + 3), nan, dtype=dtype, device="cuda")[:, 1:K_ + 1]
+    ad.copy_(a)
+    rows, cols = (N, K_) if b_kc else (K_, N)
+    bd = torch.full((rows, cols + 5), nan, dtype=dtype, device="cuda")[:, 2:cols + 2]
+    bd.copy_(b.t() if b_kc else b)
+    out = torch.full((M + 1, N + 1), 7.0, dtype=dtype, device="cuda")
+    K.gemm(ad, bd.t() if b_kc else bd, bias=bias.cuda(), relu=True, out=out[:M, :N])
+    ad_, bd_ = a.double(), b.double()
+    want = torch.relu(ad_ @ bd_ + bias.double())
+    mag = ad_.abs() @ bd_.abs() + bias.double().abs()
+    bound = 8 * 2.0 ** -23 * mag + (2.0 ** -8 if dtype == torch.bfloat16 else 0) * want.abs()
+    assert bool(((out[:M, :N].cpu().double() - want).abs() <= bound).all())
+    assert bool((out[M] == 7).all()) and bool((out[:, N] == 7).all())
+
+
+def test_gemm_few_rows_batched_and_split(K):
+    """Batches with a broadcast B, and the split-K entry at few rows."""
+    g = torch.Generator().manual_seed(3)
+    a, b = torch.randn(5, 7, 100, generator=g), torch.randn(100, 48, generator=g)
+    got = K.gemm(a.cuda(), b.cuda())
+    want = a.double() @ b.double()
+    assert bool(((got.cpu().double() - want).abs() <= 8 * 2.0 ** -23 * (a.double().abs() @ b.double().abs())).all())
+    x, w = torch.randn(9, 1024, generator=g).bfloat16(), torch.randn(1024, 64, generator=g).bfloat16()
+    got = K.gemm_splitk(x.cuda(), w.cuda(), 4)
+    want = x.double() @ w.double()
+    assert bool(((got.cpu().double() - want).abs() <= 8 * 2.0 ** -23 * (x.double().abs() @ w.double().abs())).all())

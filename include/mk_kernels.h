@@ -186,6 +186,18 @@ int mk_sdpa_fwd(void* stream, int64_t B, int64_t H, int64_t Sq, int64_t Sk, int6
                 void* o, int64_t o_bs, int64_t o_hs, int64_t o_ss,
                 float scale, int causal, float* lse);
 
+/* mk_sdpa_fwd with a workspace of mk_sdpa_fwd_workspace_bytes (0 bytes: none
+ * is used; NULL: mk_sdpa_fwd): with at most 16 queries, no causal mask and too
+ * few heads to fill the chip, the keys are cut into runs whose partial
+ * results are merged in order by a second launch. */
+size_t mk_sdpa_fwd_workspace_bytes(int64_t B, int64_t H, int64_t Sq, int64_t Sk, int64_t D, int causal);
+int mk_sdpa_fwd_ws(void* stream, int64_t B, int64_t H, int64_t Sq, int64_t Sk, int64_t D,
+                   const void* q, int64_t q_bs, int64_t q_hs, int64_t q_ss,
+                   const void* k, int64_t k_bs, int64_t k_hs, int64_t k_ss,
+                   const void* v, int64_t v_bs, int64_t v_hs, int64_t v_ss,
+                   void* o, int64_t o_bs, int64_t o_hs, int64_t o_ss,
+                   float scale, int causal, float* lse, void* workspace);
+
 /* ------------------------------------------------------------------------
  * a8  row reduction over the innermost (contiguous) axis.
  * Replaces: src/jam/ops/reduce.mm:97-106 (reductionSum/Max/Min/Product).

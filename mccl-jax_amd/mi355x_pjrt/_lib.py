@@ -45,6 +45,13 @@ SIGNATURES = {
                          _P, _I64, _I64, _I64,
                          _P, _I64, _I64, _I64,
                          _F, _I, _P]),
+    "mk_sdpa_fwd_workspace_bytes": (ctypes.c_size_t, [_I64, _I64, _I64, _I64, _I64, _I]),
+    "mk_sdpa_fwd_ws": (_I, [_P, _I64, _I64, _I64, _I64, _I64,
+                            _P, _I64, _I64, _I64,
+                            _P, _I64, _I64, _I64,
+                            _P, _I64, _I64, _I64,
+                            _P, _I64, _I64, _I64,
+                            _F, _I, _P, _P]),
     "mk_row_reduce": (_I, [_P, _I, _I, _I, _I64, _I64, _P, _F, _P]),
     "mk_row_argmax": (_I, [_P, _I, _I, _I64, _I64, _P, _P, _I, _P]),
     "mk_layernorm": (_I, [_P, _I, _I64, _I64, _P, _P, _P, _F, _P]),

@@ -69,13 +69,17 @@ def sdpa_fwd(q, k, v, scale: float, causal: bool = True, out=None, lse=None, str
             raise ValueError("sdpa_fwd: bf16 tensors with contiguous head_dim")
     if out is None:
         out = torch.empty((B, H, Sq, D), dtype=torch.bfloat16, device=q.device)
-    rc = lib().mk_sdpa_fwd(
+    ws = None
+    if Sq <= 16 and Sk >= 512 and not causal and stream is None:  # few queries: the keys may be cut over workgroups
+        nbytes = lib().mk_sdpa_fwd_workspace_bytes(B, H, Sq, Sk, D, 0)
+        ws = torch.empty(nbytes, dtype=torch.uint8, device=q.device) if nbytes else None
+    rc = lib().mk_sdpa_fwd_ws(
         _stream(stream), B, H, Sq, Sk, D,
         _ptr(q), q.stride(0), q.stride(1), q.stride(2),
         _ptr(k), k.stride(0), k.stride(1), k.stride(2),
         _ptr(v), v.stride(0), v.stride(1), v.stride(2),
         _ptr(out), out.stride(0), out.stride(1), out.stride(2),
-        float(scale), int(bool(causal)), _ptr(lse))
+        float(scale), int(bool(causal)), _ptr(lse), _ptr(ws))
     _check(rc, "mk_sdpa_fwd")
     return out
 

@@ -823,12 +823,27 @@ __global__ __launch_bounds__(256, 1) void sdpa_fwd_wide_kernel(const SdpaArgs p)
 
 using namespace mk;
 
+extern "C" size_t mk_sdpa_fwd_workspace_bytes(int64_t B, int64_t H, int64_t Sq, int64_t Sk, int64_t D, int causal) {
+  if (B <= 0 || H <= 0 || Sq <= 0 || !sdpa_decode_fits(Sq, Sk, causal)) return 0;
+  return sdpa_decode_workspace(B * H, Sq, Sk, D);
+}
+
 extern "C" int mk_sdpa_fwd(void* stream, int64_t B, int64_t H, int64_t Sq, int64_t Sk, int64_t D,
                            const void* q, int64_t q_bs, int64_t q_hs, int64_t q_ss,
                            const void* k, int64_t k_bs, int64_t k_hs, int64_t k_ss,
                            const void* v, int64_t v_bs, int64_t v_hs, int64_t v_ss,
                            void* o, int64_t o_bs, int64_t o_hs, int64_t o_ss,
                            float scale, int causal, float* lse) {
+  return mk_sdpa_fwd_ws(stream, B, H, Sq, Sk, D, q, q_bs, q_hs, q_ss, k, k_bs, k_hs, k_ss, v, v_bs, v_hs, v_ss, o,
+                        o_bs, o_hs, o_ss, scale, causal, lse, nullptr);
+}
+
+extern "C" int mk_sdpa_fwd_ws(void* stream, int64_t B, int64_t H, int64_t Sq, int64_t Sk, int64_t D,
+                              const void* q, int64_t q_bs, int64_t q_hs, int64_t q_ss,
+                              const void* k, int64_t k_bs, int64_t k_hs, int64_t k_ss,
+                              const void* v, int64_t v_bs, int64_t v_hs, int64_t v_ss,
+                              void* o, int64_t o_bs, int64_t o_hs, int64_t o_ss,
+                              float scale, int causal, float* lse, void* workspace) {
   clear_error();
   if (B < 0 || H < 0 || Sq < 0 || Sk < 0) return fail(MK_ERR_INVALID, "mk_sdpa_fwd: negative shape");
   if (D != 64 && D != 128) return fail(MK_ERR_UNSUPPORTED, "mk_sdpa_fwd: head_dim must be 64 or 128");
@@ -847,6 +862,9 @@ extern "C" int mk_sdpa_fwd(void* stream, int64_t B, int64_t H, int64_t Sq, int64
     return fail(MK_ERR_UNSUPPORTED, "mk_sdpa_fwd: q/k/v need 16-byte aligned rows (strides % 8 == 0), o strides % 4 == 0");
   if (k_ss < D || v_ss < D || k_ss >= (int64_t(1) << 24) || v_ss >= (int64_t(1) << 24))
     return fail(MK_ERR_UNSUPPORTED, "mk_sdpa_fwd: k/v sequence strides must be in [D, 2^24)");
+  if (sdpa_decode_fits(Sq, Sk, causal))
+    return sdpa_decode(as_stream(stream), B, H, Sq, Sk, D, q, q_bs, q_hs, q_ss, k, k_bs, k_hs, k_ss, v, v_bs, v_hs,
+                       v_ss, o, o_bs, o_hs, o_ss, scale, lse, workspace);
   SdpaArgs a;
   a.q = (const uint16_t*)q; a.k = (const uint16_t*)k; a.v = (const uint16_t*)v; a.o = (uint16_t*)o;
   a.lse = lse;

@@ -136,3 +136,45 @@ def test_gemm_few_rows_batched_and_split(K):
     got = K.gemm_splitk(x.cuda(), w.cuda(), 4)
     want = x.double() @ w.double()
     assert bool(((got.cpu().double() - want).abs() <= 8 * 2.0 ** -23 * (x.double().abs() @ w.double().abs())).all())
+
+
+# few queries: key counts around the 32-key steps, the 4 waves' shares and the 256-key slices
+@pytest.mark.parametrize("B,H,Sq,Sk,D", [(1, 1, 1, 1, 128), (2, 3, 1, 31, 64), (1, 2, 7, 33, 128), (1, 2, 16, 129, 64),
+                                         (2, 2, 1, 511, 128), (1, 2, 2, 513, 128), (1, 3, 16, 2049, 128),
+                                         (3, 5, 4, 1000, 64), (1, 1, 1, 16391, 128), (32, 16, 1, 300, 64)])
+@pytest.mark.parametrize("slices", [True, False])
+def test_sdpa_few_queries(K, B, H, Sq, Sk, D, slices):
+    """O and lse against float64 softmax; the cache holds NaN past its keys.
+    Each probability is rounded to bf16 (2^-8) in numerator and sum, O once."""
+    print(f"case: sdpa {B}x{H} Sq={Sq} Sk={Sk} D={D} slices={slices}", flush=True)
+    g = torch.Generator().manual_seed(Sk * 31 + Sq)
+    q = torch.randn(B, Sq, H, D, generator=g).bfloat16().transpose(1, 2)
+    k, v = (torch.randn(B, H, Sk, D, generator=g).bfloat16() for _ in range(2))
+    q[:, :, 0] *= 6  # a peaked row beside flat ones
+    room = torch.full((2, B, H, Sk + 40, D), float("nan"), dtype=torch.bfloat16, device="cuda")
+    kd, vd = room[0, :, :, :Sk], room[1, :, :, :Sk]
+    kd.copy_(k)
+    vd.copy_(v)
+    out = torch.full((B, H, Sq, D), float("nan"), dtype=torch.bfloat16, device="cuda")
+    lse = torch.full((B, H, Sq), float("nan"), device="cuda")
+    # an explicit stream runs without a workspace: one workgroup per head
+    K.sdpa_fwd(q.cuda(), kd, vd, D ** -0.5, causal=False, out=out, lse=lse,
+               stream=None if slices else torch.cuda.current_stream())
+    s = (q.double() @ k.double().transpose(-1, -2)) * D ** -0.5
+    p = torch.softmax(s, -1)
+    want, u = p @ v.double(), 2.0 ** -8
+    bound = 2 * u * (p @ v.double().abs()) + u * want.abs() + 1e-6
+    assert bool(((out.cpu().double() - want).abs() <= bound).all())
+    assert bool(((lse.cpu().double() - torch.logsumexp(s, -1)).abs() <= u + 1e-5).all())
+
+
+def test_sdpa_few_queries_infinities(K):
+    """Scores of -inf at the first keys do not poison later ones, and a NaN
+    key makes exactly its head NaN."""
+    q = torch.ones(1, 3, 2, 64, dtype=torch.bfloat16, device="cuda")
+    k = torch.ones(1, 3, 700, 64, dtype=torch.bfloat16, device="cuda")
+    v = torch.ones(1, 3, 700, 64, dtype=torch.bfloat16, device="cuda") * 2
+    k[0, 0, :650] = -float("inf")
+    k[0, 1, 699, 3] = float("nan")
+    o = K.sdpa_fwd(q, k, v, 0.125, causal=False)
+    assert bool((o[0, 0] == 2).all()) and bool(o[0, 1].isnan().all()) and bool((o[0, 2] == 2).all())

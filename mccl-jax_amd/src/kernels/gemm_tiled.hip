@@ -254,6 +254,11 @@ __device__ inline void finish4(const TiledGemm& p, int64_t n, float (&v)[4]) {
 // rows 2 apart share the bank offset).  Then the workgroup stores runs of consecutive
 // C rows: whole 16-byte chunks when C rows are 16-byte aligned (ROWS16),
 // else one element per thread, consecutive threads on consecutive columns.
+// The chunks are stored non-temporally: a round of workgroups writes as much
+// as an XCD's whole L2 holds (32 tiles of 96 or 128 KB), which evicted the
+// operand rows and columns its next round shares.  8192 x 50257 x 768 with
+// bf16 C: 775 -> 703 us on 256 x 256 tiles, 764 -> 668 us on 128 x 192.  fp32
+// C keeps ordinary stores (no gain, and split-K slices are read back at once).
 template <int CT, bool ROWS16, int TM, int TN, int kW, int kWM, int kWN, int kI, int kJ>
 __device__ __attribute__((always_inline)) inline void store_staged(const TiledGemm& p,
                                                                    const f32x16_t (&acc)[kI][kJ], uint16_t* st,
@@ -338,8 +343,9 @@ __device__ __attribute__((always_inline)) inline void store_staged(const TiledGe
       *reinterpret_cast<u32x4_t*>(st + row * TN + 8 * pos(row, cn)) = v;
     }
     if (m < p.M && n + 8 <= p.N) {
-      *reinterpret_cast<u32x4_t*>(Cz + 2 * (m * p.ldc + n)) = v;
-      if (p.epilogue & kEpiGeluAux) *reinterpret_cast<u32x4_t*>(p.aux + m * p.ld_aux + n) = gelu8_bf16(v);
+      __builtin_nontemporal_store(v, reinterpret_cast<u32x4_t*>(Cz + 2 * (m * p.ldc + n)));
+      if (p.epilogue & kEpiGeluAux)
+        __builtin_nontemporal_store(gelu8_bf16(v), reinterpret_cast<u32x4_t*>(p.aux + m * p.ld_aux + n));
     } else if (m < p.M && n < p.N) {  // the chunk that straddles N: its columns below N only
       uint16_t* Ce = reinterpret_cast<uint16_t*>(Cz) + m * p.ldc + n;
       const u32x4_t gv = gelu8_bf16(v);
@@ -756,20 +762,23 @@ int gemm_tiled(hipStream_t s, int c_type, int64_t batch, int64_t M, int64_t N, i
   if (!tiled_args(a, a_kc, b_kc, c_type, batch, M, N, K, A, a_bs, a_ms, a_ks, B, b_bs, b_ks, b_ns, C, c_bs, c_ms,
                   bias, epilogue, k_rem, Y, y_ms, colpart))
     return -1;
-  // Kernel shape: the one with the least estimated time.  Each shape has a
-  // throughput per CU measured on a large product (8192 x 8192 x 4096: 1240,
-  // 1083 and 1017 TFLOP/s) and a number of workgroups a CU holds at once (one
-  // 256 x 256 workgroup, two of the smaller ones).  Whole rounds of
-  // workgroups over the CUs run at that throughput; a last partial round
-  // that leaves every workgroup alone on its CU runs each at about 0.8 of it
-  // (a CU's throughput with one 8-wave workgroup instead of two, measured on
-  // the 8192 x 768 products with K = 768 .. 3072).
+  // Kernel shape: the one with the least estimated time.  A round of
+  // workgroups costs nk + e k tiles, each of its area over the shape's rate:
+  // the rate per CU in the k loop and e, the first loads and the epilogue in
+  // k tiles (twice that for fp32 C), are fitted to 8192 x 8192 x 4096 and
+  // 8192 x 50257 x 768 (256 x 256: 437 and 703 us; 128 x 192: 485 and 668;
+  // 128 x 128: 521 and 740).  A CU holds one 256 x 256 workgroup or two of
+  // the smaller ones.  A last partial round that leaves every workgroup alone
+  // on its CU runs each at about 0.8 of the pair's rate (8192 x 768 products,
+  // K = 768 .. 3072), and one on fewer than half of the CUs takes about 0.8
+  // of a full round of 256 x 256 tiles.
   struct Option {
     int tm, tn, per_cu;
-    double rate;
+    double rate, e;
   };
-  static const Option options[3] = {{256, 256, 1, 1240.0}, {128, 192, 2, 1083.0}, {128, 128, 2, 1017.0}};
+  static const Option options[3] = {{256, 256, 1, 1240.0, 7.5}, {128, 192, 2, 1120.0, 5.3}, {128, 128, 2, 971.0, 3.3}};
   const int64_t cus = cu_count();
+  const double nk = double((K + 63) / 64);
   int best = -1;
   double best_t = 0;
   for (int o = 0; o < 3; ++o) {
@@ -777,9 +786,12 @@ int gemm_tiled(hipStream_t s, int c_type, int64_t batch, int64_t M, int64_t N, i
     if (M < op.tm || N < op.tn) continue;
     const int64_t tiles = ((M + op.tm - 1) / op.tm) * ((N + op.tn - 1) / op.tn) * batch;
     const int64_t slots = cus * op.per_cu, rem = tiles % slots;
-    const double tile = double(op.tm) * op.tn / op.rate;
+    const double tile = double(op.tm) * op.tn / op.rate * (nk + (c_type == MK_F32 ? 2 * op.e : op.e));
     double t = double(tiles / slots) * op.per_cu * tile;
-    if (rem > 0) t += (op.per_cu > 1 && rem <= cus) ? tile / 0.8 : op.per_cu * tile;
+    if (rem > 0) {
+      if (op.per_cu > 1) t += rem <= cus ? tile / 0.8 : op.per_cu * tile;
+      else t += 2 * rem < cus ? 0.8 * tile : tile;
+    }
     if (best < 0 || t < best_t) best = o, best_t = t;
   }
   if (best == 0) return launch<Shape<256, 256, 2, 4, 64, 2>>(s, a, batch, a_kc, b_kc);

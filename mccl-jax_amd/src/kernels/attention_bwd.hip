@@ -7,7 +7,7 @@
 //   dV = Pᵀ dO,  dK = scale dSᵀ Q,  dQ = scale dS K.
 // Three launches, none with atomics, so results are deterministic:
 //   stats  D_r and lse_r · log2(e) per query row, packed per 64-row tile
-//          ([bh][tile][lse2 x 64 | D x 64]; rows past Sq: +inf, 0, which
+//          ([bh][tile][lse2 x 64 | -D x 64]; rows past Sq: +inf, 0, which
 //          makes their P and dS exactly 0);
 //   kv     one workgroup per 128 keys of one (b, h), wave w owning keys
 //          32 w .. 32 w + 31: dVᵀ and dKᵀ accumulate in registers while
@@ -26,6 +26,14 @@
 // q: Sᵀ = K Qᵀ with the wave's queries as columns (Q, dO fragments in
 // registers), a lane owns one query (one lse2 and D in registers), and
 // dSᵀ is the B operand of dQᵀ = Kᵀ dSᵀ (Kᵀ read transposed from LDS).
+//
+// Bound: VALU beside the MFMAs (per score: an FMA, an exponential, a multiply,
+// two conversions; 4 + 3 products of 64 or 128 deep).  So the masks run only
+// on blocks that hold the diagonal or the last keys (wave-uniform branches),
+// dP accumulates from -D instead of subtracting it after, and the file is
+// compiled with MFMA results in VGPRs (in AGPRs every score and dP was moved
+// with v_accvgpr_read first).  Forward and backward, 96 heads x 1024 x 64
+// causal 123 -> 106 us; 64 x 4096 x 64 772 -> 649; 32 x 4096 x 128 780 -> 680.
 //
 // Tiles are copied HBM -> LDS with buffer_load ... lds, double-buffered: the
 // copy of tile t+1 is issued before tile t is computed, and each wave waits
@@ -70,41 +78,41 @@ struct BwdArgs {
 };
 
 // ---------------------------------------------------------------- stats
+// D / 8 consecutive lanes per row, 16 bytes of O and dO each: a wave reads whole
+// rows (a thread per row read 16 bytes of 64 rows per instruction: 8.8 -> 5.6 us
+// for 96 x 1024 rows of 64).
 template <int D>
 __global__ __launch_bounds__(256) void attn_bwd_stats_kernel(const BwdArgs p, const uint16_t* __restrict__ o,
                                                             int64_t o_bs, int64_t o_hs, int64_t o_ss,
                                                             const float* __restrict__ lse,
                                                             float* __restrict__ stats) {
-  const int64_t t = int64_t(blockIdx.x) * 256 + threadIdx.x;
+  constexpr int L = D / 8;
+  const int64_t t = (int64_t(blockIdx.x) * 256 + threadIdx.x) / L;
+  const int ch = int(threadIdx.x) % L;
   const int64_t per = int64_t(p.n_qt) * kTile;
-  if (t >= int64_t(p.BH) * per) return;
+  if (t >= int64_t(p.BH) * per) return;  // whole rows: the 8 or 16 lanes of one leave together
   const int64_t bh = t / per;
   const int row = int(t % per);
   float l2 = INFINITY, dsum = 0.f;
   if (row < p.Sq) {
     const int64_t b = bh / p.H, h = bh % p.H;
-    const uint16_t* orow = o + b * o_bs + h * o_hs + row * o_ss;
-    const uint16_t* drow = p.dout + b * p.do_bs + h * p.do_hs + row * p.do_ss;
-    u32x4_t av[D / 8], cv[D / 8];  // all of the row's loads in flight before any use
-#pragma unroll
-    for (int k = 0; k < D / 8; ++k) {
-      av[k] = *reinterpret_cast<const u32x4_t*>(orow + 8 * k);
-      cv[k] = *reinterpret_cast<const u32x4_t*>(drow + 8 * k);
-    }
-#pragma unroll
-    for (int k = 0; k < D / 8; ++k) {
-      const u32x4_t a = av[k], c = cv[k];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        dsum += __builtin_bit_cast(float, a[j] << 16) * __builtin_bit_cast(float, c[j] << 16);
-        dsum += __builtin_bit_cast(float, a[j] & 0xFFFF0000u) * __builtin_bit_cast(float, c[j] & 0xFFFF0000u);
-      }
-    }
+    const u32x4_t a = *reinterpret_cast<const u32x4_t*>(o + b * o_bs + h * o_hs + row * o_ss + 8 * ch);
+    const u32x4_t c =
+        *reinterpret_cast<const u32x4_t*>(p.dout + b * p.do_bs + h * p.do_hs + row * p.do_ss + 8 * ch);
     l2 = lse[bh * p.Sq + row] * kLog2e;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      dsum += __builtin_bit_cast(float, a[j] << 16) * __builtin_bit_cast(float, c[j] << 16);
+      dsum += __builtin_bit_cast(float, a[j] & 0xFFFF0000u) * __builtin_bit_cast(float, c[j] & 0xFFFF0000u);
+    }
   }
-  float* st = stats + (bh * p.n_qt + row / kTile) * (2 * kTile);
-  st[row % kTile] = l2;
-  st[kTile + row % kTile] = dsum;
+#pragma unroll
+  for (int x = L / 2; x >= 1; x >>= 1) dsum += __shfl_xor(dsum, x, kWave);
+  if (ch == 0) {
+    float* st = stats + (bh * p.n_qt + row / kTile) * (2 * kTile);
+    st[row % kTile] = l2;
+    st[kTile + row % kTile] = -dsum;
+  }
 }
 
 // ---------------------------------------------------------------- tile copies
@@ -167,7 +175,7 @@ __global__ __launch_bounds__(kThreadsB) void sdpa_bwd_kv_kernel(const BwdArgs p)
 
   __shared__ __attribute__((aligned(1024))) uint16_t Qs[2][TC::ELEMS];
   __shared__ __attribute__((aligned(1024))) uint16_t Ds[2][TC::ELEMS];
-  __shared__ __attribute__((aligned(1024))) float Ss[2][256];  // lse2[64], D[64], then the zeros of the copy
+  __shared__ __attribute__((aligned(1024))) float Ss[2][256];  // lse2[64], -D[64], then the zeros of the copy
 
   // earliest key blocks (most queries) first; consecutive ids walk the heads
   const int id = blockIdx.x;
@@ -235,9 +243,15 @@ __global__ __launch_bounds__(kThreadsB) void sdpa_bwd_kv_kernel(const BwdArgs p)
       const int qm0 = t * kTile + 32 * mt;
       live[mt] = qm0 < p.Sq && (!CAUSAL || qm0 + 31 >= kw0);  // wave-uniform
       if (!live[mt]) continue;
+      // rows of reg r: query qm0 + 8 (r/4) + 4 g + r%4; dP starts from -D
       f32x16_t s, dp;
 #pragma unroll
-      for (int r = 0; r < 16; ++r) s[r] = dp[r] = 0.f;
+      for (int r4 = 0; r4 < 4; ++r4) {
+        const float4 dd = *reinterpret_cast<const float4*>(&st[kTile + 32 * mt + 8 * r4 + 4 * g]);
+        dp[4 * r4] = dd.x, dp[4 * r4 + 1] = dd.y, dp[4 * r4 + 2] = dd.z, dp[4 * r4 + 3] = dd.w;
+      }
+#pragma unroll
+      for (int r = 0; r < 16; ++r) s[r] = 0.f;
 #pragma unroll
       for (int ks = 0; ks < NKS; ++ks) {
         const u32x4_t a = *reinterpret_cast<const u32x4_t*>(&Q[rlane + 32 * mt * RS + 16 * ks]);
@@ -248,23 +262,22 @@ __global__ __launch_bounds__(kThreadsB) void sdpa_bwd_kv_kernel(const BwdArgs p)
         const u32x4_t a = *reinterpret_cast<const u32x4_t*>(&DO[rlane + 32 * mt * RS + 16 * ks]);
         dp = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(a), vf[ks], dp, 0, 0, 0);
       }
-      // rows of reg r: query qm0 + 8 (r/4) + 4 g + r%4
       float pr[16], ds[16];
 #pragma unroll
       for (int r4 = 0; r4 < 4; ++r4) {
-        const int row = 32 * mt + 8 * r4 + 4 * g;
-        const float4 l2 = *reinterpret_cast<const float4*>(&st[row]);
-        const float4 dd = *reinterpret_cast<const float4*>(&st[kTile + row]);
-        const float lv[4] = {l2.x, l2.y, l2.z, l2.w}, dv4[4] = {dd.x, dd.y, dd.z, dd.w};
+        const float4 l2 = *reinterpret_cast<const float4*>(&st[32 * mt + 8 * r4 + 4 * g]);
+        const float lv[4] = {l2.x, l2.y, l2.z, l2.w};
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int r = 4 * r4 + i;
-          float pv = __builtin_amdgcn_exp2f(fmaf(s[r], p.scale_log2, -lv[i]));
-          if (CAUSAL && key > t * kTile + row + i) pv = 0.f;
-          pr[r] = pv;
-          ds[r] = pv * (dp[r] - dv4[i]);
-        }
+        for (int i = 0; i < 4; ++i)
+          pr[4 * r4 + i] = __builtin_amdgcn_exp2f(fmaf(s[4 * r4 + i], p.scale_log2, -lv[i]));
       }
+      if (CAUSAL && kw0 + 31 > qm0) {  // wave-uniform: blocks on the diagonal
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+          if (key > qm0 + 8 * (r / 4) + 4 * g + r % 4) pr[r] = 0.f;
+      }
+#pragma unroll
+      for (int r = 0; r < 16; ++r) ds[r] = pr[r] * dp[r];
 #pragma unroll
       for (int j2 = 0; j2 < 2; ++j2) {
         const int o = 8 * j2;
@@ -342,7 +355,7 @@ __global__ __launch_bounds__(kThreadsB) void sdpa_bwd_q_kernel(const BwdArgs p) 
 
   // Q, dO fragments (B operands of Sᵀ = K Qᵀ and dPᵀ = V dOᵀ) and the row's stats
   bf16x8_t qf[NKS], df[NKS];
-  float l2 = INFINITY, dsum = 0.f;
+  float l2 = INFINITY, dneg = 0.f;
   {
     const bool ok = qrow < p.Sq;
     const uint16_t* qr = p.q + b * p.q_bs + h * p.q_hs + int64_t(qrow) * p.q_ss;
@@ -360,7 +373,7 @@ __global__ __launch_bounds__(kThreadsB) void sdpa_bwd_q_kernel(const BwdArgs p) 
     if (ok) {
       const float* st = p.stats + (int64_t(bh) * p.n_qt + qrow / kTile) * (2 * kTile) + qrow % kTile;
       l2 = st[0];
-      dsum = st[kTile];
+      dneg = st[kTile];
     }
     __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
   }
@@ -382,6 +395,9 @@ __global__ __launch_bounds__(kThreadsB) void sdpa_bwd_q_kernel(const BwdArgs p) 
   const int rlane = c * RS + 8 * g;
   const int tlane = (4 * g + ((lane & 15) >> 2)) * RS + 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
 
+  f32x16_t dinit;  // -D of the lane's query, where every dP product starts
+#pragma unroll
+  for (int r = 0; r < 16; ++r) dinit[r] = dneg;
   f32x16_t dq[NDB];
 #pragma unroll
   for (int db = 0; db < NDB; ++db)
@@ -397,9 +413,9 @@ __global__ __launch_bounds__(kThreadsB) void sdpa_bwd_q_kernel(const BwdArgs p) 
       const int kk0 = t * kTile + 32 * kb2;
       live[kb2] = kk0 < p.Sk && (!CAUSAL || kk0 <= q0 + 31);  // wave-uniform
       if (!live[kb2]) continue;
-      f32x16_t s, dp;
+      f32x16_t s, dp = dinit;
 #pragma unroll
-      for (int r = 0; r < 16; ++r) s[r] = dp[r] = 0.f;
+      for (int r = 0; r < 16; ++r) s[r] = 0.f;
 #pragma unroll
       for (int ks = 0; ks < NKS; ++ks) {
         const u32x4_t a = *reinterpret_cast<const u32x4_t*>(&K[rlane + 32 * kb2 * RS + 16 * ks]);
@@ -411,14 +427,18 @@ __global__ __launch_bounds__(kThreadsB) void sdpa_bwd_q_kernel(const BwdArgs p) 
         dp = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(a), df[ks], dp, 0, 0, 0);
       }
       // rows of reg r: key kk0 + 8 (r/4) + 4 g + r%4
-      float ds[16];
+      float pr[16], ds[16];
 #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int kk = kk0 + 8 * (r / 4) + 4 * g + (r % 4);
-        float pv = __builtin_amdgcn_exp2f(fmaf(s[r], p.scale_log2, -l2));
-        if (kk >= p.Sk || (CAUSAL && kk > qrow)) pv = 0.f;
-        ds[r] = pv * (dp[r] - dsum);
+      for (int r = 0; r < 16; ++r) pr[r] = __builtin_amdgcn_exp2f(fmaf(s[r], p.scale_log2, -l2));
+      if (kk0 + 31 >= p.Sk || (CAUSAL && kk0 + 31 > q0)) {  // wave-uniform: the last keys, the diagonal
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const int kk = kk0 + 8 * (r / 4) + 4 * g + (r % 4);
+          if (kk >= p.Sk || (CAUSAL && kk > qrow)) pr[r] = 0.f;
+        }
       }
+#pragma unroll
+      for (int r = 0; r < 16; ++r) ds[r] = pr[r] * dp[r];
 #pragma unroll
       for (int j2 = 0; j2 < 2; ++j2) {
         const int o = 8 * j2;
@@ -514,7 +534,7 @@ int sdpa_bwd_flash(hipStream_t s, int64_t B, int64_t H, int64_t Sq, int64_t Sk, 
   a.scale_log2 = scale * kLog2e;
   a.scale = scale;
 
-  const int64_t nstat = int64_t(a.BH) * a.n_qt * kTile;
+  const int64_t nstat = int64_t(a.BH) * a.n_qt * kTile * (D / 8);  // lanes
   if (D == 128)
     hipLaunchKernelGGL(attn_bwd_stats_kernel<128>, dim3(unsigned((nstat + 255) / 256)), dim3(256), 0, s, a,
                        (const uint16_t*)o, o_bs, o_hs, o_ss, lse, static_cast<float*>(workspace));

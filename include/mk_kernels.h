@@ -138,6 +138,9 @@ int mk_gemm_splitk_typed(void* stream, int ab_type, int c_type, int64_t M, int64
  * C = alpha A B + beta C; no bias.  ab_type ∈ {MK_BF16 (c_type MK_BF16 /
  * MK_F16 / MK_F32), MK_F32 (c_type MK_F32)}, fp32 accumulation.  Operands
  * with overlapping rows (leading stride below the row length) are rejected.
+ * The library's handle, and with it the workspace its kernels synchronise
+ * through, is one per GPU: calls that overlap on a GPU (several streams, or
+ * graphs captured from several) must be ordered by the caller.
  * Replaces, for these products: src/jam/ops/linalg.mm:98. */
 int mk_gemm_blas(void* stream, int ab_type, int c_type,
                  int64_t batch, int64_t M, int64_t N, int64_t K,

@@ -31,11 +31,14 @@ their gradient live in one bf16 buffer whose rows are padded from 50257 to
 tied embedding take aligned operand rows on the hand-written kernels: the
 embedding gradient on mk_gemm, the hidden-state gradient (a contraction over
 the 50257 classes into a 8192 x 768 result) on mk_gemm_splitk_typed, 8
-slices.  The logits product itself (K = 768 into 8192 x 50257) stays on
-rocBLAS (mk_gemm_blas), which runs it 10-25% faster than the tiled kernel.
-Every other operation is a hand-written kernel.  All parameters live in five flat buffers (fp32 master, bf16 working copy,
-fp32 gradient, fp32 m, fp32 v), each parameter a 64-element-aligned slice, so
-the optimizer is a single launch and every gradient is written in place.  The
+slices.  No product goes to the library: rocBLAS runs the logits product on a
+stream-K kernel whose workgroups wait for each other through the handle's one
+workspace, which steps on several streams would share (two such kernels at
+once, or two halves of the chip, need never finish); the tiled kernel takes
+667 us for it against about 600.  All parameters live in five flat buffers
+(fp32 master, bf16 working copy, fp32 gradient, fp32 m, fp32 v), each
+parameter a 64-element-aligned slice, so the optimizer is a single launch and
+every gradient is written in place.  The
 step is prepared once as a list of bound calls (device pointers and shapes
 fixed), so running it costs a few microseconds of host time per launch, and
 the list can be captured into a HIP graph.
@@ -157,8 +160,6 @@ class GPT2TrainStep:
     # out, split along K in uneven slices (measured: 8 slices 664 us, 2 693,
     # unsplit 910; rocBLAS 682-687)
     DHF_SPLITS = 8
-    # products on the library GEMM (measured faster there; see the module doc)
-    BLAS_GEMMS = ("logits",)
 
     def __init__(self, cfg: GPT2Config, params: dict | None = None, seed: int = 0, lr: float = 3e-4,
                  b1: float = 0.9, b2: float = 0.999, adam_eps: float = 1e-8, device="cuda", stream=None):
@@ -273,19 +274,12 @@ class GPT2TrainStep:
 
         def gemm(ab, ct, M, N, Kd, a, a_ms, a_ks, b, b_ks, b_ns, cptr, c_ms, tag="gemm", bias=None):
             # hand-written GEMM (optionally + bias); the fp32 weight gradients
-            # (few output tiles, K = tokens) split along K; the vocabulary
-            # GEMMs (unaligned 50257-element rows) through rocBLAS
+            # (few output tiles, K = tokens) split along K
             sp = self.DW_SPLITS.get(tag, 1)
             if sp > 1 and ct == F32 and Kd % sp == 0:
                 calls.append(_Call(lib.mk_gemm_splitk, [st, _I(ab), _I64(M), _I64(N), _I64(Kd), a, _I64(a_ms),
                                                         _I64(a_ks), b, _I64(b_ks), _I64(b_ns), cptr, _I64(c_ms),
                                                         _I64(sp), ws], "mk_gemm_splitk " + tag))
-                return
-            if tag in self.BLAS_GEMMS:
-                calls.append(_Call(lib.mk_gemm_blas, [st, _I(ab), _I(ct), _I64(1), _I64(M), _I64(N), _I64(Kd),
-                                                      a, _I64(0), _I64(a_ms), _I64(a_ks), b, _I64(0), _I64(b_ks),
-                                                      _I64(b_ns), cptr, _I64(0), _I64(c_ms), _F(1.0), _F(0.0)],
-                                   "mk_gemm_blas " + tag))
                 return
             if tag == "dhf":
                 calls.append(_Call(lib.mk_gemm_splitk_typed, [st, _I(ab), _I(ct), _I64(M), _I64(N), _I64(Kd), a,

@@ -92,3 +92,16 @@ def test_lds_copies_have_no_sgpr_hazard(src, tmp_path):
     n_copies = sum(1 for l in asm.splitlines() if _COPY.match(l.strip()))
     assert n_copies > 0, "no LDS copies found: the pattern no longer matches the kernels"
     assert hazards(asm) == []
+
+
+@pytest.mark.skipif(not shutil.which(HIPCC) and not os.path.exists(HIPCC), reason="hipcc not available")
+def test_lds_copies_of_the_backward_as_built(tmp_path):
+    """The attention backward under its Makefile flags (MFMA results in VGPRs)."""
+    out = tmp_path / "attention_bwd.s"
+    cmd = [HIPCC, "--offload-arch=gfx950", "-O3", "-std=c++17", "-Xclang", "-target-feature", "-Xclang",
+           "-packed-fp32-ops", "-mllvm", "-amdgpu-mfma-vgpr-form", "-I" + os.path.join(ROOT, "include"), "-I" + KDIR,
+           "--cuda-device-only", "-S", os.path.join(KDIR, "attention_bwd.hip"), "-o", str(out)]
+    subprocess.run(cmd, check=True, capture_output=True, timeout=300)
+    asm = out.read_text()
+    assert any(_COPY.match(l.strip()) for l in asm.splitlines())
+    assert hazards(asm) == []

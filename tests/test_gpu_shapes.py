@@ -178,3 +178,39 @@ def test_sdpa_few_queries_infinities(K):
     k[0, 1, 699, 3] = float("nan")
     o = K.sdpa_fwd(q, k, v, 0.125, causal=False)
     assert bool((o[0, 0] == 2).all()) and bool(o[0, 1].isnan().all()) and bool((o[0, 2] == 2).all())
+
+
+def test_gpt2_steps_on_several_streams(cuda):
+    """Captured steps replayed at once on streams of their own give the bits
+    each gives alone, and none of their calls shares a library workspace."""
+    from mi355x_pjrt import gpt2
+
+    cfg = gpt2.GPT2Config(n_layer=1, d_model=256, n_head=4, seq=256, batch=4, vocab=5003)
+    steps, alone = [], []
+    for i in range(3):
+        step = gpt2.GPT2TrainStep(cfg, seed=i, stream=torch.cuda.Stream())
+        assert not any("blas" in c.name for c in step.calls)
+        g = torch.Generator().manual_seed(i)
+        step.set_batch(torch.randint(cfg.vocab, (cfg.tokens,), generator=g),
+                       torch.randint(cfg.vocab, (cfg.tokens,), generator=g))
+        torch.cuda.synchronize()
+        step.step()
+        step.stream.synchronize()
+        step.capture()
+        steps.append(step)
+        start = [t.clone() for t in (step.master, step.param, step.m, step.v)]
+        torch.cuda.synchronize()
+        for _ in range(3):
+            step.replay()
+        torch.cuda.synchronize()
+        alone.append(step.master.clone())
+        for t, s0 in zip((step.master, step.param, step.m, step.v), start):
+            t.copy_(s0)
+        step.t = 1
+    torch.cuda.synchronize()
+    for _ in range(3):
+        for step in steps:
+            step.replay()
+    torch.cuda.synchronize()
+    for step, want in zip(steps, alone):
+        assert torch.equal(step.master, want)

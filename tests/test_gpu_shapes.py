@@ -214,3 +214,24 @@ def test_gpt2_steps_on_several_streams(cuda):
     torch.cuda.synchronize()
     for step, want in zip(steps, alone):
         assert torch.equal(step.master, want)
+
+
+@pytest.mark.parametrize("M,N,Kd,splits", [(200, 136, 1000, 8), (128, 256, 4120, 8), (130, 132, 520, 4), (256, 768, 50256, 8),
+                                           (128, 128, 400, 8), (129, 128, 36, 4), (300, 256, 1004, 4)])
+def test_gemm_splitk_slices_off_the_16_byte_grid(K, M, N, Kd, splits):
+    """Slice counts that divide K into slices that are no multiple of 8, on
+    the uneven slices (400 in 8: slices of 56 are too short for the tiled
+    kernel; 36 and 1004: rows off the grid, the even form), each operand
+    k-contiguous in turn.  Bound: fp32 sums in another order, K ulps of the
+    sum of magnitudes at the most."""
+    assert Kd % splits == 0 and Kd // splits % 8 != 0
+    g = torch.Generator().manual_seed(Kd)
+    a, b = torch.randn(M, Kd, generator=g).bfloat16(), torch.randn(Kd, N, generator=g).bfloat16()
+    want, norm = a.double() @ b.double(), a.double().abs() @ b.double().abs()
+    for ad, bd in ((a.cuda(), b.cuda()), (a.cuda(), b.t().contiguous().cuda().t()),
+                   (a.t().contiguous().cuda().t(), b.t().contiguous().cuda().t())):
+        got = K.gemm_splitk(ad, bd, splits)
+        assert bool(((got.cpu().double() - want).abs() <= Kd * 2.0 ** -24 * norm).all())
+        assert torch.equal(got, K.gemm_splitk(ad, bd, splits))
+        low = K.gemm_splitk(ad, bd, splits, out_dtype=torch.bfloat16)
+        assert torch.equal(low, got.bfloat16())

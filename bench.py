@@ -405,8 +405,7 @@ def run_gemm(torch, np, K, args):
             row["mk_gemm_splitk_tflops"] = round(fl / (ms * 1e-3) / 1e12, 1)
             row["splits"] = sp
             msg += f"; split {sp}: mk_gemm_splitk_typed {row['mk_gemm_splitk_tflops']}"
-        row["c5_step_path"] = ("rocBLAS" if tag in GPT2TrainStep.BLAS_GEMMS else
-                               "mk_gemm_splitk_typed" if tag == "dhf" else
+        row["c5_step_path"] = ("mk_gemm_splitk_typed" if tag == "dhf" else
                                "mk_gemm_splitk" if tag in GPT2TrainStep.DW_SPLITS else "mk_gemm")
         sp = GPT2TrainStep.DW_SPLITS.get(tag, 1)
         if sp > 1:  # the C5 step runs these fp32 weight gradients split along K

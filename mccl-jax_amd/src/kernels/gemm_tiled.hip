@@ -763,20 +763,24 @@ int gemm_tiled(hipStream_t s, int c_type, int64_t batch, int64_t M, int64_t N, i
                   bias, epilogue, k_rem, Y, y_ms, colpart))
     return -1;
   // Kernel shape: the one with the least estimated time.  A round of
-  // workgroups costs nk + e k tiles, each of its area over the shape's rate:
-  // the rate per CU in the k loop and e, the first loads and the epilogue in
-  // k tiles (twice that for fp32 C), are fitted to 8192 x 8192 x 4096 and
-  // 8192 x 50257 x 768 (256 x 256: 437 and 703 us; 128 x 192: 485 and 668;
-  // 128 x 128: 521 and 740).  A CU holds one 256 x 256 workgroup or two of
-  // the smaller ones.  A last partial round that leaves every workgroup alone
-  // on its CU runs each at about 0.8 of the pair's rate (8192 x 768 products,
-  // K = 768 .. 3072), and one on fewer than half of the CUs takes about 0.8
-  // of a full round of 256 x 256 tiles.
+  // workgroups costs nk + e k tiles, each of its area over the shape's rate
+  // per CU; e is the first loads and the epilogue in k tiles, for 16-bit C
+  // and for fp32 C (whose stores cost about the same per element in every
+  // shape).  A CU holds one 256 x 256 workgroup or two of the smaller ones; a
+  // last partial round with every workgroup alone on its CU runs each at
+  // 0.73 of the pair's rate, and one on fewer than half of the CUs takes 0.63
+  // of a full round of 256 x 256 tiles.  The constants are fitted to the three
+  // shapes' times on 58 products, 256 .. 50257 rows and columns, 64 .. 8192
+  // deep, both C types, unsplit and split: the choice is within 1% of the
+  // fastest on each (8192 x 50257 x 768, bf16 C: 694 / 657 / 717 us in the
+  // order below; 2300 x 640 x 40000 in 8 slices: 168 / 197 / 200; 40000 x 640
+  // x 2300, fp32 C: 128 / 144 / 146; 1024 x 8192 x 2048: 47 / 41 / 35).
   struct Option {
     int tm, tn, per_cu;
-    double rate, e;
+    double rate, e16, e32;
   };
-  static const Option options[3] = {{256, 256, 1, 1240.0, 7.5}, {128, 192, 2, 1120.0, 5.3}, {128, 128, 2, 971.0, 3.3}};
+  static const Option options[3] = {
+      {256, 256, 1, 1330.0, 4.5, 12.2}, {128, 192, 2, 1250.0, 1.1, 10.3}, {128, 128, 2, 1030.0, 0.7, 11.4}};
   const int64_t cus = cu_count();
   const double nk = double((K + 63) / 64);
   int best = -1;
@@ -786,11 +790,11 @@ int gemm_tiled(hipStream_t s, int c_type, int64_t batch, int64_t M, int64_t N, i
     if (M < op.tm || N < op.tn) continue;
     const int64_t tiles = ((M + op.tm - 1) / op.tm) * ((N + op.tn - 1) / op.tn) * batch;
     const int64_t slots = cus * op.per_cu, rem = tiles % slots;
-    const double tile = double(op.tm) * op.tn / op.rate * (nk + (c_type == MK_F32 ? 2 * op.e : op.e));
+    const double tile = double(op.tm) * op.tn / op.rate * (nk + (c_type == MK_F32 ? op.e32 : op.e16));
     double t = double(tiles / slots) * op.per_cu * tile;
     if (rem > 0) {
-      if (op.per_cu > 1) t += rem <= cus ? tile / 0.8 : op.per_cu * tile;
-      else t += 2 * rem < cus ? 0.8 * tile : tile;
+      if (op.per_cu > 1) t += rem <= cus ? tile / 0.73 : op.per_cu * tile;
+      else t += 2 * rem < cus ? 0.63 * tile : tile;
     }
     if (best < 0 || t < best_t) best = o, best_t = t;
   }

@@ -139,8 +139,11 @@ int mk_gemm_splitk_typed(void* stream, int ab_type, int c_type, int64_t M, int64
  * MK_F16 / MK_F32), MK_F32 (c_type MK_F32)}, fp32 accumulation.  Operands
  * with overlapping rows (leading stride below the row length) are rejected.
  * The library's handle, and with it the workspace its kernels synchronise
- * through, is one per GPU: calls that overlap on a GPU (several streams, or
- * graphs captured from several) must be ordered by the caller.
+ * through, is one per GPU, so calls take turns: the kernels of a call wait
+ * for those of the call before it, whatever its stream or thread.  On a
+ * stream that is being captured the product runs on mk_gemm's kernels
+ * instead (a graph is replayed outside any such order), so it may round
+ * differently there and take longer where rows are not 16-byte aligned.
  * Replaces, for these products: src/jam/ops/linalg.mm:98. */
 int mk_gemm_blas(void* stream, int ab_type, int c_type,
                  int64_t batch, int64_t M, int64_t N, int64_t K,
@@ -552,7 +555,7 @@ int mk_adam_update_dev(void* stream, int64_t n, int param_type, void* param, flo
  * rounded up to 64-row tiles); q/k/v/o/dout rows 16-byte aligned, dq/dk/dv
  * strides multiples of 4.  Other D (a multiple of 8, ≤ 256): S, dP (fp32)
  * and P, dS (bf16) materialised for all heads in the workspace, products on
- * the rocBLAS GEMM of mk_gemm_blas; o and dout rows 16-byte aligned.
+ * the rocBLAS GEMM of mk_gemm_blas, in one turn of its order; o and dout rows 16-byte aligned.
  * Strides as mk_sdpa_fwd (elements, D contiguous). */
 size_t mk_sdpa_bwd_workspace_bytes(int64_t B, int64_t H, int64_t Sq, int64_t Sk, int64_t D);
 int mk_sdpa_bwd(void* stream, int64_t B, int64_t H, int64_t Sq, int64_t Sk, int64_t D,

@@ -393,7 +393,8 @@ def _mat_strides(t):
 
 def gemm_blas(a, b, out=None, out_dtype=None, alpha=1.0, beta=0.0, stream=None):
     """out = alpha a @ b + beta out through rocBLAS (mk_gemm_blas); a [.., M, K],
-    b [.., K, N] views with one unit stride each (either orientation)."""
+    b [.., K, N] views with one unit stride each (either orientation).  Calls
+    take turns on a GPU across streams; captured ones run on gemm's kernels."""
     _require_cuda(a, b)
     M, Kd = a.shape[-2:]
     N = b.shape[-1]

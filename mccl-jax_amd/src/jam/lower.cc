@@ -3901,9 +3901,10 @@ class Lowerer {
     st.kind = StepKind::kGemm;
     // bf16 operands whose rows are not 16-byte aligned (a vocabulary of
     // 50257) rule out the tiled kernel's 16-byte HBM->LDS copies; large such
-    // products go to the library GEMM, as the hand-scheduled step's
-    // vocabulary products do (the general kernel runs them at a tenth of
-    // its rate), the rest to mk_gemm's general kernel
+    // products go to the library GEMM (the general kernel runs them at a
+    // tenth of its rate; mk_gemm_blas keeps the library's kernels from
+    // overlapping with those of other streams), the rest to mk_gemm's
+    // general kernel
     const auto rows8 = [](int64_t bs, int64_t ms, int64_t ks) { return bs % 8 == 0 && (ms == 1 ? ks : ms) % 8 == 0; };
     if (at == DType::kBF16 && !epi && (ct == DType::kF32 || ct == DType::kBF16) &&
         !(rows8(a_bs, a_ms, a_ks) && rows8(b_bs, b_ns, b_ks)) && double(B) * M * N * K >= double(int64_t(1) << 30))

@@ -15,28 +15,17 @@
 namespace mk {
 namespace {
 
+// The library's state on one GPU, kept for the process: the handle, whose
+// workspace the library's stream-K kernels synchronise their workgroups
+// through (two of them at once overwrite each other's flags and can wait
+// forever), and an event recorded behind the last turn's kernels.
+struct Library {
+  rocblas_handle handle = nullptr;
+  hipEvent_t done = nullptr;
+  bool used = false;  // `done` has been recorded
+};
 std::mutex g_blas_mu;
-std::vector<rocblas_handle> g_handles;  // one per device, kept for the process
-
-rocblas_handle handle_for_current_device(int* err) {
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess) {
-    *err = fail(MK_ERR_LAUNCH, "mk_gemm_blas: hipGetDevice failed");
-    return nullptr;
-  }
-  std::lock_guard<std::mutex> lk(g_blas_mu);
-  if (int(g_handles.size()) <= dev) g_handles.resize(dev + 1, nullptr);
-  if (!g_handles[dev]) {
-    rocblas_handle h = nullptr;
-    if (rocblas_create_handle(&h) != rocblas_status_success) {
-      *err = fail(MK_ERR_LAUNCH, "mk_gemm_blas: rocblas_create_handle failed");
-      return nullptr;
-    }
-    rocblas_set_pointer_mode(h, rocblas_pointer_mode_host);
-    g_handles[dev] = h;
-  }
-  return g_handles[dev];
-}
+std::vector<Library> g_libraries;  // by device
 
 bool blas_type(int t, rocblas_datatype* out) {
   if (t == MK_BF16) *out = rocblas_datatype_bf16_r;
@@ -48,8 +37,57 @@ bool blas_type(int t, rocblas_datatype* out) {
 
 }  // namespace
 
+BlasTurn::BlasTurn(hipStream_t stream) : stream_(stream) {
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(stream, &cap) != hipSuccess) (void)hipGetLastError();
+  else captured_ = cap != hipStreamCaptureStatusNone;
+  if (captured_) return;
+  lock_ = std::unique_lock<std::mutex>(g_blas_mu);
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess) {
+    rc_ = fail(MK_ERR_LAUNCH, "mk_gemm_blas: hipGetDevice failed");
+    return;
+  }
+  dev_ = dev;
+  if (int(g_libraries.size()) <= dev) g_libraries.resize(dev + 1);
+  Library& l = g_libraries[dev];
+  if (!l.done && hipEventCreateWithFlags(&l.done, hipEventDisableTiming) != hipSuccess) {
+    l.done = nullptr;
+    rc_ = fail(MK_ERR_LAUNCH, "mk_gemm_blas: hipEventCreateWithFlags failed");
+    return;
+  }
+  if (!l.handle) {
+    rocblas_handle h = nullptr;
+    if (rocblas_create_handle(&h) != rocblas_status_success) {
+      rc_ = fail(MK_ERR_LAUNCH, "mk_gemm_blas: rocblas_create_handle failed");
+      return;
+    }
+    rocblas_set_pointer_mode(h, rocblas_pointer_mode_host);
+    l.handle = h;
+  }
+  if (l.used && hipStreamWaitEvent(stream, l.done, 0) != hipSuccess) {
+    rc_ = fail(MK_ERR_LAUNCH, "mk_gemm_blas: hipStreamWaitEvent failed");
+    return;
+  }
+  if (rocblas_set_stream(l.handle, stream) != rocblas_status_success) {
+    rc_ = fail(MK_ERR_LAUNCH, "mk_gemm_blas: rocblas_set_stream failed");
+    return;
+  }
+  handle_ = l.handle;
+}
+
+BlasTurn::~BlasTurn() {
+  if (!handle_) return;
+  Library& l = g_libraries[dev_];
+  l.used = true;
+  if (hipEventRecord(l.done, stream_) != hipSuccess) {
+    (void)hipGetLastError();
+    (void)hipStreamSynchronize(stream_);  // nothing left for the next turn to wait for
+  }
+}
+
 // shared with the attention backward (train.hip)
-int gemm_blas(hipStream_t stream, int ab_type, int c_type, int64_t batch, int64_t M, int64_t N, int64_t K,
+int gemm_blas(const BlasTurn& turn, int ab_type, int c_type, int64_t batch, int64_t M, int64_t N, int64_t K,
               const void* A, int64_t a_bs, int64_t a_ms, int64_t a_ks, const void* B, int64_t b_bs, int64_t b_ks,
               int64_t b_ns, void* C, int64_t c_bs, int64_t c_ms, float alpha, float beta) {
   if (batch < 0 || M < 0 || N < 0 || K < 0) return fail(MK_ERR_INVALID, "mk_gemm_blas: negative shape");
@@ -86,14 +124,11 @@ int gemm_blas(hipStream_t stream, int ab_type, int c_type, int64_t batch, int64_
     return fail(MK_ERR_UNSUPPORTED, "mk_gemm_blas: overlapping rows (leading stride below the row length)");
   if (lda > INT32_MAX || ldb > INT32_MAX || ldc > INT32_MAX)
     return fail(MK_ERR_UNSUPPORTED, "mk_gemm_blas: leading dimension beyond int32");
-  int err = MK_OK;
-  rocblas_handle h = handle_for_current_device(&err);
-  if (!h) return err;
-  // a device's handle is shared: binding the stream and queueing the GEMM
-  // happen under one lock, so concurrent callers cannot swap streams between
-  std::lock_guard<std::mutex> lk(g_blas_mu);
-  if (rocblas_set_stream(h, stream) != rocblas_status_success)
-    return fail(MK_ERR_LAUNCH, "mk_gemm_blas: rocblas_set_stream failed");
+  if (turn.captured())
+    return gemm_own(turn.stream(), ab_type, c_type, batch, M, N, K, A, a_bs, a_ms, a_ks, B, b_bs, b_ks, b_ns, C, c_bs,
+                    c_ms, alpha, beta);
+  if (!turn.handle()) return turn.rc();
+  const rocblas_handle h = static_cast<rocblas_handle>(turn.handle());
   const rocblas_status st = rocblas_gemm_strided_batched_ex(
       h, op_a, op_b, rocblas_int(N), rocblas_int(M), rocblas_int(K), &alpha, B, ab, rocblas_int(lda), b_bs, A, ab,
       rocblas_int(ldb), a_bs, &beta, C, ct, rocblas_int(ldc), c_bs, C, ct, rocblas_int(ldc), c_bs,
@@ -188,7 +223,7 @@ extern "C" int mk_gemm_blas_splitk(void* stream, int ab_type, int64_t M, int64_t
   if (splits < 1 || K < 0 || M < 0 || N < 0) return mk::fail(MK_ERR_INVALID, "mk_gemm_blas_splitk: bad shape or splits");
   hipStream_t s = mk::as_stream(stream);
   if (splits == 1 || M == 0 || N == 0)
-    return mk::gemm_blas(s, ab_type, MK_F32, 1, M, N, K, A, 0, a_ms, a_ks, B, 0, b_ks, b_ns, C, 0, c_ms, 1.f, 0.f);
+    return mk::gemm_blas(mk::BlasTurn(s), ab_type, MK_F32, 1, M, N, K, A, 0, a_ms, a_ks, B, 0, b_ks, b_ns, C, 0, c_ms, 1.f, 0.f);
   if (K % splits != 0) return mk::fail(MK_ERR_UNSUPPORTED, "mk_gemm_blas_splitk: K must be a multiple of splits");
   if (!workspace || !C) return mk::fail(MK_ERR_INVALID, "mk_gemm_blas_splitk: null workspace or output");
   if ((N % 4) != 0 || (c_ms % 4) != 0 || ((reinterpret_cast<uintptr_t>(C) | reinterpret_cast<uintptr_t>(workspace)) & 15))
@@ -196,7 +231,7 @@ extern "C" int mk_gemm_blas_splitk(void* stream, int ab_type, int64_t M, int64_t
   const int64_t ks = K / splits;
   // slice s reads A[:, s ks : (s+1) ks] and B[s ks : (s+1) ks, :] (element strides along k) and writes W[s]
   float* W = static_cast<float*>(workspace);
-  if (int rc = mk::gemm_blas(s, ab_type, MK_F32, splits, M, N, ks, A, ks * a_ks, a_ms, a_ks, B, ks * b_ks, b_ks, b_ns,
+  if (int rc = mk::gemm_blas(mk::BlasTurn(s), ab_type, MK_F32, splits, M, N, ks, A, ks * a_ks, a_ms, a_ks, B, ks * b_ks, b_ks, b_ns,
                              W, M * N, N, 1.f, 0.f))
     return rc;
   return mk::splitk_sum(s, W, splits, M, N, C, c_ms, "mk_gemm_blas_splitk");
@@ -207,6 +242,6 @@ extern "C" int mk_gemm_blas(void* stream, int ab_type, int c_type, int64_t batch
                             const void* B, int64_t b_bs, int64_t b_ks, int64_t b_ns,
                             void* C, int64_t c_bs, int64_t c_ms, float alpha, float beta) {
   mk::clear_error();
-  return mk::gemm_blas(mk::as_stream(stream), ab_type, c_type, batch, M, N, K, A, a_bs, a_ms, a_ks, B, b_bs, b_ks,
+  return mk::gemm_blas(mk::BlasTurn(mk::as_stream(stream)), ab_type, c_type, batch, M, N, K, A, a_bs, a_ms, a_ks, B, b_bs, b_ks,
                        b_ns, C, c_bs, c_ms, alpha, beta);
 }

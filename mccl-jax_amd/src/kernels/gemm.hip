@@ -47,6 +47,7 @@ struct GemmArgs {
   int epilogue;
   int c_type;
   int vec_a, vec_b;  // 16-byte vector loads allowed along the contiguous dim
+  float alpha, beta;  // the scaled kernel's
 };
 
 // Stage one operand tile (ROWS x BK, element (row, k) = src[row*rs + k*ks])
@@ -161,8 +162,9 @@ struct TileLoader {
 
 // NW waves in an (NW / 2) x 2 arrangement: 4 waves of 64 x 64, or 8 waves of
 // 32 x 64 (the fp32 products, where one 4-wave workgroup per CU left each
-// SIMD a single wave to hide the loads behind).
-template <typename T, bool A_KC, bool B_KC, int NW = 4>
+// SIMD a single wave to hide the loads behind).  SCALED: C = alpha A B + beta C
+// (epilogue 0).
+template <typename T, bool A_KC, bool B_KC, int NW, bool SCALED>
 __global__ __launch_bounds__(64 * NW, 8 / NW) void gemm_kernel(const GemmArgs p) {
   using C = Cfg<T>;
   constexpr int NT = 64 * NW;
@@ -263,6 +265,14 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void gemm_kernel(const GemmArgs p)
         if (p.epilogue != 0) v += bias;
         if ((p.epilogue & 3) == 2) v = fmaxf(v, 0.f);
         const int64_t off = bz * p.c_bs + m * p.c_ms + n;
+        if constexpr (SCALED) {
+          v *= p.alpha;
+          if (p.beta != 0.f) {
+            const uint16_t h = cbytes == 4 ? 0 : reinterpret_cast<const uint16_t*>(Cb)[off];
+            v += p.beta * (cbytes == 4 ? reinterpret_cast<const float*>(Cb)[off]
+                                       : p.c_type == MK_BF16 ? bf16_to_f32(h) : f16_to_f32(h));
+          }
+        }
         if (cbytes == 4) reinterpret_cast<float*>(Cb)[off] = v;
         else store_from_f32(Cb, off, p.c_type, v);
       }
@@ -286,19 +296,72 @@ __global__ __launch_bounds__(256) void colpart_sum_kernel(const float* __restric
 
 // fp32 operands: 8 waves per workgroup (two per SIMD when one workgroup
 // holds a CU); bf16: 4
-template <typename T>
+template <typename T, bool SCALED = false>
 int launch_gemm(hipStream_t s, const GemmArgs& a, int64_t batch, bool a_kc, bool b_kc) {
   constexpr int NW = sizeof(T) == 4 ? 8 : 4;
   const int64_t tiles = ((a.M + kBM - 1) / kBM) * ((a.N + kBN - 1) / kBN);
   const dim3 g{unsigned(tiles), unsigned(batch)}, b{unsigned(64 * NW)};
-  if (a_kc && b_kc) hipLaunchKernelGGL((gemm_kernel<T, true, true, NW>), g, b, 0, s, a);
-  else if (a_kc && !b_kc) hipLaunchKernelGGL((gemm_kernel<T, true, false, NW>), g, b, 0, s, a);
-  else if (!a_kc && b_kc) hipLaunchKernelGGL((gemm_kernel<T, false, true, NW>), g, b, 0, s, a);
-  else hipLaunchKernelGGL((gemm_kernel<T, false, false, NW>), g, b, 0, s, a);
+  if (a_kc && b_kc) hipLaunchKernelGGL((gemm_kernel<T, true, true, NW, SCALED>), g, b, 0, s, a);
+  else if (a_kc && !b_kc) hipLaunchKernelGGL((gemm_kernel<T, true, false, NW, SCALED>), g, b, 0, s, a);
+  else if (!a_kc && b_kc) hipLaunchKernelGGL((gemm_kernel<T, false, true, NW, SCALED>), g, b, 0, s, a);
+  else hipLaunchKernelGGL((gemm_kernel<T, false, false, NW, SCALED>), g, b, 0, s, a);
   return check_launch("mk_gemm");
 }
 
+// the general kernel's arguments; unit strides of a length-1 k axis filled in
+GemmArgs gemm_args(int esz, int c_type, int64_t M, int64_t N, int64_t K, const void* A, int64_t a_bs, int64_t a_ms,
+                   int64_t a_ks, const void* B, int64_t b_bs, int64_t b_ks, int64_t b_ns, void* C, int64_t c_bs,
+                   int64_t c_ms, const void* bias, int epilogue) {
+  GemmArgs a;
+  const bool a_kc = a_ks == 1 || K == 1, b_kc = b_ks == 1 || K == 1;
+  a.A = A; a.B = B; a.C = C; a.bias = bias;
+  a.M = M; a.N = N; a.K = K;
+  a.a_bs = a_bs; a.a_ms = a_kc ? a_ms : 1; a.a_ks = a_kc ? 1 : a_ks;
+  a.b_bs = b_bs; a.b_ks = b_kc ? 1 : b_ks; a.b_ns = b_kc ? b_ns : 1;
+  a.c_bs = c_bs; a.c_ms = c_ms;
+  a.tiles_n = int((N + kBN - 1) / kBN);
+  a.epilogue = epilogue;
+  a.c_type = c_type;
+  a.alpha = 1.f, a.beta = 0.f;
+  auto al16 = [](const void* ptr) { return (reinterpret_cast<uintptr_t>(ptr) & 15u) == 0; };
+  const int vec = 16 / esz;
+  // vector loads need every chunk start 16-byte aligned: base, batch stride
+  // and the non-unit stride must be multiples of the vector width
+  a.vec_a = al16(A) && (a_bs % vec == 0) && ((a_kc ? a.a_ms : a.a_ks) % vec == 0);
+  a.vec_b = al16(B) && (b_bs % vec == 0) && ((b_kc ? a.b_ns : a.b_ks) % vec == 0);
+  return a;
+}
+
 }  // namespace
+
+int gemm_own(hipStream_t s, int ab_type, int c_type, int64_t batch, int64_t M, int64_t N, int64_t K, const void* A,
+             int64_t a_bs, int64_t a_ms, int64_t a_ks, const void* B, int64_t b_bs, int64_t b_ks, int64_t b_ns,
+             void* C, int64_t c_bs, int64_t c_ms, float alpha, float beta) {
+  const int esz = ab_type == MK_BF16 ? 2 : 4;
+  constexpr int64_t kMost = 65535;  // batches of one launch
+  for (int64_t b0 = 0; b0 < batch; b0 += kMost) {
+    const int64_t nb = batch - b0 < kMost ? batch - b0 : kMost;
+    const char* Ab = static_cast<const char*>(A) + b0 * a_bs * esz;
+    const char* Bb = static_cast<const char*>(B) + b0 * b_bs * esz;
+    char* Cb = static_cast<char*>(C) + b0 * c_bs * dtype_bytes(c_type);
+    int rc;
+    if (alpha == 1.f && beta == 0.f) {
+      rc = mk_gemm(s, ab_type, c_type, nb, M, N, K, Ab, a_bs, a_ms, a_ks, Bb, b_bs, b_ks, b_ns, Cb, c_bs, c_ms,
+                   nullptr, 0);
+    } else {
+      GemmArgs a = gemm_args(esz, c_type, M, N, K, Ab, a_bs, a_ms, a_ks, Bb, b_bs, b_ks, b_ns, Cb, c_bs, c_ms,
+                             nullptr, 0);
+      a.alpha = alpha;
+      a.beta = beta;
+      const bool a_kc = a_ks == 1 || K == 1, b_kc = b_ks == 1 || K == 1;
+      rc = ab_type == MK_BF16 ? launch_gemm<uint16_t, true>(s, a, nb, a_kc, b_kc)
+                              : launch_gemm<float, true>(s, a, nb, a_kc, b_kc);
+    }
+    if (rc) return rc;
+  }
+  return MK_OK;
+}
+
 }  // namespace mk
 
 using namespace mk;
@@ -375,22 +438,9 @@ extern "C" int mk_gemm(void* stream, int ab_type, int c_type, int64_t batch, int
   if (!b_kc && !b_nc) return fail(MK_ERR_UNSUPPORTED, "mk_gemm: B needs a unit stride along k or n");
   const int64_t tiles = ((M + kBM - 1) / kBM) * ((N + kBN - 1) / kBN);
   if (tiles >= (int64_t(1) << 31)) return fail(MK_ERR_UNSUPPORTED, "mk_gemm: too many tiles");
-  GemmArgs a;
-  a.A = A; a.B = B; a.C = C; a.bias = bias;
-  a.M = M; a.N = N; a.K = K;
-  a.a_bs = a_bs; a.a_ms = a_kc ? a_ms : 1; a.a_ks = a_kc ? 1 : a_ks;
-  a.b_bs = b_bs; a.b_ks = b_kc ? 1 : b_ks; a.b_ns = b_kc ? b_ns : 1;
-  a.c_bs = c_bs; a.c_ms = c_ms;
-  a.tiles_n = int((N + kBN - 1) / kBN);
-  a.epilogue = epilogue;
-  a.c_type = c_type;
   const int esz = ab_type == MK_BF16 ? 2 : 4;
-  auto al16 = [](const void* ptr) { return (reinterpret_cast<uintptr_t>(ptr) & 15u) == 0; };
-  const int vec = 16 / esz;
-  // vector loads need every chunk start 16-byte aligned: base, batch stride
-  // and the non-unit stride must be multiples of the vector width
-  a.vec_a = al16(A) && (a_bs % vec == 0) && ((a_kc ? a.a_ms : a.a_ks) % vec == 0);
-  a.vec_b = al16(B) && (b_bs % vec == 0) && ((b_kc ? a.b_ns : a.b_ks) % vec == 0);
+  const GemmArgs a = gemm_args(esz, c_type, M, N, K, A, a_bs, a_ms, a_ks, B, b_bs, b_ks, b_ns, C, c_bs, c_ms, bias,
+                               epilogue);
   hipStream_t s = as_stream(stream);
   // few rows: one pass over B whatever its size, strides and alignment
   if (const int r = gemm_skinny(s, ab_type, c_type, batch, M, N, K, A, a_bs, a.a_ms, a.a_ks, B, b_bs, a.b_ks, a.b_ns,

@@ -3,6 +3,7 @@
 
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+#include <mutex>
 #include <string>
 
 #include "mk_kernels.h"
@@ -20,10 +21,42 @@ int check_launch(const char* what);
 
 inline hipStream_t as_stream(void* s) { return reinterpret_cast<hipStream_t>(s); }
 
-// rocBLAS GEMM behind mk_gemm_blas (blas.hip), same operand convention.
-int gemm_blas(hipStream_t stream, int ab_type, int c_type, int64_t batch, int64_t M, int64_t N, int64_t K,
+// One turn of the library GEMM on a GPU (blas.hip): holds the GPU's handle
+// from construction to destruction.  A turn's stream first waits for the
+// kernels of the turn before it, whatever stream that ran on, so two of the
+// library's kernels never share its workspace at a time.  A captured stream
+// gets no handle: its graph would be replayed outside any such order, so its
+// products run on the kernels of this library (gemm_own).
+class BlasTurn {
+ public:
+  explicit BlasTurn(hipStream_t stream);
+  ~BlasTurn();
+  BlasTurn(const BlasTurn&) = delete;
+  BlasTurn& operator=(const BlasTurn&) = delete;
+  bool captured() const { return captured_; }
+  void* handle() const { return handle_; }  // rocblas_handle; null: rc()
+  int rc() const { return rc_; }
+  hipStream_t stream() const { return stream_; }
+
+ private:
+  hipStream_t stream_;
+  std::unique_lock<std::mutex> lock_;
+  void* handle_ = nullptr;
+  int dev_ = 0, rc_ = 0;
+  bool captured_ = false;
+};
+
+// rocBLAS GEMM behind mk_gemm_blas (blas.hip), same operand convention, as
+// part of a turn.
+int gemm_blas(const BlasTurn& turn, int ab_type, int c_type, int64_t batch, int64_t M, int64_t N, int64_t K,
               const void* A, int64_t a_bs, int64_t a_ms, int64_t a_ks, const void* B, int64_t b_bs, int64_t b_ks,
               int64_t b_ns, void* C, int64_t c_bs, int64_t c_ms, float alpha, float beta);
+
+// C[b] = alpha A[b] B[b] + beta C[b] without the library (gemm.hip): operands
+// as mk_gemm's, any batch, already checked.
+int gemm_own(hipStream_t s, int ab_type, int c_type, int64_t batch, int64_t M, int64_t N, int64_t K, const void* A,
+             int64_t a_bs, int64_t a_ms, int64_t a_ks, const void* B, int64_t b_bs, int64_t b_ks, int64_t b_ns,
+             void* C, int64_t c_bs, int64_t c_ms, float alpha, float beta);
 
 // C = sum of the splits dense M x N fp32 slices of W, added in slice order
 // (blas.hip), then + bias (c_type, per column; epilogue 1) and max(., 0)

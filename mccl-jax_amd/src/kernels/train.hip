@@ -1625,13 +1625,14 @@ extern "C" int mk_sdpa_bwd(void* stream, int64_t B, int64_t H, int64_t Sq, int64
                      nrows, Dsum);
   if (int rc = check_launch("mk_sdpa_bwd")) return rc;
   const int64_t SS = Sq * Sk;
+  const BlasTurn turn(s);  // all of this call's products
   // per batch index: H heads as one batched GEMM (head stride), S / dP rows of Sk
   for (int64_t b = 0; b < B; ++b) {
     const uint16_t* qb = static_cast<const uint16_t*>(q) + b * q_bs;
     const uint16_t* kb = static_cast<const uint16_t*>(k) + b * k_bs;
     float* Fb = F + b * H * SS;
     // S = Q Kᵀ  [Sq x Sk], fp32
-    if (int rc = gemm_blas(s, MK_BF16, MK_F32, H, Sq, Sk, D, qb, q_hs, q_ss, 1, kb, k_hs, 1, k_ss, Fb, SS, Sk, 1.f, 0.f))
+    if (int rc = gemm_blas(turn, MK_BF16, MK_F32, H, Sq, Sk, D, qb, q_hs, q_ss, 1, kb, k_hs, 1, k_ss, Fb, SS, Sk, 1.f, 0.f))
       return rc;
   }
   hipLaunchKernelGGL(attn_probs_kernel, dim3(grid_for(n)), dim3(kBlock), 0, s, F, lse, Sq, Sk, scale, causal, P, n);
@@ -1642,11 +1643,11 @@ extern "C" int mk_sdpa_bwd(void* stream, int64_t B, int64_t H, int64_t Sq, int64
     const uint16_t* Pb = P + b * H * SS;
     float* Fb = F + b * H * SS;
     // dV = Pᵀ dO  [Sk x D]
-    if (int rc = gemm_blas(s, MK_BF16, MK_BF16, H, Sk, D, Sq, Pb, SS, 1, Sk, db, do_hs, do_ss, 1,
+    if (int rc = gemm_blas(turn, MK_BF16, MK_BF16, H, Sk, D, Sq, Pb, SS, 1, Sk, db, do_hs, do_ss, 1,
                            static_cast<uint16_t*>(dv) + b * dv_bs, dv_hs, dv_ss, 1.f, 0.f))
       return rc;
     // dP = dO Vᵀ  [Sq x Sk], fp32 (over the scores)
-    if (int rc = gemm_blas(s, MK_BF16, MK_F32, H, Sq, Sk, D, db, do_hs, do_ss, 1, vb, v_hs, 1, v_ss, Fb, SS, Sk, 1.f, 0.f))
+    if (int rc = gemm_blas(turn, MK_BF16, MK_F32, H, Sq, Sk, D, db, do_hs, do_ss, 1, vb, v_hs, 1, v_ss, Fb, SS, Sk, 1.f, 0.f))
       return rc;
   }
   hipLaunchKernelGGL(attn_dscores_kernel, dim3(grid_for(n)), dim3(kBlock), 0, s, F, Dsum, Sk, scale, P, n);
@@ -1656,11 +1657,11 @@ extern "C" int mk_sdpa_bwd(void* stream, int64_t B, int64_t H, int64_t Sq, int64
     const uint16_t* kb = static_cast<const uint16_t*>(k) + b * k_bs;
     const uint16_t* Pb = P + b * H * SS;
     // dQ = dS K  [Sq x D]
-    if (int rc = gemm_blas(s, MK_BF16, MK_BF16, H, Sq, D, Sk, Pb, SS, Sk, 1, kb, k_hs, k_ss, 1,
+    if (int rc = gemm_blas(turn, MK_BF16, MK_BF16, H, Sq, D, Sk, Pb, SS, Sk, 1, kb, k_hs, k_ss, 1,
                            static_cast<uint16_t*>(dq) + b * dq_bs, dq_hs, dq_ss, 1.f, 0.f))
       return rc;
     // dK = dSᵀ Q  [Sk x D]
-    if (int rc = gemm_blas(s, MK_BF16, MK_BF16, H, Sk, D, Sq, Pb, SS, 1, Sk, qb, q_hs, q_ss, 1,
+    if (int rc = gemm_blas(turn, MK_BF16, MK_BF16, H, Sk, D, Sq, Pb, SS, 1, Sk, qb, q_hs, q_ss, 1,
                            static_cast<uint16_t*>(dk) + b * dk_bs, dk_hs, dk_ss, 1.f, 0.f))
       return rc;
   }

@@ -114,6 +114,40 @@ def test_gemm_blas_batched_alpha_beta_and_f32(K):
     assert float((_f64(got) - ref).abs().max()) < 1e-4
 
 
+@pytest.mark.parametrize("dtype,out_dtype", [(torch.bfloat16, torch.bfloat16), (torch.bfloat16, torch.float16),
+                                             (torch.bfloat16, torch.float32), (torch.float32, torch.float32)])
+@pytest.mark.parametrize("alpha,beta", [(1.0, 0.0), (0.5, 0.0), (-1.5, 2.0)])
+def test_gemm_blas_captured(K, dtype, out_dtype, alpha, beta):
+    """A captured library product runs on this library's own kernels: aligned,
+    ragged and few-row shapes, batches, both orientations, against float64 on
+    every replay.  Bounds: fp32 sums, then one rounding to the stored type of
+    a result that is also read (beta)."""
+    eps = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11, torch.float32: 2.0 ** -23}[out_dtype]
+    g = torch.Generator().manual_seed(5)
+    for batch, M, N, Kd, ta, tb in [(1, 256, 384, 128, False, False), (1, 77, 1001, 133, True, True),
+                                    (3, 9, 130, 65, False, True), (2, 130, 66, 40, True, False)]:
+        print(f"case: {batch}x{M}x{N}x{Kd} {dtype} -> {out_dtype} alpha={alpha} beta={beta}", flush=True)
+        a = (torch.randn(batch, Kd, M, generator=g).to(dtype).cuda().transpose(1, 2) if ta else
+             torch.randn(batch, M, Kd, generator=g).to(dtype).cuda())
+        b = (torch.randn(batch, N, Kd, generator=g).to(dtype).cuda().transpose(1, 2) if tb else
+             torch.randn(batch, Kd, N, generator=g).to(dtype).cuda())
+        out = torch.zeros(batch, M, N, dtype=out_dtype, device="cuda")
+        s = torch.cuda.Stream()
+        s.wait_stream(torch.cuda.current_stream())
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=s):
+            K.gemm_blas(a, b, out=out, alpha=alpha, beta=beta)
+        ad, bd = _f64(a), _f64(b).contiguous()
+        prod, mag = alpha * torch.bmm(ad, bd), abs(alpha) * torch.bmm(ad.abs(), bd.abs())
+        for _ in range(3):
+            c0 = torch.randn(batch, M, N, generator=g).to(out_dtype)
+            out.copy_(c0 if beta else torch.full_like(c0, float("nan")))
+            graph.replay()
+            torch.cuda.synchronize()
+            want, m = prod + beta * _f64(c0), mag + abs(beta) * _f64(c0).abs()
+            assert bool(((_f64(out) - want).abs() <= Kd * 2.0 ** -24 * m + eps * want.abs()).all())
+
+
 @pytest.mark.parametrize("M,N,Kd,splits", [(768, 3072, 8192, 4), (96, 64, 512, 8), (64, 32, 64, 1)])
 def test_gemm_blas_splitk(K, M, N, Kd, splits):
     """Weight-gradient form (A = Xᵀ stored [K, M]): split-K agrees with the

@@ -41,6 +41,7 @@
 // padded by 16 bytes, so the row-wise operand reads are conflict-free.
 #include "attn_common.h"
 
+#include <algorithm>
 #include <cmath>
 
 namespace mk {
@@ -87,31 +88,32 @@ __global__ __launch_bounds__(256) void attn_bwd_stats_kernel(const BwdArgs p, co
                                                             const float* __restrict__ lse,
                                                             float* __restrict__ stats) {
   constexpr int L = D / 8;
-  const int64_t t = (int64_t(blockIdx.x) * 256 + threadIdx.x) / L;
   const int ch = int(threadIdx.x) % L;
-  const int64_t per = int64_t(p.n_qt) * kTile;
-  if (t >= int64_t(p.BH) * per) return;  // whole rows: the 8 or 16 lanes of one leave together
-  const int64_t bh = t / per;
-  const int row = int(t % per);
-  float l2 = INFINITY, dsum = 0.f;
-  if (row < p.Sq) {
-    const int64_t b = bh / p.H, h = bh % p.H;
-    const u32x4_t a = *reinterpret_cast<const u32x4_t*>(o + b * o_bs + h * o_hs + row * o_ss + 8 * ch);
-    const u32x4_t c =
-        *reinterpret_cast<const u32x4_t*>(p.dout + b * p.do_bs + h * p.do_hs + row * p.do_ss + 8 * ch);
-    l2 = lse[bh * p.Sq + row] * kLog2e;
+  const int64_t per = int64_t(p.n_qt) * kTile, rows = int64_t(p.BH) * per;
+  // whole rows: the 8 or 16 lanes of one leave together
+  for (int64_t t = (int64_t(blockIdx.x) * 256 + threadIdx.x) / L; t < rows; t += int64_t(gridDim.x) * (256 / L)) {
+    const int64_t bh = t / per;
+    const int row = int(t % per);
+    float l2 = INFINITY, dsum = 0.f;
+    if (row < p.Sq) {
+      const int64_t b = bh / p.H, h = bh % p.H;
+      const u32x4_t a = *reinterpret_cast<const u32x4_t*>(o + b * o_bs + h * o_hs + row * o_ss + 8 * ch);
+      const u32x4_t c =
+          *reinterpret_cast<const u32x4_t*>(p.dout + b * p.do_bs + h * p.do_hs + row * p.do_ss + 8 * ch);
+      l2 = lse[bh * p.Sq + row] * kLog2e;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      dsum += __builtin_bit_cast(float, a[j] << 16) * __builtin_bit_cast(float, c[j] << 16);
-      dsum += __builtin_bit_cast(float, a[j] & 0xFFFF0000u) * __builtin_bit_cast(float, c[j] & 0xFFFF0000u);
+      for (int j = 0; j < 4; ++j) {
+        dsum += __builtin_bit_cast(float, a[j] << 16) * __builtin_bit_cast(float, c[j] << 16);
+        dsum += __builtin_bit_cast(float, a[j] & 0xFFFF0000u) * __builtin_bit_cast(float, c[j] & 0xFFFF0000u);
+      }
     }
-  }
 #pragma unroll
-  for (int x = L / 2; x >= 1; x >>= 1) dsum += __shfl_xor(dsum, x, kWave);
-  if (ch == 0) {
-    float* st = stats + (bh * p.n_qt + row / kTile) * (2 * kTile);
-    st[row % kTile] = l2;
-    st[kTile + row % kTile] = -dsum;
+    for (int x = L / 2; x >= 1; x >>= 1) dsum += __shfl_xor(dsum, x, kWave);
+    if (ch == 0) {
+      float* st = stats + (bh * p.n_qt + row / kTile) * (2 * kTile);
+      st[row % kTile] = l2;
+      st[kTile + row % kTile] = -dsum;
+    }
   }
 }
 
@@ -535,11 +537,13 @@ int sdpa_bwd_flash(hipStream_t s, int64_t B, int64_t H, int64_t Sq, int64_t Sk, 
   a.scale = scale;
 
   const int64_t nstat = int64_t(a.BH) * a.n_qt * kTile * (D / 8);  // lanes
+  // HIP refuses grids of 2^32 threads; the kernel walks what is left
+  const dim3 gs{unsigned(std::min<int64_t>((nstat + 255) / 256, (1 << 24) - 1))};
   if (D == 128)
-    hipLaunchKernelGGL(attn_bwd_stats_kernel<128>, dim3(unsigned((nstat + 255) / 256)), dim3(256), 0, s, a,
+    hipLaunchKernelGGL(attn_bwd_stats_kernel<128>, gs, dim3(256), 0, s, a,
                        (const uint16_t*)o, o_bs, o_hs, o_ss, lse, static_cast<float*>(workspace));
   else
-    hipLaunchKernelGGL(attn_bwd_stats_kernel<64>, dim3(unsigned((nstat + 255) / 256)), dim3(256), 0, s, a,
+    hipLaunchKernelGGL(attn_bwd_stats_kernel<64>, gs, dim3(256), 0, s, a,
                        (const uint16_t*)o, o_bs, o_hs, o_ss, lse, static_cast<float*>(workspace));
   if (int rc = check_launch("mk_sdpa_bwd")) return rc;
 

@@ -268,8 +268,10 @@ void launch(hipStream_t s, const SkinnyArgs& a, int64_t batch) {
 
 }  // namespace
 
+// N: a workgroup of 1024 threads per 64 columns, and HIP refuses grids of 2^32
+// threads
 bool gemm_skinny_fits(int64_t M, int64_t N, int64_t K, int64_t a_ks, int64_t b_ks, int64_t b_ns) {
-  return M <= 64 && N >= 16 && K >= 1 && a_ks == 1 && (b_ks == 1 || b_ns == 1);
+  return M <= 64 && N >= 16 && N <= (int64_t(1) << 27) && K >= 1 && a_ks == 1 && (b_ks == 1 || b_ns == 1);
 }
 
 int64_t gemm_skinny_slices(int ab_type, int64_t N, int64_t K, int64_t most) {

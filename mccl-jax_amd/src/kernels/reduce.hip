@@ -730,13 +730,23 @@ void with_team(int64_t rows, int64_t vecs, F f) {
   }
 }
 template <int W> dim3 team_grid(int64_t rows) { return dim3(unsigned((rows + Team<W>::kRows - 1) / Team<W>::kRows)); }
+// f(first row, rows) in runs that a launch takes: HIP refuses grids of 2^32
+// threads, 2^22 rows of a 16-wave team
+template <int W, class F>
+void for_row_runs(int64_t rows, F f) {
+  constexpr int64_t kMost = (int64_t(1) << 32) / (W * kWave) - Team<W>::kRows;
+  for (int64_t r = 0; r < rows; r += kMost) f(r, std::min(kMost, rows - r));
+}
 
 template <typename T, bool IS_F16, int OP>
 void launch_reduce_op(hipStream_t s, int64_t rows, int64_t cols, const void* x, float init, void* y, int out_type) {
   with_team(rows, cols / Vec<T>::N, [&](auto w) {
     constexpr int W = decltype(w)::value;
-    hipLaunchKernelGGL((row_reduce_kernel<T, IS_F16, OP, W>), team_grid<W>(rows), dim3(kTeamBlock<W>), 0, s,
-                       reinterpret_cast<const T*>(x), rows, cols, init, y, out_type);
+    for_row_runs<W>(rows, [&](int64_t r, int64_t n) {
+      hipLaunchKernelGGL((row_reduce_kernel<T, IS_F16, OP, W>), team_grid<W>(n), dim3(kTeamBlock<W>), 0, s,
+                         reinterpret_cast<const T*>(x) + r * cols, n, cols, init,
+                         static_cast<void*>(static_cast<char*>(y) + r * dtype_bytes(out_type)), out_type);
+    });
   });
 }
 
@@ -758,8 +768,11 @@ int launch_argmax_as(hipStream_t s, int64_t rows, int64_t cols, const void* x, v
   with_team(rows, cols / Vec<T>::N, [&](auto w) {
     constexpr int W = decltype(w)::value;
     auto go = [&](auto kernel) {
-      hipLaunchKernelGGL(kernel, team_grid<W>(rows), dim3(kTeamBlock<W>), 0, s, reinterpret_cast<const T*>(x), rows,
-                         cols, reinterpret_cast<T*>(values), reinterpret_cast<IdxT*>(indices));
+      for_row_runs<W>(rows, [&](int64_t r, int64_t n) {
+        T* v = reinterpret_cast<T*>(values);
+        hipLaunchKernelGGL(kernel, team_grid<W>(n), dim3(kTeamBlock<W>), 0, s, reinterpret_cast<const T*>(x) + r * cols,
+                           n, cols, v ? v + r : v, reinterpret_cast<IdxT*>(indices) + r);
+      });
     };
     if constexpr (sizeof(T) == 2) {
       if (cols <= 65536) return go(row_argmax_kernel<T, IS_F16, IS_MIN, IdxT, true, W>);
@@ -791,33 +804,34 @@ template <typename T, typename TO>
 void launch_layernorm_any(hipStream_t s, int64_t rows, int64_t cols, const T* x, const T* gamma, const T* beta,
                           float eps, TO* y, const T* x2 = nullptr, T* xsum = nullptr) {
   const int64_t vecs = cols / Vec<T>::N;
-  if (vecs > kTeamMaxVecs) {
-    hipLaunchKernelGGL((layernorm_loop_kernel<T, TO>), team_grid<16>(rows), dim3(kTeamBlock<16>), 0, s, x, gamma,
-                       beta, rows, cols, eps, y, x2, xsum);
-    return;
-  }
+  auto go = [&](auto w, auto kernel) {
+    constexpr int W = decltype(w)::value;
+    for_row_runs<W>(rows, [&](int64_t r, int64_t n) {
+      const int64_t at = r * cols;
+      hipLaunchKernelGGL(kernel, team_grid<W>(n), dim3(kTeamBlock<W>), 0, s, x + at, gamma, beta, n, cols, eps, y + at,
+                         x2 ? x2 + at : x2, xsum ? xsum + at : xsum);
+    });
+  };
+  if (vecs > kTeamMaxVecs) return go(Waves<16>{}, layernorm_loop_kernel<T, TO>);
   with_team(rows, vecs, [&](auto w) {
     constexpr int W = decltype(w)::value;
-    with_share(vecs, W, [&](auto kv) {
-      hipLaunchKernelGGL((layernorm_team_kernel<T, TO, W, decltype(kv)::value>), team_grid<W>(rows),
-                         dim3(kTeamBlock<W>), 0, s, x, gamma, beta, rows, cols, eps, y, x2, xsum);
-    });
+    with_share(vecs, W, [&](auto kv) { go(w, layernorm_team_kernel<T, TO, W, decltype(kv)::value>); });
   });
 }
 
 template <typename T>
 void launch_softmax(hipStream_t s, int64_t rows, int64_t cols, const T* x, T* y) {
   const int64_t vecs = cols / Vec<T>::N;
-  if (vecs > kTeamMaxVecs) {
-    hipLaunchKernelGGL((softmax_loop_kernel<T>), team_grid<16>(rows), dim3(kTeamBlock<16>), 0, s, x, rows, cols, y);
-    return;
-  }
+  auto go = [&](auto w, auto kernel) {
+    constexpr int W = decltype(w)::value;
+    for_row_runs<W>(rows, [&](int64_t r, int64_t n) {
+      hipLaunchKernelGGL(kernel, team_grid<W>(n), dim3(kTeamBlock<W>), 0, s, x + r * cols, n, cols, y + r * cols);
+    });
+  };
+  if (vecs > kTeamMaxVecs) return go(Waves<16>{}, softmax_loop_kernel<T>);
   with_team(rows, vecs, [&](auto w) {
     constexpr int W = decltype(w)::value;
-    with_share(vecs, W, [&](auto kv) {
-      hipLaunchKernelGGL((softmax_team_kernel<T, W, decltype(kv)::value>), team_grid<W>(rows), dim3(kTeamBlock<W>), 0,
-                         s, x, rows, cols, y);
-    });
+    with_share(vecs, W, [&](auto kv) { go(w, softmax_team_kernel<T, W, decltype(kv)::value>); });
   });
 }
 

@@ -1,0 +1,135 @@
+// The host side of the row kernels (src/kernels/reduce.hip), the GEMMs and
+// the attention backward against a HIP runtime that only writes down its
+// launches: the largest shapes the entry points take must stay within the
+// 2^32 - 1 threads per grid axis that HIP launches.  Nothing is allocated and
+// nothing runs on a GPU.  Prints "ok".
+#include <hip/hip_runtime_api.h>
+
+#include <cstdio>
+#include <cstdlib>
+#include <string>
+#include <utility>
+#include <vector>
+
+#include "mk_kernels.h"
+
+namespace {
+struct Launch {
+  uint64_t threads;         // along x
+  std::vector<void*> args;  // the first g_args arguments' first 8 bytes
+};
+std::vector<Launch> g_launches;
+int g_args = 4;
+dim3 g_grid, g_block;
+
+void expect(bool ok, const std::string& what) {
+  if (ok) return;
+  std::printf("FAILED: %s\n", what.c_str());
+  std::exit(1);
+}
+void* ptr(uint64_t v) { return reinterpret_cast<void*>(v); }
+
+// every launch within the limit
+void limits(const std::string& what, int rc) {
+  expect(rc == MK_OK && !g_launches.empty(), what + ": not launched");
+  for (const Launch& l : g_launches)
+    expect(l.threads < (uint64_t(1) << 32), what + ": " + std::to_string(l.threads) + " threads along x");
+}
+// the launches' rows (argument rows_arg), each from where the one before ended
+// (argument 0, a row being row_bytes), are all `rows` rows
+void covers(const std::string& what, int rc, uint64_t x, int64_t rows, uint64_t row_bytes, int rows_arg) {
+  limits(what, rc);
+  uint64_t at = 0;
+  for (const Launch& l : g_launches) {
+    expect(reinterpret_cast<uint64_t>(l.args[0]) == x + at * row_bytes, what + ": a gap in the rows");
+    at += reinterpret_cast<uint64_t>(l.args[rows_arg]);
+  }
+  expect(at == uint64_t(rows), what + ": " + std::to_string(at) + " rows of " + std::to_string(rows));
+  g_launches.clear();
+}
+}  // namespace
+
+// ---------------------------------------------------------------- the runtime
+extern "C" {
+hipError_t hipGetLastError() { return hipSuccess; }
+const char* hipGetErrorString(hipError_t) { return "error"; }
+hipError_t hipGetDevice(int* d) { return *d = 0, hipSuccess; }
+hipError_t hipDeviceGetAttribute(int* v, hipDeviceAttribute_t, int) { return *v = 256, hipSuccess; }
+hipError_t hipFuncSetAttribute(const void*, hipFuncAttribute, int) { return hipSuccess; }
+void** __hipRegisterFatBinary(const void*) { return nullptr; }
+void __hipRegisterFunction(void**, const void*, char*, const char*, unsigned, void*, void*, void*, void*, int*) {}
+void __hipUnregisterFatBinary(void**) {}
+hipError_t __hipPushCallConfiguration(dim3 g, dim3 b, size_t, hipStream_t) { return g_grid = g, g_block = b, hipSuccess; }
+hipError_t __hipPopCallConfiguration(dim3* g, dim3* b, size_t* lds, hipStream_t* s) {
+  return *g = g_grid, *b = g_block, *lds = 0, *s = nullptr, hipSuccess;
+}
+hipError_t hipLaunchKernel(const void*, dim3 g, dim3 b, void** args, size_t, hipStream_t) {
+  Launch l{uint64_t(g.x) * b.x, {}};
+  expect(g.x > 0 && g.y > 0 && g.z > 0 && g.y < 65536 && g.z < 65536, "an empty or too large grid");
+  for (int i = 0; i < g_args; ++i) l.args.push_back(*static_cast<void**>(args[i]));
+  return g_launches.push_back(l), hipSuccess;
+}
+}
+
+namespace mk {
+int sdpa_bwd_flash(hipStream_t, int64_t B, int64_t H, int64_t Sq, int64_t Sk, int64_t D, const void*, int64_t, int64_t,
+                   int64_t, const void*, int64_t, int64_t, int64_t, const void*, int64_t, int64_t, int64_t, const void*,
+                   int64_t, int64_t, int64_t, const void*, int64_t, int64_t, int64_t, const float*, void*, int64_t,
+                   int64_t, int64_t, void*, int64_t, int64_t, int64_t, void*, int64_t, int64_t, int64_t, float, int,
+                   void*);
+// takes at least 128 rows
+int gemm_tiled(hipStream_t, int, int64_t, int64_t, int64_t, int64_t, const void*, int64_t, int64_t, int64_t, const void*,
+               int64_t, int64_t, int64_t, void*, int64_t, int64_t, const void*, int, int64_t, void*, int64_t, float*) {
+  return -1;
+}
+void clear_error() {}
+int fail(int code, const std::string& what) { return std::printf("%s\n", what.c_str()), code; }
+int check_launch(const char*) { return MK_OK; }
+}  // namespace mk
+
+int main() {
+  const uint64_t X = uint64_t(1) << 44, Y = uint64_t(1) << 46;  // never touched
+  // rows at the teams' limits (2^22, 2^24 and 2^26 rows of 16, 4 and 1 waves), lengths of each team
+  for (int64_t rows : {int64_t(1) << 22, (int64_t(1) << 24) - 1, (int64_t(1) << 24) + 3, (int64_t(1) << 26) - 1,
+                       (int64_t(1) << 26) + 5})
+    for (int64_t cols : {7, 2048, 4104, 16400, 70001, 530000})
+      for (int t : {MK_BF16, MK_F32}) {
+        const uint64_t row = uint64_t(cols) * (t == MK_BF16 ? 2 : 4);
+        const std::string at = " of " + std::to_string(rows) + " x " + std::to_string(cols);
+        covers("sum" + at, mk_row_reduce(nullptr, t, MK_F32, 0, rows, cols, ptr(X), 0.f, ptr(Y)), X, rows, row, 1);
+        covers("argmax" + at, mk_row_argmax(nullptr, t, 0, rows, cols, ptr(X), nullptr, MK_S32, ptr(Y)), X, rows, row, 1);
+        covers("softmax" + at, mk_softmax_rows(nullptr, t, rows, cols, ptr(X), ptr(Y)), X, rows, row, 1);
+        // + 2 / 4: rows off the 16-byte grid, on the kernels that take any alignment
+        covers("LayerNorm" + at, mk_layernorm(nullptr, t, rows, cols, ptr(X + (t == MK_BF16 ? 2 : 4)), nullptr, nullptr,
+                                              1e-5f, ptr(Y)), X + (t == MK_BF16 ? 2 : 4), rows, row, 3);
+        if (t == MK_F32)
+          covers("add + LayerNorm" + at, mk_add_layernorm_typed(nullptr, t, MK_BF16, rows, cols, ptr(X + 4), ptr(X), nullptr,
+                                                                nullptr, nullptr, 1e-5f, ptr(Y), ptr(Y)), X + 4, rows, row, 3);
+      }
+
+  // the backward's row statistics: 8 or 16 lanes a row
+  g_args = 0;
+  for (int64_t D : {64, 128}) {
+    const int64_t H = 1 << 18, Sq = D == 64 ? 2048 : 1024, n = Sq * D, z = 64 * D;
+    float* lse = static_cast<float*>(ptr(X));
+    limits("attention backward, head_dim " + std::to_string(D),
+           mk::sdpa_bwd_flash(nullptr, 1, H, Sq, 64, D, ptr(X), 0, n, D, ptr(X), 0, z, D, ptr(X), 0, z, D, ptr(X), 0, n,
+                              D, ptr(X), 0, n, D, lse, ptr(Y), 0, n, D, ptr(Y), 0, z, D, ptr(Y), 0, z, D, 1.f, 0,
+                              ptr(Y)));
+    g_launches.clear();
+  }
+
+  // few rows and any number of columns: up to the 2^31 (bf16) and 2^30 (fp32)
+  // that 256 and 512 threads per 128 columns allow
+  for (int64_t M : {1, 16, 17, 64})
+    for (int64_t N : {(int64_t(1) << 28) - 1, (int64_t(1) << 28) + 1, (int64_t(1) << 29) + 5, (int64_t(1) << 30) - 128})
+      for (int64_t K : {1, 64, 512, 16384})
+        for (int t : {MK_BF16, MK_F32})
+          for (bool kc : {false, true}) {
+            limits("few rows, N " + std::to_string(N) + ", K " + std::to_string(K),
+                   mk_gemm(nullptr, t, t, 1, M, N, K, ptr(X), 0, K, 1, ptr(X), 0, kc ? 1 : N, kc ? K : 1, ptr(Y), 0, N,
+                           nullptr, 0));
+            g_launches.clear();
+          }
+  std::printf("ok\n");
+}

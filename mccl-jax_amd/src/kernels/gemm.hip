@@ -333,35 +333,6 @@ GemmArgs gemm_args(int esz, int c_type, int64_t M, int64_t N, int64_t K, const v
 }
 
 }  // namespace
-
-int gemm_own(hipStream_t s, int ab_type, int c_type, int64_t batch, int64_t M, int64_t N, int64_t K, const void* A,
-             int64_t a_bs, int64_t a_ms, int64_t a_ks, const void* B, int64_t b_bs, int64_t b_ks, int64_t b_ns,
-             void* C, int64_t c_bs, int64_t c_ms, float alpha, float beta) {
-  const int esz = ab_type == MK_BF16 ? 2 : 4;
-  constexpr int64_t kMost = 65535;  // batches of one launch
-  for (int64_t b0 = 0; b0 < batch; b0 += kMost) {
-    const int64_t nb = batch - b0 < kMost ? batch - b0 : kMost;
-    const char* Ab = static_cast<const char*>(A) + b0 * a_bs * esz;
-    const char* Bb = static_cast<const char*>(B) + b0 * b_bs * esz;
-    char* Cb = static_cast<char*>(C) + b0 * c_bs * dtype_bytes(c_type);
-    int rc;
-    if (alpha == 1.f && beta == 0.f) {
-      rc = mk_gemm(s, ab_type, c_type, nb, M, N, K, Ab, a_bs, a_ms, a_ks, Bb, b_bs, b_ks, b_ns, Cb, c_bs, c_ms,
-                   nullptr, 0);
-    } else {
-      GemmArgs a = gemm_args(esz, c_type, M, N, K, Ab, a_bs, a_ms, a_ks, Bb, b_bs, b_ks, b_ns, Cb, c_bs, c_ms,
-                             nullptr, 0);
-      a.alpha = alpha;
-      a.beta = beta;
-      const bool a_kc = a_ks == 1 || K == 1, b_kc = b_ks == 1 || K == 1;
-      rc = ab_type == MK_BF16 ? launch_gemm<uint16_t, true>(s, a, nb, a_kc, b_kc)
-                              : launch_gemm<float, true>(s, a, nb, a_kc, b_kc);
-    }
-    if (rc) return rc;
-  }
-  return MK_OK;
-}
-
 }  // namespace mk
 
 using namespace mk;
@@ -442,11 +413,12 @@ extern "C" int mk_gemm(void* stream, int ab_type, int c_type, int64_t batch, int
   const GemmArgs a = gemm_args(esz, c_type, M, N, K, A, a_bs, a_ms, a_ks, B, b_bs, b_ks, b_ns, C, c_bs, c_ms, bias,
                                epilogue);
   hipStream_t s = as_stream(stream);
-  // few rows: one pass over B whatever its size, strides and alignment
-  if (const int r = gemm_skinny(s, ab_type, c_type, batch, M, N, K, A, a_bs, a.a_ms, a.a_ks, B, b_bs, a.b_ks, a.b_ns,
-                                C, c_bs, c_ms, bias, epilogue);
-      r >= 0)
-    return r;
+  // few rows: one pass over B, of any strides and alignment
+  if (gemm_skinny_pays(ab_type, batch, M, N, K, b_kc, a.vec_b)) {
+    const int r = gemm_skinny(s, ab_type, c_type, batch, M, N, K, A, a_bs, a.a_ms, a.a_ks, B, b_bs, a.b_ks, a.b_ns, C,
+                              c_bs, c_ms, bias, epilogue);
+    if (r >= 0) return r;
+  }
   if (ab_type == MK_BF16) {
     const int r = gemm_tiled(s, c_type, batch, M, N, K, A, a_bs, a_ms, a_ks, B, b_bs, b_ks, b_ns, C, c_bs,
                              c_ms, bias, epilogue);
@@ -536,3 +508,33 @@ extern "C" int mk_gemm_splitk(void* stream, int ab_type, int64_t M, int64_t N, i
   return mk_gemm_splitk_typed(stream, ab_type, MK_F32, M, N, K, A, a_ms, a_ks, B, b_ks, b_ns, C, c_ms, splits,
                               workspace, nullptr, 0);
 }
+
+namespace mk {
+int gemm_own(hipStream_t s, int ab_type, int c_type, int64_t batch, int64_t M, int64_t N, int64_t K, const void* A,
+             int64_t a_bs, int64_t a_ms, int64_t a_ks, const void* B, int64_t b_bs, int64_t b_ks, int64_t b_ns,
+             void* C, int64_t c_bs, int64_t c_ms, float alpha, float beta) {
+  const int esz = ab_type == MK_BF16 ? 2 : 4;
+  constexpr int64_t kMost = 65535;  // batches of one launch
+  for (int64_t b0 = 0; b0 < batch; b0 += kMost) {
+    const int64_t nb = batch - b0 < kMost ? batch - b0 : kMost;
+    const char* Ab = static_cast<const char*>(A) + b0 * a_bs * esz;
+    const char* Bb = static_cast<const char*>(B) + b0 * b_bs * esz;
+    char* Cb = static_cast<char*>(C) + b0 * c_bs * dtype_bytes(c_type);
+    int rc;
+    if (alpha == 1.f && beta == 0.f) {
+      rc = mk_gemm(s, ab_type, c_type, nb, M, N, K, Ab, a_bs, a_ms, a_ks, Bb, b_bs, b_ks, b_ns, Cb, c_bs, c_ms,
+                   nullptr, 0);
+    } else {
+      GemmArgs a = gemm_args(esz, c_type, M, N, K, Ab, a_bs, a_ms, a_ks, Bb, b_bs, b_ks, b_ns, Cb, c_bs, c_ms,
+                             nullptr, 0);
+      a.alpha = alpha;
+      a.beta = beta;
+      const bool a_kc = a_ks == 1 || K == 1, b_kc = b_ks == 1 || K == 1;
+      rc = ab_type == MK_BF16 ? launch_gemm<uint16_t, true>(s, a, nb, a_kc, b_kc)
+                              : launch_gemm<float, true>(s, a, nb, a_kc, b_kc);
+    }
+    if (rc) return rc;
+  }
+  return MK_OK;
+}
+}  // namespace mk

@@ -274,6 +274,27 @@ bool gemm_skinny_fits(int64_t M, int64_t N, int64_t K, int64_t a_ks, int64_t b_k
   return M <= 64 && N >= 16 && N <= (int64_t(1) << 27) && K >= 1 && a_ks == 1 && (b_ks == 1 || b_ns == 1);
 }
 
+bool gemm_skinny_pays(int ab_type, int64_t batch, int64_t M, int64_t N, int64_t K, bool b_kc, bool b_aligned) {
+  // A workgroup of this kernel fills a CU and takes 2 - 5 us however short k
+  // is (the first loads, the waves' sums through LDS: MT 16-row blocks of
+  // them), so it pays where its workgroups are few or k is long.  Up to one
+  // workgroup of either kernel per CU it is always ahead, but for 33 - 64 rows
+  // at k of a few steps.  Past that the two were timed on 3000 products
+  // (batches up to 4096, 16 - 131072 columns, k 8 - 4096): the least k from
+  // which this kernel is no slower grows with MT, is shorter where the general
+  // kernel's last 128-column tile is half empty, and is longer where that
+  // kernel is at its best, k-contiguous bf16 on the 16-byte grid.  4096 x 64 x
+  // 8 x 512 (batch x M x K x N), bf16: general 313 us, this kernel 608; 4096 x
+  // 64 x 128 x 128 k-contiguous 90 and 163; 512 x 64 x 512 x 64: 38 and 20.
+  const int64_t tiles = (N + 127) / 128 * batch, mine = (N + 63) / 64 * batch, mt = M <= 16 ? 1 : M <= 32 ? 2 : 4;
+  if (mine <= 256) return true;
+  if (tiles <= 256) return K >= 32 * mt;
+  const bool half = 2 * mine < 3 * tiles;
+  if (ab_type != MK_BF16) return K >= (!b_aligned ? 32 : half ? 16 : b_kc ? 96 : 64) * mt;
+  if (!b_aligned) return K >= (b_kc ? 96 : 32) * mt;
+  return K >= (b_kc ? (half ? 128 : 2048) : (half ? 64 : 256)) * mt;
+}
+
 int64_t gemm_skinny_slices(int ab_type, int64_t N, int64_t K, int64_t most) {
   // a workgroup's time is its lines at 8 clocks each, one 128-byte line per
   // k-row of bf16, two of fp32: below 2048 lines (about 7 us) it costs no

@@ -89,7 +89,10 @@ int gemm_tiled(hipStream_t s, int c_type, int64_t batch, int64_t M, int64_t N, i
 // strides do not fit it (gemm_skinny_fits), else MK_OK or an MK_ERR_* code.
 // slices > 1 (batch 1): slice i of k writes its partial product at C + i c_bs;
 // gemm_skinny_slices: how many of at most `most` slices pay.
+// gemm_skinny_pays: whether it is no slower than the general kernel
+// (b_aligned: B's rows on the 16-byte grid).
 bool gemm_skinny_fits(int64_t M, int64_t N, int64_t K, int64_t a_ks, int64_t b_ks, int64_t b_ns);
+bool gemm_skinny_pays(int ab_type, int64_t batch, int64_t M, int64_t N, int64_t K, bool b_kc, bool b_aligned);
 int gemm_skinny(hipStream_t s, int ab_type, int c_type, int64_t batch, int64_t M, int64_t N, int64_t K,
                 const void* A, int64_t a_bs, int64_t a_ms, int64_t a_ks, const void* B, int64_t b_bs, int64_t b_ks,
                 int64_t b_ns, void* C, int64_t c_bs, int64_t c_ms, const void* bias, int epilogue,

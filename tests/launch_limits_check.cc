@@ -1,7 +1,8 @@
 // The host side of the row kernels (src/kernels/reduce.hip), the GEMMs and
 // the attention backward against a HIP runtime that only writes down its
 // launches: the largest shapes the entry points take must stay within the
-// 2^32 - 1 threads per grid axis that HIP launches.  Nothing is allocated and
+// 2^32 - 1 threads per grid axis that HIP launches, and products of few rows
+// must run on the kernel that the dispatch rule names.  Nothing is allocated and
 // nothing runs on a GPU.  Prints "ok".
 #include <hip/hip_runtime_api.h>
 
@@ -15,7 +16,7 @@
 
 namespace {
 struct Launch {
-  uint64_t threads;         // along x
+  uint64_t threads, grid;   // along x
   std::vector<void*> args;  // the first g_args arguments' first 8 bytes
 };
 std::vector<Launch> g_launches;
@@ -64,7 +65,7 @@ hipError_t __hipPopCallConfiguration(dim3* g, dim3* b, size_t* lds, hipStream_t*
   return *g = g_grid, *b = g_block, *lds = 0, *s = nullptr, hipSuccess;
 }
 hipError_t hipLaunchKernel(const void*, dim3 g, dim3 b, void** args, size_t, hipStream_t) {
-  Launch l{uint64_t(g.x) * b.x, {}};
+  Launch l{uint64_t(g.x) * b.x, g.x, {}};
   expect(g.x > 0 && g.y > 0 && g.z > 0 && g.y < 65536 && g.z < 65536, "an empty or too large grid");
   for (int i = 0; i < g_args; ++i) l.args.push_back(*static_cast<void**>(args[i]));
   return g_launches.push_back(l), hipSuccess;
@@ -131,5 +132,24 @@ int main() {
                            nullptr, 0));
             g_launches.clear();
           }
+
+  // few rows: many short products stay on the 128-column tiles, deep or few
+  // ones run on the kernel that reads B once (16- to 64-column workgroups)
+  struct { int64_t batch, M, N, K; int type; bool kc, tiles; } routes[] = {
+      {4096, 64, 512, 8, MK_BF16, false, true},    {4096, 64, 128, 128, MK_BF16, true, true},
+      {512, 64, 256, 64, MK_F32, false, true},     {1, 33, 65536, 16, MK_BF16, true, true},
+      {4096, 1, 1024, 128, MK_BF16, true, true},   {1, 16, 16384, 4096, MK_BF16, false, false},
+      {512, 64, 64, 512, MK_BF16, false, false},   {1, 64, 4096, 8, MK_F32, true, false},
+      {4096, 16, 192, 64, MK_F32, false, false},    {512, 8, 128, 2048, MK_BF16, true, false},
+      {2, 64, 16384, 96, MK_F32, false, true},     {2, 64, 16384, 128, MK_F32, false, false}};
+  for (const auto& r : routes) {
+    limits("few rows", mk_gemm(nullptr, r.type, r.type, r.batch, r.M, r.N, r.K, ptr(X), r.M * r.K, r.K, 1, ptr(X),
+                               r.K * r.N, r.kc ? 1 : r.N, r.kc ? r.K : 1, ptr(Y), r.M * r.N, r.N, nullptr, 0));
+    const uint64_t tiles = (r.N + 127) / 128, block = r.type == MK_BF16 ? 256 : 512;
+    expect((g_launches[0].grid == tiles && g_launches[0].threads == tiles * block) == r.tiles,
+           "the kernel of " + std::to_string(r.batch) + " x " + std::to_string(r.M) + " x " + std::to_string(r.K) +
+               " x " + std::to_string(r.N));
+    g_launches.clear();
+  }
   std::printf("ok\n");
 }

@@ -92,26 +92,61 @@ struct Team {
   }
 };
 
-// f(i, vector i) for the lane's vectors of a row, up to 4 loads in flight
+// What a row's lanes read (one wave per row only, but for kLoop): kElements
+// one or two elements and no vector (nv 0), kOne at most one vector, kLoop any
+// number of them.  Rows of at most 64 elements, or 128 where they are no whole
+// vectors, are read by element: more lanes share the arithmetic; and without
+// the loop a short row's wave is a few instructions shorter (65536 rows, bf16, in
+// us with vectors and the loop / so: sum of 7 9.6 / 8.4, max of 100 13.0 / 10.5,
+// softmax of 64 18.4 / 13.0, LayerNorm of 65 25.1 / 18.0).
+enum RowPath { kElements, kOne, kLoop };
+
+// f(i, vector i) for the lane's vectors of a row in order, 4 loads in flight.
+// The last up to 4 per lane are loaded together too, lanes past the end the
+// last vector: with a branch per lane around them a wave waited up to three
+// times (argmax of 4096 x 2000 bf16: 6.4 us, 5.1 now).
 template <int W, typename T, class F>
 __device__ inline void for_vectors(const T* xr, int64_t nv, int t, F f) {
   constexpr int S = W * kWave, N = Vec<T>::N;
-  int64_t i = t;
-  for (; i + 3 * S < nv; i += 4 * S) {
-    const u32x4_t a = ld_row(xr + i * N), b = ld_row(xr + (i + S) * N);
-    const u32x4_t c = ld_row(xr + (i + 2 * S) * N), d = ld_row(xr + (i + 3 * S) * N);
-    f(i, a);
-    f(i + S, b);
-    f(i + 2 * S, c);
-    f(i + 3 * S, d);
+  int64_t base = 0;
+  for (; base + 4 * S <= nv; base += 4 * S) {
+    const T* p = xr + (base + t) * N;
+    const u32x4_t a = ld_row(p), b = ld_row(p + S * N), c = ld_row(p + 2 * S * N), d = ld_row(p + 3 * S * N);
+    f(base + t, a);
+    f(base + t + S, b);
+    f(base + t + 2 * S, c);
+    f(base + t + 3 * S, d);
   }
-  if (i + S < nv) {
-    const u32x4_t a = ld_row(xr + i * N), b = ld_row(xr + (i + S) * N);
-    f(i, a);
-    f(i + S, b);
-    i += 2 * S;
+  const int64_t i = base + t;
+  auto rest = [&](auto count) __attribute__((always_inline)) {
+    constexpr int C = decltype(count)::value;
+    u32x4_t v[C];
+#pragma unroll
+    for (int k = 0; k < C; ++k) v[k] = ld_row(xr + (i + k * S < nv ? i + k * S : nv - 1) * N);
+#pragma unroll
+    for (int k = 0; k < C; ++k)
+      if (i + k * S < nv) f(i + k * S, v[k]);
+  };
+  const int64_t left = nv - base;  // uniform
+  if (left > 2 * S) rest(std::integral_constant<int, 4>{});
+  else if (left > S) rest(std::integral_constant<int, 2>{});
+  else if (left > 0) rest(std::integral_constant<int, 1>{});
+}
+
+template <int W, RowPath PATH, typename T, class F>
+__device__ inline void row_vectors(const T* xr, int64_t nv, int t, F f) {
+  if constexpr (PATH == kLoop) for_vectors<W>(xr, nv, t, f);
+  else if constexpr (PATH == kOne) {
+    if (t < nv) f(int64_t(t), ld_row(xr + t * Vec<T>::N));
   }
-  if (i < nv) f(i, ld_row(xr + i * N));
+}
+
+// f(c) for the lane's elements past the vectors, the first of them at c
+template <int W, RowPath PATH, class F>
+__device__ inline void row_elements(int64_t c, int64_t cols, F f) {
+  if (c < cols) f(c);
+  if constexpr (PATH == kElements)
+    if (c + W * kWave < cols) f(c + W * kWave);
 }
 
 // element j of a 16-byte vector as fp32
@@ -128,9 +163,9 @@ __device__ inline float elem(const u32x4_t& v, int j) {
 
 // StableHLO max/min propagate NaN; fmaxf/fminf drop it, so NaN is tracked
 // separately for OP 1/2.
-template <typename T, bool IS_F16, int OP, int W>
+template <typename T, bool IS_F16, int OP, int W, RowPath PATH>
 __global__ __launch_bounds__(kTeamBlock<W>) void row_reduce_kernel(const T* __restrict__ x, int64_t rows,
-                                                                   int64_t cols, float init, void* y,
+                                                                   int64_t cols, int64_t nv, float init, void* y,
                                                                    int out_type) {
   __shared__ float red[W];
   __shared__ int red_nan[W];
@@ -138,18 +173,17 @@ __global__ __launch_bounds__(kTeamBlock<W>) void row_reduce_kernel(const T* __re
   if (W == 1 && tm.row >= rows) return;
   const T* xr = x + tm.row * cols;
   constexpr int N = Vec<T>::N;
-  const int64_t nv = cols / N;
   float acc = identity<OP>();
   bool nan = false;
   auto take = [&](float f) {
     nan |= (f != f);
     acc = combine<OP>(acc, f);
   };
-  for_vectors<W>(xr, nv, tm.t, [&](int64_t, const u32x4_t& v) {
+  row_vectors<W, PATH>(xr, nv, tm.t, [&](int64_t, const u32x4_t& v) {
 #pragma unroll
     for (int j = 0; j < N; ++j) take(elem<T, IS_F16>(v, j));
   });
-  if (nv * N + tm.t < cols) take(ld<T, IS_F16>(xr[nv * N + tm.t]));
+  row_elements<W, PATH>(nv * N + tm.t, cols, [&](int64_t c) { take(ld<T, IS_F16>(xr[c])); });
   acc = tm.combine(wave_combine<OP>(acc), red, [](float a, float b) { return combine<OP>(a, b); });
   // the vote must run with the whole wave active, before the lane-0 branch
   const int any_nan = tm.combine(int(__any(nan)), red_nan, [](int a, int b) { return a | b; });
@@ -200,9 +234,9 @@ __device__ inline uint32_t order_key32(uint32_t w) {
 // (key << 16) | (0xFFFF - index), so the row winner is the unsigned max of
 // the words.  Otherwise key and index are kept apart; a lane visits its
 // elements in increasing index, so only a larger key replaces its winner.
-template <typename T, bool IS_F16, bool IS_MIN, typename IdxT, bool NARROW, int W>
+template <typename T, bool IS_F16, bool IS_MIN, typename IdxT, bool NARROW, int W, RowPath PATH>
 __global__ __launch_bounds__(kTeamBlock<W>) void row_argmax_kernel(const T* __restrict__ x, int64_t rows,
-                                                                   int64_t cols, T* __restrict__ values,
+                                                                   int64_t cols, int64_t nv, T* __restrict__ values,
                                                                    IdxT* __restrict__ indices) {
   constexpr uint32_t kInf = IS_F16 ? 0x7C00u : 0x7F80u;
   constexpr int N = Vec<T>::N;
@@ -211,12 +245,12 @@ __global__ __launch_bounds__(kTeamBlock<W>) void row_argmax_kernel(const T* __re
   const Team<W> tm;
   if (W == 1 && tm.row >= rows) return;
   const T* xr = x + tm.row * cols;
-  const int64_t nv = cols / N, tail = nv * N + tm.t;
+  const int64_t tail = nv * N + tm.t;
   uint32_t best = 0;  // below every element's word; at or below every key
   int64_t at = INT64_MAX;
   if constexpr (NARROW) {
     static_assert(sizeof(T) == 2, "16-bit floats");
-    for_vectors<W>(xr, nv, tm.t, [&](int64_t i, const u32x4_t& v) {
+    row_vectors<W, PATH>(xr, nv, tm.t, [&](int64_t i, const u32x4_t& v) {
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         const uint32_t k = order_keys<IS_MIN, kInf>(v[j]);
@@ -225,7 +259,9 @@ __global__ __launch_bounds__(kTeamBlock<W>) void row_argmax_kernel(const T* __re
         best = max(best, max(p0, p1));
       }
     });
-    if (tail < cols) best = max(best, (order_keys<IS_MIN, kInf>(xr[tail]) << 16) | (0xFFFFu - uint32_t(tail)));
+    row_elements<W, PATH>(tail, cols, [&](int64_t c) {
+      best = max(best, (order_keys<IS_MIN, kInf>(xr[c]) << 16) | (0xFFFFu - uint32_t(c)));
+    });
 #pragma unroll
     for (int m = 32; m >= 1; m >>= 1) best = max(best, uint32_t(__shfl_xor(int(best), m, kWave)));
     best = tm.combine(best, red_key, [](uint32_t a, uint32_t b) { return max(a, b); });
@@ -234,7 +270,7 @@ __global__ __launch_bounds__(kTeamBlock<W>) void row_argmax_kernel(const T* __re
     auto take = [&](uint32_t key, int64_t i) {
       if (key > best || at == INT64_MAX) best = key, at = i;
     };
-    for_vectors<W>(xr, nv, tm.t, [&](int64_t i, const u32x4_t& v) {
+    row_vectors<W, PATH>(xr, nv, tm.t, [&](int64_t i, const u32x4_t& v) {
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         if constexpr (sizeof(T) == 2) {
@@ -246,10 +282,10 @@ __global__ __launch_bounds__(kTeamBlock<W>) void row_argmax_kernel(const T* __re
         }
       }
     });
-    if (tail < cols) {
-      if constexpr (sizeof(T) == 2) take(order_keys<IS_MIN, kInf>(xr[tail]) & 0xFFFFu, tail);
-      else take(order_key32<IS_MIN>(__builtin_bit_cast(uint32_t, xr[tail])), tail);
-    }
+    row_elements<W, PATH>(tail, cols, [&](int64_t c) {
+      if constexpr (sizeof(T) == 2) take(order_keys<IS_MIN, kInf>(xr[c]) & 0xFFFFu, c);
+      else take(order_key32<IS_MIN>(__builtin_bit_cast(uint32_t, xr[c])), c);
+    });
     // lanes without an element hold (0, INT64_MAX) and lose every tie
 #pragma unroll
     for (int m = 32; m >= 1; m >>= 1) {
@@ -461,26 +497,28 @@ __global__ __launch_bounds__(kBlock) void layernorm_bf16_split_kernel(
 // A lane's share of a team's row: KV 16-byte vectors (vector t + 64 W k; nv
 // whole ones in the row) and the row's element nv N + t past them.  The loads
 // are unconditional (vector 0 where the row has no such vector), so all of
-// them are in flight together.
+// them are in flight together.  KV = 0: no vectors, the row's elements t and
+// t + 64 W.
 template <typename T, int W, int KV>
 struct RowShare {
-  static constexpr int N = Vec<T>::N, S = W * kWave;
-  u32x4_t v[KV];
-  float tail;
-  int64_t nv;
+  static constexpr int N = Vec<T>::N, S = W * kWave, E = KV > 0 ? 1 : 2;
+  u32x4_t v[KV > 0 ? KV : 1];
+  float tail[E];
+  int64_t nv, cols;
   int t;
-  bool has_tail;
-  __device__ inline RowShare(const T* xr, int64_t cols, int t_) : t(t_) {
-    nv = cols / N;
-    has_tail = nv * N + t < cols;
+  __device__ inline RowShare(const T* xr, int64_t cols_, int t_) : cols(cols_), t(t_) {
+    nv = KV > 0 ? cols / N : 0;
     if (nv > 0) {
 #pragma unroll
       for (int k = 0; k < KV; ++k) v[k] = ld_row(xr + (has(k) ? t + k * S : 0) * int64_t(N));
     }
-    tail = has_tail ? to_f32<T>(xr[nv * N + t]) : 0.f;
+#pragma unroll
+    for (int e = 0; e < E; ++e) tail[e] = has_tail(e) ? to_f32<T>(xr[tail_at(e)]) : 0.f;
   }
   __device__ inline bool has(int k) const { return t + k * S < nv; }
   __device__ inline float at(int k, int j) const { return elem<T, false>(v[k], j); }
+  __device__ inline int64_t tail_at(int e) const { return nv * N + t + e * S; }
+  __device__ inline bool has_tail(int e) const { return tail_at(e) < cols; }
 };
 
 template <typename T>
@@ -514,7 +552,6 @@ __global__ __launch_bounds__(kTeamBlock<W>) void layernorm_team_kernel(
   const Team<W> tm;
   if (W == 1 && tm.row >= rows) return;
   R r(x + tm.row * cols, cols, tm.t);
-  const int64_t tail = r.nv * N + tm.t;
   if constexpr (sizeof(T) == 4) {
     if (x2) {
       const R r2(x2 + tm.row * cols, cols, tm.t);
@@ -529,20 +566,28 @@ __global__ __launch_bounds__(kTeamBlock<W>) void layernorm_team_kernel(
         }
         if (r.has(k)) st_values<T, N>(sr + int64_t(tm.t + k * R::S) * N, o);
       }
-      r.tail += r2.tail;
-      if (r.has_tail) sr[tail] = r.tail;
+#pragma unroll
+      for (int e = 0; e < R::E; ++e) {
+        r.tail[e] += r2.tail[e];
+        if (r.has_tail(e)) sr[r.tail_at(e)] = r.tail[e];
+      }
     }
   }
   auto add = [](float a, float b) { return a + b; };
   const float inv_n = 1.f / float(cols);
-  float s = r.tail;
+  float s = r.tail[0];
+#pragma unroll
+  for (int e = 1; e < R::E; ++e) s += r.tail[e];
 #pragma unroll
   for (int k = 0; k < KV; ++k)
     if (r.has(k))
 #pragma unroll
       for (int j = 0; j < N; ++j) s += r.at(k, j);
   const float mean = tm.combine(wave_sum(s), red[0], add) * inv_n;
-  float q = r.has_tail ? (r.tail - mean) * (r.tail - mean) : 0.f;
+  float q = 0.f;
+#pragma unroll
+  for (int e = 0; e < R::E; ++e)
+    if (r.has_tail(e)) q += (r.tail[e] - mean) * (r.tail[e] - mean);
 #pragma unroll
   for (int k = 0; k < KV; ++k)
     if (r.has(k))
@@ -565,9 +610,13 @@ __global__ __launch_bounds__(kTeamBlock<W>) void layernorm_team_kernel(
       o[j] = (r.at(k, j) - mean) * rstd * (gamma ? elem<T, false>(g, j) : 1.f) + elem<T, false>(b, j);
     st_values<TO, N>(yr + c, o);
   }
-  if (r.has_tail)
-    yr[tail] = narrow<TO>((r.tail - mean) * rstd * (gamma ? to_f32<T>(gamma[tail]) : 1.f) +
-                          (beta ? to_f32<T>(beta[tail]) : 0.f));
+#pragma unroll
+  for (int e = 0; e < R::E; ++e) {
+    if (!r.has_tail(e)) continue;
+    const int64_t c = r.tail_at(e);
+    yr[c] = narrow<TO>((r.tail[e] - mean) * rstd * (gamma ? to_f32<T>(gamma[c]) : 1.f) +
+                       (beta ? to_f32<T>(beta[c]) : 0.f));
+  }
 }
 
 // LayerNorm of rows longer than a 16-wave team holds: three passes over the
@@ -639,14 +688,17 @@ __global__ __launch_bounds__(kTeamBlock<W>) void softmax_team_kernel(const T* __
   const Team<W> tm;
   if (W == 1 && tm.row >= rows) return;
   const R r(x + tm.row * cols, cols, tm.t);
-  float m = r.has_tail ? r.tail : -INFINITY;
+  float m = -INFINITY;
+#pragma unroll
+  for (int e = 0; e < R::E; ++e)
+    if (r.has_tail(e)) m = fmaxf(m, r.tail[e]);
 #pragma unroll
   for (int k = 0; k < KV; ++k)
     if (r.has(k))
 #pragma unroll
       for (int j = 0; j < N; ++j) m = fmaxf(m, r.at(k, j));
   m = tm.combine(wave_max(m), red[0], [](float a, float b) { return fmaxf(a, b); });
-  float e[KV][N], s = 0.f;
+  float e[KV > 0 ? KV : 1][N], s = 0.f;
 #pragma unroll
   for (int k = 0; k < KV; ++k)
     if (r.has(k))
@@ -655,8 +707,12 @@ __global__ __launch_bounds__(kTeamBlock<W>) void softmax_team_kernel(const T* __
         e[k][j] = __expf(r.at(k, j) - m);
         s += e[k][j];
       }
-  const float et = __expf(r.tail - m);
-  if (r.has_tail) s += et;
+  float et[R::E];
+#pragma unroll
+  for (int k = 0; k < R::E; ++k) {
+    et[k] = __expf(r.tail[k] - m);
+    if (r.has_tail(k)) s += et[k];
+  }
   const float inv = 1.f / tm.combine(wave_sum(s), red[1], [](float a, float b) { return a + b; });
   T* yr = y + tm.row * cols;
 #pragma unroll
@@ -666,7 +722,9 @@ __global__ __launch_bounds__(kTeamBlock<W>) void softmax_team_kernel(const T* __
     for (int j = 0; j < N; ++j) e[k][j] *= inv;
     st_values<T, N>(yr + int64_t(tm.t + k * R::S) * N, e[k]);
   }
-  if (r.has_tail) yr[r.nv * N + tm.t] = narrow<T>(et * inv);
+#pragma unroll
+  for (int k = 0; k < R::E; ++k)
+    if (r.has_tail(k)) yr[r.tail_at(k)] = narrow<T>(et[k] * inv);
 }
 
 // Softmax of rows longer than a 16-wave team holds: max pass, sum-of-exp
@@ -720,14 +778,32 @@ inline int team_waves(int64_t rows, int64_t vecs) {
   return 1;
 }
 template <int W> using Waves = std::integral_constant<int, W>;
-// f(Waves<W>{}) with the team of rows x vecs 16-byte vectors
+template <RowPath P> using Path = std::integral_constant<RowPath, P>;
+// f(Waves<W>{}) with W = waves
 template <class F>
-void with_team(int64_t rows, int64_t vecs, F f) {
-  switch (team_waves(rows, vecs)) {
+void with_waves(int waves, F f) {
+  switch (waves) {
     case 1: f(Waves<1>{}); break;
     case 4: f(Waves<4>{}); break;
     default: f(Waves<16>{}); break;
   }
+}
+// whether rows are read by element (RowPath)
+template <typename T> bool short_row(int64_t cols) { return cols <= (cols % Vec<T>::N == 0 ? 64 : 128); }
+// f(Waves<W>{}, Path<P>{}, whole vectors per row) for the kernels that loop over a
+// row of any length (reduce, argmax).  With 2048 rows or more the chip is full
+// with one wave each, or four where a wave's share is long; fewer rows as
+// team_waves.  argmax of 8192 x 16384 fp32, us with 1 / 4 / 16 waves: 106 / 90 /
+// 114, 65536 x 2052: 92 / 110 / 437; sum of 4096 x 32768 bf16: 46.2 / 39.8 / 38.9.
+template <typename T, class F>
+void with_loop(int64_t rows, int64_t cols, F f) {
+  const int64_t vecs = cols / Vec<T>::N;
+  if (short_row<T>(cols)) return f(Waves<1>{}, Path<kElements>{}, int64_t(0));
+  const int w = rows >= 4096 && vecs <= 1024 ? 1 : rows >= 2048 ? (vecs > 512 ? 4 : 1) : team_waves(rows, vecs);
+  if (w == 1 && vecs <= kWave) f(Waves<1>{}, Path<kOne>{}, vecs);
+  else if (w == 1) f(Waves<1>{}, Path<kLoop>{}, vecs);
+  else if (w == 4) f(Waves<4>{}, Path<kLoop>{}, vecs);
+  else f(Waves<16>{}, Path<kLoop>{}, vecs);
 }
 template <int W> dim3 team_grid(int64_t rows) { return dim3(unsigned((rows + Team<W>::kRows - 1) / Team<W>::kRows)); }
 // f(first row, rows) in runs that a launch takes: HIP refuses grids of 2^32
@@ -740,11 +816,11 @@ void for_row_runs(int64_t rows, F f) {
 
 template <typename T, bool IS_F16, int OP>
 void launch_reduce_op(hipStream_t s, int64_t rows, int64_t cols, const void* x, float init, void* y, int out_type) {
-  with_team(rows, cols / Vec<T>::N, [&](auto w) {
+  with_loop<T>(rows, cols, [&](auto w, auto path, int64_t nv) {
     constexpr int W = decltype(w)::value;
     for_row_runs<W>(rows, [&](int64_t r, int64_t n) {
-      hipLaunchKernelGGL((row_reduce_kernel<T, IS_F16, OP, W>), team_grid<W>(n), dim3(kTeamBlock<W>), 0, s,
-                         reinterpret_cast<const T*>(x) + r * cols, n, cols, init,
+      hipLaunchKernelGGL((row_reduce_kernel<T, IS_F16, OP, W, decltype(path)::value>), team_grid<W>(n), dim3(kTeamBlock<W>), 0, s,
+                         reinterpret_cast<const T*>(x) + r * cols, n, cols, nv, init,
                          static_cast<void*>(static_cast<char*>(y) + r * dtype_bytes(out_type)), out_type);
     });
   });
@@ -765,19 +841,20 @@ int launch_reduce(hipStream_t s, int op, int64_t rows, int64_t cols, const void*
 
 template <typename T, bool IS_F16, bool IS_MIN, typename IdxT>
 int launch_argmax_as(hipStream_t s, int64_t rows, int64_t cols, const void* x, void* values, void* indices) {
-  with_team(rows, cols / Vec<T>::N, [&](auto w) {
+  with_loop<T>(rows, cols, [&](auto w, auto path, int64_t nv) {
     constexpr int W = decltype(w)::value;
+    constexpr RowPath P = decltype(path)::value;
     auto go = [&](auto kernel) {
       for_row_runs<W>(rows, [&](int64_t r, int64_t n) {
         T* v = reinterpret_cast<T*>(values);
         hipLaunchKernelGGL(kernel, team_grid<W>(n), dim3(kTeamBlock<W>), 0, s, reinterpret_cast<const T*>(x) + r * cols,
-                           n, cols, v ? v + r : v, reinterpret_cast<IdxT*>(indices) + r);
+                           n, cols, nv, v ? v + r : v, reinterpret_cast<IdxT*>(indices) + r);
       });
     };
     if constexpr (sizeof(T) == 2) {
-      if (cols <= 65536) return go(row_argmax_kernel<T, IS_F16, IS_MIN, IdxT, true, W>);
+      if (cols <= 65536) return go(row_argmax_kernel<T, IS_F16, IS_MIN, IdxT, true, W, P>);
     }
-    go(row_argmax_kernel<T, IS_F16, IS_MIN, IdxT, false, W>);
+    go(row_argmax_kernel<T, IS_F16, IS_MIN, IdxT, false, W, P>);
   });
   return check_launch("mk_row_argmax");
 }
@@ -813,7 +890,8 @@ void launch_layernorm_any(hipStream_t s, int64_t rows, int64_t cols, const T* x,
     });
   };
   if (vecs > kTeamMaxVecs) return go(Waves<16>{}, layernorm_loop_kernel<T, TO>);
-  with_team(rows, vecs, [&](auto w) {
+  if (short_row<T>(cols)) return go(Waves<1>{}, layernorm_team_kernel<T, TO, 1, 0>);
+  with_waves(team_waves(rows, vecs), [&](auto w) {
     constexpr int W = decltype(w)::value;
     with_share(vecs, W, [&](auto kv) { go(w, layernorm_team_kernel<T, TO, W, decltype(kv)::value>); });
   });
@@ -829,7 +907,8 @@ void launch_softmax(hipStream_t s, int64_t rows, int64_t cols, const T* x, T* y)
     });
   };
   if (vecs > kTeamMaxVecs) return go(Waves<16>{}, softmax_loop_kernel<T>);
-  with_team(rows, vecs, [&](auto w) {
+  if (short_row<T>(cols)) return go(Waves<1>{}, softmax_team_kernel<T, 1, 0>);
+  with_waves(team_waves(rows, vecs), [&](auto w) {
     constexpr int W = decltype(w)::value;
     with_share(vecs, W, [&](auto kv) { go(w, softmax_team_kernel<T, W, decltype(kv)::value>); });
   });

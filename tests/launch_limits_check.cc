@@ -108,6 +108,25 @@ int main() {
                                                                 nullptr, nullptr, 1e-5f, ptr(Y), ptr(Y)), X + 4, rows, row, 3);
       }
 
+  // reduce and argmax: waves per row by rows and length, and no vectors (argument
+  // 3) in short rows
+  struct { int64_t rows, cols; int type; int64_t waves, vectors; } teams[] = {
+      {8192, 16384, MK_F32, 4, 4096}, {65536, 2052, MK_F32, 1, 513},   {4096, 8192, MK_BF16, 1, 1024},
+      {4096, 8200, MK_BF16, 4, 1025}, {4095, 4096, MK_BF16, 1, 512},   {4095, 4104, MK_BF16, 4, 513},
+      {32, 50257, MK_BF16, 16, 6282}, {65536, 64, MK_BF16, 1, 0},      {65536, 100, MK_BF16, 1, 0},
+      {65536, 128, MK_BF16, 1, 16},   {65536, 7, MK_F32, 1, 0},        {65536, 130, MK_F32, 1, 32}};
+  for (const auto& t : teams) {
+    const std::string at = " of " + std::to_string(t.rows) + " x " + std::to_string(t.cols);
+    const uint64_t threads = t.waves == 1 ? (t.rows + 3) / 4 * 256 : uint64_t(t.rows) * 64 * t.waves;
+    for (bool argmax : {false, true}) {
+      limits("row", argmax ? mk_row_argmax(nullptr, t.type, 0, t.rows, t.cols, ptr(X), nullptr, MK_S32, ptr(Y))
+                           : mk_row_reduce(nullptr, t.type, MK_F32, 1, t.rows, t.cols, ptr(X), 0.f, ptr(Y)));
+      expect(g_launches[0].threads == threads, "waves per row" + at);
+      expect(g_launches[0].args[3] == ptr(t.vectors), "vectors" + at);
+      g_launches.clear();
+    }
+  }
+
   // the backward's row statistics: 8 or 16 lanes a row
   g_args = 0;
   for (int64_t D : {64, 128}) {

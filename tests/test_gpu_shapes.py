@@ -77,6 +77,19 @@ def test_row_kernels_any_width(K, rows, cols, off, dtype):
     assert np.all(np.abs(got - want) <= out * np.abs(want) + 1e-5 * scale)
 
 
+# short rows, read by element (up to 64, or 128 that are no whole vectors), and the row counts from
+# which rows take fewer waves
+@pytest.mark.parametrize("rows,cols,off", [(9, 1, 0), (4097, 63, 1), (70, 64, 0), (70, 64, 1), (4100, 65, 0), (9, 127, 1),
+                                           (9, 128, 0), (4096, 4100, 0), (4095, 4100, 1)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_row_kernels_short_and_many(K, rows, cols, off, dtype):
+    test_row_kernels_any_width(K, rows, cols, off, dtype)
+    x = torch.randn(rows, cols, generator=torch.Generator().manual_seed(cols)).to(torch.float16)
+    xd = shifted(x, off)
+    np.testing.assert_array_equal(K.row_reduce(xd, "max").cpu().numpy(), x.float().numpy().max(-1))
+    np.testing.assert_array_equal(K.row_argmax(xd)[0].cpu().numpy(), ops.argmax_rows(x.float().numpy())[0])
+
+
 @pytest.mark.parametrize("rows,cols", [(5, 2052), (3, 4099), (2, 33000)])
 def test_add_layernorm_f32_wide(K, rows, cols):
     """The fp32 residual add inside the LayerNorm of rows the one-wave kernel

@@ -824,7 +824,7 @@ __global__ __launch_bounds__(256, 1) void sdpa_fwd_wide_kernel(const SdpaArgs p)
 using namespace mk;
 
 extern "C" size_t mk_sdpa_fwd_workspace_bytes(int64_t B, int64_t H, int64_t Sq, int64_t Sk, int64_t D, int causal) {
-  if (B <= 0 || H <= 0 || Sq <= 0 || !sdpa_decode_fits(Sq, Sk, causal)) return 0;
+  if (B <= 0 || H <= 0 || Sq <= 0 || !sdpa_decode_fits(B * H, Sq, Sk, D, causal)) return 0;
   return sdpa_decode_workspace(B * H, Sq, Sk, D);
 }
 
@@ -862,7 +862,7 @@ extern "C" int mk_sdpa_fwd_ws(void* stream, int64_t B, int64_t H, int64_t Sq, in
     return fail(MK_ERR_UNSUPPORTED, "mk_sdpa_fwd: q/k/v need 16-byte aligned rows (strides % 8 == 0), o strides % 4 == 0");
   if (k_ss < D || v_ss < D || k_ss >= (int64_t(1) << 24) || v_ss >= (int64_t(1) << 24))
     return fail(MK_ERR_UNSUPPORTED, "mk_sdpa_fwd: k/v sequence strides must be in [D, 2^24)");
-  if (sdpa_decode_fits(Sq, Sk, causal))
+  if (sdpa_decode_fits(B * H, Sq, Sk, D, causal))
     return sdpa_decode(as_stream(stream), B, H, Sq, Sk, D, q, q_bs, q_hs, q_ss, k, k_bs, k_hs, k_ss, v, v_bs, v_hs,
                        v_ss, o, o_bs, o_hs, o_ss, scale, lse, workspace);
   SdpaArgs a;

@@ -37,7 +37,7 @@ using namespace attn;
 
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 
-constexpr int kNW = 4;         // waves per workgroup
+constexpr int kNW = 4;         // waves per workgroup (one per lane group g in the merge)
 constexpr int kMaxQ = 16;      // queries per head
 constexpr int kStepKeys = 32;
 constexpr float kNoMax = -3.0e38f;  // running max before any score
@@ -67,8 +67,10 @@ __global__ __launch_bounds__(64 * kNW, 2) void sdpa_decode_kernel(const DecodeAr
   constexpr int KK = D / 32;      // MFMAs over d per 16 keys
   constexpr int VJ = D / 16;      // d per lane of a V row
   constexpr int kD = D == 128 ? 2 : 3;  // steps in flight
-  __shared__ __attribute__((aligned(16))) float os[kNW][kMaxQ][D];
-  __shared__ float ms[kNW][kMaxQ], ls[kNW][kMaxQ];
+  // rows of O 4 floats past a multiple of the banks: the 16 queries' lanes
+  // write 16 bytes each to different ones
+  __shared__ __attribute__((aligned(16))) float os[kNW][kMaxQ][D + 4];
+  __shared__ float ms[kNW][kMaxQ], ls[kNW][kMaxQ], fs[kNW][kMaxQ], tops[kMaxQ];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int c = lane & 15, g = lane >> 4;
   const int bh = blockIdx.x / p.slices, slice = blockIdx.x % p.slices;
@@ -208,21 +210,29 @@ __global__ __launch_bounds__(64 * kNW, 2) void sdpa_decode_kernel(const DecodeAr
 #pragma unroll
     for (int r = 0; r < 4; ++r)
 #pragma unroll
-      for (int j = 0; j < VJ; ++j) os[wave][c][VJ * (4 * g + r) + j] = acc[j][r];
+      for (int j = 0; j < VJ; j += 4)
+        *reinterpret_cast<f32x4_t*>(&os[wave][c][VJ * (4 * g + r) + j]) =
+            f32x4_t{acc[j][r], acc[j + 1][r], acc[j + 2][r], acc[j + 3][r]};
     if (g == 0) ms[wave][c] = m, ls[wave][c] = l;
+  }
+  __syncthreads();
+  // each wave's weight of each query, once
+  if (wave == 0 && c < p.Sq) {
+    float top = ms[0][c];
+#pragma unroll
+    for (int w = 1; w < kNW; ++w) top = fmaxf(top, ms[w][c]);
+    fs[g][c] = exp2f(ms[g][c] - top);
+    if (g == 0) tops[c] = top;
   }
   __syncthreads();
   for (int e = threadIdx.x; e < p.Sq * D; e += 64 * kNW) {
     const int q = e / D, d = e % D;
-    float top = ms[0][q];
-#pragma unroll
-    for (int w = 1; w < kNW; ++w) top = fmaxf(top, ms[w][q]);
+    const float top = tops[q];
     float o = 0.f, sum = 0.f;
 #pragma unroll
     for (int w = 0; w < kNW; ++w) {
-      const float f = exp2f(ms[w][q] - top);
-      o += f * os[w][q][d];
-      sum += f * ls[w][q];
+      o += fs[w][q] * os[w][q][d];
+      sum += fs[w][q] * ls[w][q];
     }
     if (p.slices == 1) {
       store_out<D>(p, bh, q, d, o, sum, top);
@@ -255,7 +265,13 @@ __global__ __launch_bounds__(D) void sdpa_decode_merge_kernel(const DecodeArgs p
 
 }  // namespace
 
-bool sdpa_decode_fits(int64_t Sq, int64_t Sk, int causal) { return Sq <= kMaxQ && Sk >= 1 && !causal; }
+// The 128-query-tile kernel keeps calls of few heads, one or two key steps and
+// many queries' values to merge over the waves: D 128, 64 heads, 16 queries, 64
+// keys 4.8 us there and 5.5 here (6.4 before the merge's padded rows and its
+// weights computed once); 10 queries 4.9 and 5.0, 16 queries and 128 keys 6.5 and 6.1.
+bool sdpa_decode_fits(int64_t BH, int64_t Sq, int64_t Sk, int64_t D, int causal) {
+  return Sq <= kMaxQ && Sk >= 1 && !causal && !(BH <= 256 && Sk <= 64 && Sq * D > 1280);
+}
 
 int64_t sdpa_decode_slices(int64_t BH, int64_t Sk) {
   // two workgroups of 4 waves per CU (256 CUs), each with at least 256 keys

@@ -100,10 +100,10 @@ int gemm_skinny(hipStream_t s, int ab_type, int c_type, int64_t batch, int64_t M
 int64_t gemm_skinny_slices(int ab_type, int64_t N, int64_t K, int64_t most);
 
 // Attention forward for at most 16 queries without a mask
-// (attention_decode.hip); arguments as mk_sdpa_fwd's, already checked.  With a
+// (attention_decode.hip; sdpa_decode_fits: where it is used); arguments as mk_sdpa_fwd's, already checked.  With a
 // workspace of sdpa_decode_workspace bytes the keys may be cut over
 // workgroups.
-bool sdpa_decode_fits(int64_t Sq, int64_t Sk, int causal);
+bool sdpa_decode_fits(int64_t BH, int64_t Sq, int64_t Sk, int64_t D, int causal);
 size_t sdpa_decode_workspace(int64_t BH, int64_t Sq, int64_t Sk, int64_t D);
 int sdpa_decode(hipStream_t s, int64_t B, int64_t H, int64_t Sq, int64_t Sk, int64_t D,
                 const void* q, int64_t q_bs, int64_t q_hs, int64_t q_ss,

@@ -2,7 +2,7 @@
 // the attention backward against a HIP runtime that only writes down its
 // launches: the largest shapes the entry points take must stay within the
 // 2^32 - 1 threads per grid axis that HIP launches, and products of few rows
-// must run on the kernel that the dispatch rule names.  Nothing is allocated and
+// must run on the kernel that the dispatch rule names (attention of few queries too).  Nothing is allocated and
 // nothing runs on a GPU.  Prints "ok".
 #include <hip/hip_runtime_api.h>
 
@@ -16,6 +16,7 @@
 
 namespace {
 struct Launch {
+  const void* kernel;       // its host stub
   uint64_t threads, grid;   // along x
   std::vector<void*> args;  // the first g_args arguments' first 8 bytes
 };
@@ -64,8 +65,8 @@ hipError_t __hipPushCallConfiguration(dim3 g, dim3 b, size_t, hipStream_t) { ret
 hipError_t __hipPopCallConfiguration(dim3* g, dim3* b, size_t* lds, hipStream_t* s) {
   return *g = g_grid, *b = g_block, *lds = 0, *s = nullptr, hipSuccess;
 }
-hipError_t hipLaunchKernel(const void*, dim3 g, dim3 b, void** args, size_t, hipStream_t) {
-  Launch l{uint64_t(g.x) * b.x, g.x, {}};
+hipError_t hipLaunchKernel(const void* kernel, dim3 g, dim3 b, void** args, size_t, hipStream_t) {
+  Launch l{kernel, uint64_t(g.x) * b.x, g.x, {}};
   expect(g.x > 0 && g.y > 0 && g.z > 0 && g.y < 65536 && g.z < 65536, "an empty or too large grid");
   for (int i = 0; i < g_args; ++i) l.args.push_back(*static_cast<void**>(args[i]));
   return g_launches.push_back(l), hipSuccess;
@@ -170,5 +171,21 @@ int main() {
                " x " + std::to_string(r.N));
     g_launches.clear();
   }
+
+  // few queries, many of them beside few keys: the query-tile kernel of 17 queries
+  auto kernel = [&](int64_t BH, int64_t Sq, int64_t Sk, int64_t D, int causal) {
+    limits("attention", mk_sdpa_fwd(nullptr, 1, BH, Sq, Sk, D, ptr(X), 0, Sq * D, D, ptr(X), 0, Sk * D, D, ptr(X), 0,
+                                    Sk * D, D, ptr(Y), 0, Sq * D, D, 1.f, causal, nullptr));
+    const void* k = g_launches[0].kernel;
+    return g_launches.clear(), k;
+  };
+  g_args = 1;
+  const void *tile = kernel(64, 17, 64, 128, 0), *few = kernel(64, 1, 4096, 128, 0);
+  expect(tile != few && kernel(64, 16, 64, 128, 0) == tile && kernel(256, 11, 1, 128, 0) == tile &&
+             kernel(64, 10, 64, 128, 0) == few && kernel(64, 16, 65, 128, 0) == few &&
+             kernel(257, 16, 64, 128, 0) == few && kernel(64, 16, 64, 64, 0) == kernel(64, 1, 4096, 64, 0) &&
+             kernel(64, 1, 64, 128, 1) != few,
+         "the kernel of few queries");
+  expect(mk_sdpa_fwd_workspace_bytes(1, 64, 16, 64, 128, 0) == 0, "no workspace for the query-tile kernel");
   std::printf("ok\n");
 }

@@ -154,7 +154,9 @@ def test_gemm_few_rows_batched_and_split(K):
 # few queries: key counts around the 32-key steps, the 4 waves' shares and the 256-key slices
 @pytest.mark.parametrize("B,H,Sq,Sk,D", [(1, 1, 1, 1, 128), (2, 3, 1, 31, 64), (1, 2, 7, 33, 128), (1, 2, 16, 129, 64),
                                          (2, 2, 1, 511, 128), (1, 2, 2, 513, 128), (1, 3, 16, 2049, 128),
-                                         (3, 5, 4, 1000, 64), (1, 1, 1, 16391, 128), (32, 16, 1, 300, 64)])
+                                         (3, 5, 4, 1000, 64), (1, 1, 1, 16391, 128), (32, 16, 1, 300, 64),
+                                         (1, 2, 10, 64, 128), (2, 3, 11, 33, 128), (1, 2, 16, 64, 128),
+                                         (1, 2, 16, 65, 128), (32, 16, 16, 64, 128), (16, 16, 12, 1, 128)])
 @pytest.mark.parametrize("slices", [True, False])
 def test_sdpa_few_queries(K, B, H, Sq, Sk, D, slices):
     """O and lse against float64 softmax; the cache holds NaN past its keys.

@@ -767,20 +767,22 @@ int gemm_tiled(hipStream_t s, int c_type, int64_t batch, int64_t M, int64_t N, i
   // per CU; e is the first loads and the epilogue in k tiles, for 16-bit C
   // and for fp32 C (whose stores cost about the same per element in every
   // shape).  A CU holds one 256 x 256 workgroup or two of the smaller ones; a
-  // last partial round with every workgroup alone on its CU runs each at
-  // 0.73 of the pair's rate, and one on fewer than half of the CUs takes 0.63
-  // of a full round of 256 x 256 tiles.  The constants are fitted to the three
-  // shapes' times on 58 products, 256 .. 50257 rows and columns, 64 .. 8192
-  // deep, both C types, unsplit and split: the choice is within 1% of the
-  // fastest on each (8192 x 50257 x 768, bf16 C: 694 / 657 / 717 us in the
-  // order below; 2300 x 640 x 40000 in 8 slices: 168 / 197 / 200; 40000 x 640
-  // x 2300, fp32 C: 128 / 144 / 146; 1024 x 8192 x 2048: 47 / 41 / 35).
+  // last partial round of those with every workgroup alone on its CU runs
+  // each at 0.64 of the pair's rate.  A partial round of 256 x 256 tiles takes
+  // a full one's time, however few they are.  The constants are fitted to the
+  // three shapes' times on 860 drawn products and the training step's
+  // (profiles/gemm_tile_shapes.txt; 250 .. 50257 rows and columns, 64 .. 8192
+  // deep, both C types, unsplit, split and batched).  The choice costs 0.3% on
+  // average over always taking the fastest, 11% at the worst but for two
+  // products.  In the order below, us: 8192 x 50257 x 768, bf16 C 774 / 618 /
+  // 741; 3245 x 2112 x 1344, fp32 C 42 / 35 / 29; 8192 x 8192 x 4096 451 /
+  // 487 / 519; 8192 x 6144 x 2048 181 / 187 / 201.
   struct Option {
     int tm, tn, per_cu;
     double rate, e16, e32;
   };
   static const Option options[3] = {
-      {256, 256, 1, 1330.0, 4.5, 12.2}, {128, 192, 2, 1250.0, 1.1, 10.3}, {128, 128, 2, 1030.0, 0.7, 11.4}};
+      {256, 256, 1, 1240.0, 3.8, 8.1}, {128, 192, 2, 1110.0, 0.7, 6.9}, {128, 128, 2, 900.0, 0.8, 5.4}};
   const int64_t cus = cu_count();
   const double nk = double((K + 63) / 64);
   int best = -1;
@@ -792,10 +794,7 @@ int gemm_tiled(hipStream_t s, int c_type, int64_t batch, int64_t M, int64_t N, i
     const int64_t slots = cus * op.per_cu, rem = tiles % slots;
     const double tile = double(op.tm) * op.tn / op.rate * (nk + (c_type == MK_F32 ? op.e32 : op.e16));
     double t = double(tiles / slots) * op.per_cu * tile;
-    if (rem > 0) {
-      if (op.per_cu > 1) t += rem <= cus ? tile / 0.73 : op.per_cu * tile;
-      else t += 2 * rem < cus ? 0.63 * tile : tile;
-    }
+    if (rem > 0) t += op.per_cu > 1 && rem <= cus ? tile / 0.64 : op.per_cu * tile;
     if (best < 0 || t < best_t) best = o, best_t = t;
   }
   if (best == 0) return launch<Shape<256, 256, 2, 4, 64, 2>>(s, a, batch, a_kc, b_kc);

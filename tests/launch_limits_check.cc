@@ -79,11 +79,6 @@ int sdpa_bwd_flash(hipStream_t, int64_t B, int64_t H, int64_t Sq, int64_t Sk, in
                    int64_t, int64_t, int64_t, const void*, int64_t, int64_t, int64_t, const float*, void*, int64_t,
                    int64_t, int64_t, void*, int64_t, int64_t, int64_t, void*, int64_t, int64_t, int64_t, float, int,
                    void*);
-// takes at least 128 rows
-int gemm_tiled(hipStream_t, int, int64_t, int64_t, int64_t, int64_t, const void*, int64_t, int64_t, int64_t, const void*,
-               int64_t, int64_t, int64_t, void*, int64_t, int64_t, const void*, int, int64_t, void*, int64_t, float*) {
-  return -1;
-}
 void clear_error() {}
 int fail(int code, const std::string& what) { return std::printf("%s\n", what.c_str()), code; }
 int check_launch(const char*) { return MK_OK; }
@@ -169,6 +164,19 @@ int main() {
     expect((g_launches[0].grid == tiles && g_launches[0].threads == tiles * block) == r.tiles,
            "the kernel of " + std::to_string(r.batch) + " x " + std::to_string(r.M) + " x " + std::to_string(r.K) +
                " x " + std::to_string(r.N));
+    g_launches.clear();
+  }
+
+  // tile shapes of large products: the grid's tiles name them
+  struct { int64_t M, N, K; int c_type; int64_t tm, tn; } tiles[] = {
+      {8192, 8192, 4096, MK_BF16, 256, 256}, {8192, 50264, 768, MK_BF16, 128, 192}, {3248, 2112, 1344, MK_F32, 128, 128},
+      {15336, 416, 1408, MK_F32, 128, 128},  {8192, 6144, 2048, MK_BF16, 256, 256}, {8192, 768, 3072, MK_BF16, 128, 192},
+      {1024, 8192, 2048, MK_BF16, 128, 128}, {4096, 4096, 4096, MK_BF16, 256, 256}};
+  for (const auto& t : tiles) {
+    limits("tiled", mk_gemm(nullptr, MK_BF16, t.c_type, 1, t.M, t.N, t.K, ptr(X), 0, t.K, 1, ptr(X), 0, t.N, 1, ptr(Y), 0,
+                            t.N, nullptr, 0));
+    expect(g_launches[0].grid == uint64_t((t.M + t.tm - 1) / t.tm * ((t.N + t.tn - 1) / t.tn)),
+           "the tile shape of " + std::to_string(t.M) + " x " + std::to_string(t.N) + " x " + std::to_string(t.K));
     g_launches.clear();
   }
 

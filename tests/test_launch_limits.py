@@ -18,7 +18,7 @@ HIPCC = os.path.join(ROCM, "bin", "hipcc")
 def test_launches_stay_within_the_grid(tmp_path):
     inc, kdir = os.path.join(ROOT, "include"), os.path.join(ROOT, "mccl-jax_amd", "src", "kernels")
     objs, exe = [], str(tmp_path / "check")
-    for src in ("reduce", "attention_bwd", "gemm", "gemm_skinny", "attention", "attention_decode"):
+    for src in ("reduce", "attention_bwd", "gemm", "gemm_skinny", "gemm_tiled", "attention", "attention_decode"):
         objs.append(str(tmp_path / (src + ".o")))
         subprocess.run([HIPCC, "--offload-arch=gfx950", "--cuda-host-only", "-std=c++17", "-fPIC", "-I" + inc,
                         "-I" + kdir, "-c", os.path.join(kdir, src + ".hip"), "-o", objs[-1]], check=True, timeout=300)

@@ -132,6 +132,11 @@ int mk_gemm_splitk_typed(void* stream, int ab_type, int c_type, int64_t M, int64
                          int64_t a_ms, int64_t a_ks, const void* B, int64_t b_ks, int64_t b_ns, void* C,
                          int64_t c_ms, int64_t splits, void* workspace, const void* bias, int epilogue);
 
+/* Workspace of a product of few rows that gains from a cut along K; 0: it does
+ * not, call mk_gemm.  With it: mk_gemm_splitk_typed, splits 16. */
+size_t mk_gemm_few_rows_workspace_bytes(int ab_type, int64_t M, int64_t N, int64_t K, int64_t a_ks, int64_t b_ks,
+                                        int64_t b_ns);
+
 /* Plain GEMM through rocBLAS (the linear layers of the training step and
  * their gradients: with no epilogue to fuse, a library GEMM does the work).  Same operand convention as
  * mk_gemm (row-major C with row stride c_ms, one unit stride per operand),

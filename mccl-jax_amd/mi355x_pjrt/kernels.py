@@ -60,6 +60,16 @@ def _ptr(t):
     return None if t is None else t.data_ptr()
 
 
+def _scratch(nbytes, device, stream):
+    """A call's workspace on `stream` (None: the current one), from that
+    stream's memory: freed when the call returns, it goes to later work of the
+    same stream only."""
+    if stream is None:
+        return torch.empty(nbytes, dtype=torch.uint8, device=device)
+    with torch.cuda.stream(stream):
+        return torch.empty(nbytes, dtype=torch.uint8, device=device)
+
+
 def _check(rc, what):
     _lib.check(rc, what)
 
@@ -85,9 +95,9 @@ def sdpa_fwd(q, k, v, scale: float, causal: bool = True, out=None, lse=None, str
         out = torch.empty((B, H, Sq, D), dtype=torch.bfloat16, device=q.device)
     os = out.stride()
     ws = None
-    if Sq <= 16 and Sk >= 512 and not causal and stream is None:  # few queries: the keys may be cut over workgroups
+    if Sq <= 16 and Sk >= 512 and not causal:  # few queries: the keys may be cut over workgroups
         nbytes = lib().mk_sdpa_fwd_workspace_bytes(B, H, Sq, Sk, D, 0)
-        ws = torch.empty(nbytes, dtype=torch.uint8, device=q.device) if nbytes else None
+        ws = _scratch(nbytes, q.device, stream) if nbytes else None
     rc = lib().mk_sdpa_fwd_ws(
         _stream(stream), B, H, Sq, Sk, D, q.data_ptr(), qs[0], qs[1], qs[2], k.data_ptr(), ks[0], ks[1], ks[2],
         v.data_ptr(), vs[0], vs[1], vs[2], out.data_ptr(), os[0], os[1], os[2],
@@ -97,17 +107,6 @@ def sdpa_fwd(q, k, v, scale: float, causal: bool = True, out=None, lse=None, str
 
 
 # ------------------------------------------------------------------ a4 GEMM
-def _few_row_slices(M, N, K, esz, sa, so, out):
-    """Slices of the contraction for a product of few rows and too few
-    columns to fill the chip's 256 CUs with 64-column workgroups (1: none).
-    16 x 16384 x 4096 bf16 (M x K x N): 72 us in one launch, 32 in 4 slices and
-    their sum; below 4096 bf16 deep the second launch costs what it saves."""
-    if M > 64 or K * esz < 8192 or N < 16 or N % 4 or sa[1] != 1 or so[0] % 4 or out.data_ptr() % 16:
-        return 1
-    tiles = (N + 63) // 64
-    return 1 if tiles >= 192 else min(16, 256 // tiles, K // 512)
-
-
 def _gemm2(a, b, out_dtype, bias, relu, out, stream):
     """gemm of 2-D views."""
     M, K = a.shape
@@ -120,12 +119,13 @@ def _gemm2(a, b, out_dtype, bias, relu, out, stream):
     if bias is not None and bias.dtype == torch.float32 and out_dtype != torch.float32:
         epi |= 4  # an fp32 bias added before the narrowing store
     ab, ct, sa, sb, so = mk_dtype(a.dtype), mk_dtype(out_dtype), a.stride(), b.stride(), out.stride()
-    if stream is None and out_dtype != torch.float16:
-        slices = _few_row_slices(M, N, K, a.element_size(), sa, so, out)
-        if slices > 1:
-            ws = torch.empty(slices * M * N, dtype=torch.float32, device=a.device)
-            rc = lib().mk_gemm_splitk_typed(_stream(), ab, ct, M, N, K, a.data_ptr(), sa[0], sa[1], b.data_ptr(), sb[0],
-                                            sb[1], out.data_ptr(), so[0], slices, ws.data_ptr(), _ptr(bias), epi)
+    # few rows and columns: the contraction may be cut over workgroups
+    if 0 < M <= 64 and K >= 1024 and so[0] % 4 == 0 and out.data_ptr() % 16 == 0 and out_dtype != torch.float16:
+        nbytes = lib().mk_gemm_few_rows_workspace_bytes(ab, M, N, K, sa[1], sb[0], sb[1])
+        if nbytes:
+            ws = _scratch(nbytes, a.device, stream)
+            rc = lib().mk_gemm_splitk_typed(_stream(stream), ab, ct, M, N, K, a.data_ptr(), sa[0], sa[1], b.data_ptr(),
+                                            sb[0], sb[1], out.data_ptr(), so[0], 16, ws.data_ptr(), _ptr(bias), epi)
             _check(rc, "mk_gemm_splitk_typed")
             return out
     rc = lib().mk_gemm(_stream(stream), ab, ct, 1, M, N, K, a.data_ptr(), 0, sa[0], sa[1], b.data_ptr(), 0, sb[0],
@@ -142,6 +142,11 @@ def gemm(a, b, out_dtype=None, bias=None, relu=False, out=None, stream=None):
         raise ValueError("gemm: operand dtypes differ")
     if a.dim() == 2 and b.dim() == 2 and (out is None or out.dim() == 2):
         return _gemm2(a, b, out_dtype or a.dtype, bias, relu, out, stream)
+    if a.dim() == 3 and a.shape[0] == 1:  # a batch of one
+        out = torch.empty(1, a.shape[1], b.shape[-1], dtype=out_dtype or a.dtype, device=a.device) if out is None else out
+        _gemm2(a[0], b[0] if b.dim() == 3 else b, out_dtype or a.dtype, bias, relu, out[0] if out.dim() == 3 else out,
+               stream)
+        return out
     squeeze = a.dim() == 2
     a3 = a.unsqueeze(0) if squeeze else a
     b3 = b.unsqueeze(0) if b.dim() == 2 else b
@@ -349,7 +354,7 @@ def scatter_add_rows(table, ids, updates, out=None, workspace=None, stream=None)
         out = torch.empty_like(table)
     nbytes = lib().mk_scatter_add_workspace_bytes(n_rows, ids_c.numel())
     if workspace is None:
-        workspace = torch.empty(max(int(nbytes), 1), dtype=torch.uint8, device=table.device)
+        workspace = _scratch(max(int(nbytes), 1), table.device, stream)
     elif workspace.numel() < nbytes:
         raise ValueError("scatter_add_rows: workspace too small")
     rc = lib().mk_scatter_add_rows(_stream(stream), mk_dtype(table.dtype), n_rows, row_len,
@@ -376,9 +381,9 @@ def scatter_add_rows_noalloc(table, ids, updates, out=None, stream=None):
 
 
 # ------------------------------------------------------------------ C5 training step
-def _ws(nbytes, device, workspace):
+def _ws(nbytes, device, workspace, stream=None):
     if workspace is None:
-        return torch.empty(max(int(nbytes), 1), dtype=torch.uint8, device=device)
+        return _scratch(max(int(nbytes), 1), device, stream)
     if workspace.numel() * workspace.element_size() < nbytes:
         raise ValueError("workspace too small")
     return workspace
@@ -436,7 +441,7 @@ def gemm_gelu_bwd(a, b, pre, out=None, workspace=None, stream=None):
     N = b.shape[1]
     out = torch.empty(M, N, dtype=torch.bfloat16, device=a.device) if out is None else out
     colsum = torch.empty(N, dtype=torch.float32, device=a.device)
-    ws = _ws(lib().mk_gemm_gelu_bwd_workspace_bytes(M, N), a.device, workspace)
+    ws = _ws(lib().mk_gemm_gelu_bwd_workspace_bytes(M, N), a.device, workspace, stream)
     rc = lib().mk_gemm_gelu_bwd(_stream(stream), mk_dtype(a.dtype), M, N, Kd, _ptr(a), a.stride(0), a.stride(1),
                                 _ptr(b), b.stride(0), b.stride(1), _ptr(out), out.stride(0), _ptr(pre), pre.stride(0),
                                 _ptr(colsum), _ptr(ws))
@@ -454,7 +459,7 @@ def gemm_splitk(a, b, splits, out=None, workspace=None, stream=None, out_dtype=t
     M, Kd = a.shape
     N = b.shape[1]
     out = torch.empty(M, N, dtype=out_dtype, device=a.device) if out is None else out
-    ws = _ws(lib().mk_gemm_splitk_workspace_bytes(M, N, splits), a.device, workspace)
+    ws = _ws(lib().mk_gemm_splitk_workspace_bytes(M, N, splits), a.device, workspace, stream)
     if out.dtype == torch.float32 and Kd % splits == 0 and bias is None:
         rc = lib().mk_gemm_splitk(_stream(stream), mk_dtype(a.dtype), M, N, Kd, _ptr(a), a.stride(0), a.stride(1),
                                   _ptr(b), b.stride(0), b.stride(1), _ptr(out), out.stride(0), splits, _ptr(ws))
@@ -476,7 +481,7 @@ def gemm_blas_splitk(a, b, splits, out=None, workspace=None, stream=None):
     M, Kd = a.shape
     N = b.shape[1]
     out = torch.empty(M, N, dtype=torch.float32, device=a.device) if out is None else out
-    ws = _ws(lib().mk_gemm_blas_splitk_workspace_bytes(M, N, splits), a.device, workspace)
+    ws = _ws(lib().mk_gemm_blas_splitk_workspace_bytes(M, N, splits), a.device, workspace, stream)
     rc = lib().mk_gemm_blas_splitk(_stream(stream), mk_dtype(a.dtype), M, N, Kd, _ptr(a), a.stride(0), a.stride(1),
                                    _ptr(b), b.stride(0), b.stride(1), _ptr(out), out.stride(0), splits, _ptr(ws))
     _check(rc, "mk_gemm_blas_splitk")
@@ -543,7 +548,7 @@ def col_sum(x, out=None, workspace=None, stream=None):
     _require_cuda(x)
     rows, cols = x.shape
     out = torch.empty(cols, dtype=torch.float32, device=x.device) if out is None else out
-    ws = _ws(lib().mk_col_sum_workspace_bytes(rows, cols), x.device, workspace)
+    ws = _ws(lib().mk_col_sum_workspace_bytes(rows, cols), x.device, workspace, stream)
     rc = lib().mk_col_sum(_stream(stream), mk_dtype(x.dtype), rows, cols, _ptr(x), _ptr(out), _ptr(ws))
     _check(rc, "mk_col_sum")
     return out
@@ -562,7 +567,7 @@ def layernorm_bwd(x, gamma, dy, eps=1e-5, dx=None, dgamma=None, dbeta=None, work
         dgamma = torch.empty(cols, dtype=torch.float32, device=x.device) if dgamma is None else dgamma
         dbeta = torch.empty(cols, dtype=torch.float32, device=x.device) if dbeta is None else dbeta
     colsum = torch.empty(cols, dtype=torch.float32, device=x.device) if want_colsum else None
-    ws = _ws(lib().mk_layernorm_bwd_workspace_bytes(rows, cols), x.device, workspace)
+    ws = _ws(lib().mk_layernorm_bwd_workspace_bytes(rows, cols), x.device, workspace, stream)
     rc = lib().mk_layernorm_bwd_typed(_stream(stream), mk_dtype(x.dtype), rows, cols, _ptr(x), _ptr(gamma),
                                       _ptr(dy), _ptr(dres), float(eps), _ptr(dx), _ptr(dx_bf16),
                                       _ptr(dgamma if want_params else None), _ptr(dbeta if want_params else None),
@@ -577,7 +582,7 @@ def gelu_tanh_bwd_colsum(x, dy, out=None, workspace=None, stream=None):
     rows, cols = x.shape
     out = torch.empty_like(x) if out is None else out
     colsum = torch.empty(cols, dtype=torch.float32, device=x.device)
-    ws = _ws(lib().mk_col_sum_workspace_bytes(rows, cols), x.device, workspace)
+    ws = _ws(lib().mk_col_sum_workspace_bytes(rows, cols), x.device, workspace, stream)
     rc = lib().mk_gelu_tanh_bwd_colsum(_stream(stream), mk_dtype(x.dtype), rows, cols, _ptr(x), _ptr(dy), _ptr(out),
                                        _ptr(colsum), _ptr(ws))
     _check(rc, "mk_gelu_tanh_bwd_colsum")
@@ -634,7 +639,7 @@ def sdpa_bwd(q, k, v, o, dout, lse, scale, causal=True, dq=None, dk=None, dv=Non
     dq = torch.empty_like(q) if dq is None else dq
     dk = torch.empty_like(k) if dk is None else dk
     dv = torch.empty_like(v) if dv is None else dv
-    ws = _ws(lib().mk_sdpa_bwd_workspace_bytes(B, H, Sq, Sk, D), q.device, workspace)
+    ws = _ws(lib().mk_sdpa_bwd_workspace_bytes(B, H, Sq, Sk, D), q.device, workspace, stream)
     args = [_stream(stream), B, H, Sq, Sk, D]
     for t in (q, k, v, o, dout):
         args += [_ptr(t), *t.stride()[:3]]

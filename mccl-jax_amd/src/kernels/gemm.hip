@@ -433,6 +433,14 @@ extern "C" size_t mk_gemm_splitk_workspace_bytes(int64_t M, int64_t N, int64_t s
   return size_t(M * N * splits * 4);
 }
 
+extern "C" size_t mk_gemm_few_rows_workspace_bytes(int ab_type, int64_t M, int64_t N, int64_t K, int64_t a_ks,
+                                                   int64_t b_ks, int64_t b_ns) {
+  if (M <= 0 || N % 4 != 0 || (ab_type != MK_BF16 && ab_type != MK_F32) || !gemm_skinny_fits(M, N, K, a_ks, b_ks, b_ns))
+    return 0;
+  const int64_t slices = gemm_skinny_slices(ab_type, M, N, K, b_ks == 1, 16);
+  return slices == 1 ? 0 : size_t(slices * M * N * 4);
+}
+
 extern "C" int mk_gemm_splitk_typed(void* stream, int ab_type, int c_type, int64_t M, int64_t N, int64_t K,
                                     const void* A, int64_t a_ms, int64_t a_ks, const void* B, int64_t b_ks,
                                     int64_t b_ns, void* C, int64_t c_ms, int64_t splits, void* workspace,
@@ -453,7 +461,7 @@ extern "C" int mk_gemm_splitk_typed(void* stream, int ab_type, int c_type, int64
   // few rows: the kernel that takes them splits k inside the workgroup, and
   // over workgroups only where the columns alone leave the chip idle
   if (gemm_skinny_fits(M, N, K, a_ks, b_ks, b_ns)) {
-    const int64_t slices = gemm_skinny_slices(ab_type, N, K, splits);
+    const int64_t slices = gemm_skinny_slices(ab_type, M, N, K, b_ks == 1, splits);
     if (slices == 1 || !A || !B)
       return mk_gemm(stream, ab_type, c_type, 1, M, N, K, A, 0, a_ms, a_ks, B, 0, b_ks, b_ns, C, 0, c_ms, bias,
                      epilogue);

@@ -295,12 +295,19 @@ bool gemm_skinny_pays(int ab_type, int64_t batch, int64_t M, int64_t N, int64_t 
   return K >= (b_kc ? (half ? 128 : 2048) : (half ? 64 : 256)) * mt;
 }
 
-int64_t gemm_skinny_slices(int ab_type, int64_t N, int64_t K, int64_t most) {
-  // a workgroup's time is its lines at 8 clocks each, one 128-byte line per
-  // k-row of bf16, two of fp32: below 2048 lines (about 7 us) it costs no
-  // more than the slices' second pass of about 4 us saves
+int64_t gemm_skinny_slices(int ab_type, int64_t M, int64_t N, int64_t K, bool b_kc, int64_t most) {
+  // A workgroup's time is its lines at 8 clocks each, one 128-byte line per
+  // k-row of bf16, two of fp32; the slices' second pass costs about 4 us.  Timed
+  // on 1000 products, in one launch and in slices: slices gain from 2048 lines
+  // on (16 x 2048 x 768 bf16: 9.0 -> 7.1 us, 16 x 16384 x 4096: 47.9 -> 26.3), but
+  // not where only two find CUs, unless a workgroup's rows are many (n-contiguous
+  // 16 x 2048 x 6000: 10.8 -> 12.1), and with at most 16 rows of k-contiguous B only
+  // from 4096 lines below 2560 columns: its 16-column workgroups fill the chip
+  // alone (1 x 4096 x 4096: 8.6 -> 10.5).
   const int64_t tiles = (N + 63) / 64, lines = ab_type == MK_BF16 ? K : 2 * K;
-  if (tiles >= 192 || lines < 2048) return 1;
+  const bool few = M <= 16;
+  if (tiles >= (b_kc ? (few ? 40 : 192) : (ab_type == MK_BF16 && !few ? 192 : 86))) return 1;
+  if (lines < (b_kc && few ? 4096 : 2048)) return 1;
   return std::max<int64_t>(1, std::min({most, 256 / tiles, K / 512, int64_t(16)}));
 }
 

@@ -97,7 +97,7 @@ int gemm_skinny(hipStream_t s, int ab_type, int c_type, int64_t batch, int64_t M
                 const void* A, int64_t a_bs, int64_t a_ms, int64_t a_ks, const void* B, int64_t b_bs, int64_t b_ks,
                 int64_t b_ns, void* C, int64_t c_bs, int64_t c_ms, const void* bias, int epilogue,
                 int64_t slices = 1);
-int64_t gemm_skinny_slices(int ab_type, int64_t N, int64_t K, int64_t most);
+int64_t gemm_skinny_slices(int ab_type, int64_t M, int64_t N, int64_t K, bool b_kc, int64_t most);
 
 // Attention forward for at most 16 queries without a mask
 // (attention_decode.hip; sdpa_decode_fits: where it is used); arguments as mk_sdpa_fwd's, already checked.  With a

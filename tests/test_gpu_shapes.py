@@ -172,15 +172,42 @@ def test_sdpa_few_queries(K, B, H, Sq, Sk, D, slices):
     vd.copy_(v)
     out = torch.full((B, H, Sq, D), float("nan"), dtype=torch.bfloat16, device="cuda")
     lse = torch.full((B, H, Sq), float("nan"), device="cuda")
-    # an explicit stream runs without a workspace: one workgroup per head
-    K.sdpa_fwd(q.cuda(), kd, vd, D ** -0.5, causal=False, out=out, lse=lse,
-               stream=None if slices else torch.cuda.current_stream())
+    if slices:
+        K.sdpa_fwd(q.cuda(), kd, vd, D ** -0.5, causal=False, out=out, lse=lse)
+    else:  # the entry without a workspace: one workgroup per head
+        qd = q.cuda()
+        strides = [[t.data_ptr(), *t.stride()[:3]] for t in (qd, kd, vd, out)]
+        assert K.lib().mk_sdpa_fwd(K._stream(), B, H, Sq, Sk, D, *sum(strides, []), D ** -0.5, 0, lse.data_ptr()) == 0
     s = (q.double() @ k.double().transpose(-1, -2)) * D ** -0.5
     p = torch.softmax(s, -1)
     want, u = p @ v.double(), 2.0 ** -8
     bound = 2 * u * (p @ v.double().abs()) + u * want.abs() + 1e-6
     assert bool(((out.cpu().double() - want).abs() <= bound).all())
     assert bool(((lse.cpu().double() - torch.logsumexp(s, -1)).abs() <= u + 1e-5).all())
+
+
+def test_few_rows_and_queries_on_an_explicit_stream(K):
+    """The cuts along the contraction and the keys don't depend on how the
+    stream is named or on a batch dimension of one: the same bits.  The
+    workspace is the stream's own memory."""
+    g = torch.Generator().manual_seed(8)
+    x, w = torch.randn(16, 8192, generator=g).bfloat16().cuda(), torch.randn(8192, 512, generator=g).bfloat16().cuda()
+    assert K.lib().mk_gemm_few_rows_workspace_bytes(K.mk_dtype(x.dtype), 16, 512, 8192, 1, 512, 1) > 0
+    q, k, v = (torch.randn(1, 4, s, 128, generator=g).bfloat16().cuda() for s in (2, 8192, 8192))
+    assert K.lib().mk_sdpa_fwd_workspace_bytes(1, 4, 2, 8192, 128, 0) > 0
+    y, o = K.gemm(x, w), K.sdpa_fwd(q, k, v, 0.1, causal=False)
+    torch.cuda.synchronize()
+    s = torch.cuda.Stream()
+    for stream in (torch.cuda.current_stream(), s):
+        ys = K.gemm(x, w, stream=stream)
+        os = K.sdpa_fwd(q, k, v, 0.1, causal=False, stream=stream)
+        stream.synchronize()
+        assert torch.equal(ys, y) and torch.equal(os, o)
+    assert torch.equal(K.gemm(x[None], w), y[None]) and torch.equal(K.gemm(x[None], w[None]), y[None])
+    held = K._scratch(1 << 22, x.device, s).data_ptr()  # freed at once: the current stream must not get it
+    blocks = [torch.empty(1 << 22, dtype=torch.uint8, device="cuda") for _ in range(4)]
+    assert all(b.data_ptr() != held for b in blocks)
+    assert K._scratch(1 << 22, x.device, s).data_ptr() == held
 
 
 def test_sdpa_few_queries_infinities(K):

@@ -40,7 +40,6 @@ typedef float f32x4_t __attribute__((ext_vector_type(4)));
 constexpr int kNW = 4;         // waves per workgroup (one per lane group g in the merge)
 constexpr int kMaxQ = 16;      // queries per head
 constexpr int kStepKeys = 32;
-constexpr float kNoMax = -3.0e38f;  // running max before any score
 
 struct DecodeArgs {
   const uint16_t *q, *k, *v;
@@ -51,6 +50,9 @@ struct DecodeArgs {
   int H, Sq, Sk, slices, slice_keys;
   float scale_log2;
 };
+
+// what sums taken at max m are worth at max top (>= m); no score above -inf: 0
+__device__ inline float weight(float m, float top) { return m == -INFINITY ? 0.f : exp2f(m - top); }
 
 // one query's D outputs from weighted partial rows: out(i) = sum_w wt_w O_w[i]
 // / l, thread-strided; shared by the in-workgroup and the slice merge
@@ -113,7 +115,7 @@ __global__ __launch_bounds__(64 * kNW, 2) void sdpa_decode_kernel(const DecodeAr
     }
   };
   f32x4_t acc[VJ] = {};
-  float m = kNoMax, l = 0.f;
+  float m = -INFINITY, l = 0.f;  // the max is -inf until a score above it is seen
   auto use = [&](Step& s, int key0) __attribute__((always_inline)) {
     float x[8];
 #pragma unroll
@@ -141,7 +143,7 @@ __global__ __launch_bounds__(64 * kNW, 2) void sdpa_decode_kernel(const DecodeAr
       float nm = fmaxf(m, top);
       nm = fmaxf(nm, __shfl_xor(nm, 16, 64));
       nm = fmaxf(nm, __shfl_xor(nm, 32, 64));
-      const float f = exp2f(m - nm);
+      const float f = weight(m, nm);
       m = nm;
       l *= f;
 #pragma unroll
@@ -149,9 +151,10 @@ __global__ __launch_bounds__(64 * kNW, 2) void sdpa_decode_kernel(const DecodeAr
 #pragma unroll
         for (int r = 0; r < 4; ++r) acc[j][r] *= f;
     }
+    const float base = m == -INFINITY ? 0.f : m;
     float e[8];
 #pragma unroll
-    for (int u = 0; u < 8; ++u) e[u] = __builtin_amdgcn_exp2f(x[u] - m);
+    for (int u = 0; u < 8; ++u) e[u] = __builtin_amdgcn_exp2f(x[u] - base);
     const bf16x8_t pr = pack8(e[0], e[1], e[2], e[3], e[4], e[5], e[6], e[7]);
     const u32x4_t pw = __builtin_bit_cast(u32x4_t, pr);
 #pragma unroll
@@ -221,7 +224,7 @@ __global__ __launch_bounds__(64 * kNW, 2) void sdpa_decode_kernel(const DecodeAr
     float top = ms[0][c];
 #pragma unroll
     for (int w = 1; w < kNW; ++w) top = fmaxf(top, ms[w][c]);
-    fs[g][c] = exp2f(ms[g][c] - top);
+    fs[g][c] = weight(ms[g][c], top);
     if (g == 0) tops[c] = top;
   }
   __syncthreads();
@@ -256,7 +259,7 @@ __global__ __launch_bounds__(D) void sdpa_decode_merge_kernel(const DecodeArgs p
   float o = 0.f, sum = 0.f;
 #pragma unroll 4
   for (int s = 0; s < p.slices; ++s) {
-    const float f = exp2f(rows[s * pitch + D] - top);
+    const float f = weight(rows[s * pitch + D], top);
     o += f * rows[s * pitch + d];
     sum += f * rows[s * pitch + D + 1];
   }

@@ -220,6 +220,18 @@ def test_sdpa_few_queries_infinities(K):
     k[0, 1, 699, 3] = float("nan")
     o = K.sdpa_fwd(q, k, v, 0.125, causal=False)
     assert bool((o[0, 0] == 2).all()) and bool(o[0, 1].isnan().all()) and bool((o[0, 2] == 2).all())
+    # a head without a score above -inf has no weights, a query of scores at the type's lowest value has
+    k[0, 0] = -float("inf")
+    k[0, 1] = 0
+    k[0, 1, :, 0] = torch.finfo(torch.bfloat16).min
+    q[0, 1] = 0
+    q[0, 1, 0, 0] = 1
+    lse = torch.empty(1, 3, 2, device="cuda")
+    for scale in (0.69, 0.125):  # 0.69 log2(e) leaves the scores finite
+        for n in (700, 40):
+            o = K.sdpa_fwd(q, k[:, :, :n], v[:, :, :n], scale, causal=False, lse=lse)
+            assert bool(o[0, 0].isnan().all()) and bool((lse[0, 0] == -float("inf")).all())
+            assert bool((o[0, 1] == 2).all()) and bool(lse[0, 1].isfinite().all()) and bool((o[0, 2] == 2).all())
 
 
 def test_gpt2_steps_on_several_streams(cuda):

@@ -95,7 +95,7 @@ def sdpa_fwd(q, k, v, scale: float, causal: bool = True, out=None, lse=None, str
         out = torch.empty((B, H, Sq, D), dtype=torch.bfloat16, device=q.device)
     os = out.stride()
     ws = None
-    if Sq <= 16 and Sk >= 512 and not causal:  # few queries: the keys may be cut over workgroups
+    if Sq <= 16 and Sk >= 768 and not causal:  # few queries: the keys may be cut over workgroups
         nbytes = lib().mk_sdpa_fwd_workspace_bytes(B, H, Sq, Sk, D, 0)
         ws = _scratch(nbytes, q.device, stream) if nbytes else None
     rc = lib().mk_sdpa_fwd_ws(

@@ -276,14 +276,19 @@ bool sdpa_decode_fits(int64_t BH, int64_t Sq, int64_t Sk, int64_t D, int causal)
   return Sq <= kMaxQ && Sk >= 1 && !causal && !(BH <= 256 && Sk <= 64 && Sq * D > 1280);
 }
 
-int64_t sdpa_decode_slices(int64_t BH, int64_t Sk) {
-  // two workgroups of 4 waves per CU (256 CUs), each with at least 256 keys
-  // (two steps per wave)
+int64_t sdpa_decode_slices(int64_t BH, int64_t Sk, int64_t D) {
+  // Two workgroups of 4 waves per CU (256 CUs), each with at least 256 keys
+  // (two steps per wave), where that gains more than the partial results and
+  // the second launch cost, 2 - 6 us.  One run / cut, caches not in the L2s, us:
+  // D 128, 64 heads x 1024 keys 15.0 / 11.6, 128 x 1024 16.8 / 17.3, 128 x 4096
+  // 60.8 / 53.3, 170 x 2048 33.2 / 37.0, 256 x 1024 26.9 / 29.8 (16 queries 28.1 /
+  // 33.0); D 64, 64 heads x 768 8.6 / 9.2.  More than 128 heads never gain.
+  if (BH > 128 || Sk < (BH <= 64 ? (D == 128 ? 768 : 1024) : 16 * BH)) return 1;
   return std::max<int64_t>(1, std::min<int64_t>({512 / std::max<int64_t>(BH, 1), Sk / 256, 64}));
 }
 
 size_t sdpa_decode_workspace(int64_t BH, int64_t Sq, int64_t Sk, int64_t D) {
-  const int64_t slices = sdpa_decode_slices(BH, Sk);
+  const int64_t slices = sdpa_decode_slices(BH, Sk, D);
   return slices == 1 ? 0 : size_t(BH * slices * Sq * (D + 2) * 4);
 }
 
@@ -292,7 +297,7 @@ int sdpa_decode(hipStream_t s, int64_t B, int64_t H, int64_t Sq, int64_t Sk, int
                 const void* k, int64_t k_bs, int64_t k_hs, int64_t k_ss,
                 const void* v, int64_t v_bs, int64_t v_hs, int64_t v_ss,
                 void* o, int64_t o_bs, int64_t o_hs, int64_t o_ss, float scale, float* lse, void* workspace) {
-  const int64_t slices = workspace ? sdpa_decode_slices(B * H, Sk) : 1;
+  const int64_t slices = workspace ? sdpa_decode_slices(B * H, Sk, D) : 1;
   const int64_t keys = ((Sk + slices - 1) / slices + kStepKeys - 1) / kStepKeys * kStepKeys;
   DecodeArgs a{(const uint16_t*)q, (const uint16_t*)k, (const uint16_t*)v, (uint16_t*)o, lse, (float*)workspace,
                q_bs, q_hs, q_ss, k_bs, k_hs, k_ss, v_bs, v_hs, v_ss, o_bs, o_hs, o_ss,

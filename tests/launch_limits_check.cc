@@ -195,5 +195,12 @@ int main() {
              kernel(64, 1, 64, 128, 1) != few,
          "the kernel of few queries");
   expect(mk_sdpa_fwd_workspace_bytes(1, 64, 16, 64, 128, 0) == 0, "no workspace for the query-tile kernel");
+  // runs of keys: heads, keys, head_dim, how many
+  const int64_t runs[][4] = {{256, 1024, 128, 1}, {129, 16384, 64, 1}, {128, 2047, 128, 1}, {128, 2048, 128, 4},
+                             {96, 1536, 64, 5},   {64, 767, 128, 1},   {64, 768, 128, 3},   {64, 1000, 64, 1},
+                             {64, 1024, 64, 4},   {1, 16384, 128, 64}, {8, 16384, 64, 64}};
+  for (const auto& r : runs)
+    expect(mk_sdpa_fwd_workspace_bytes(1, r[0], 2, r[1], r[2], 0) == (r[3] == 1 ? 0 : uint64_t(r[0] * r[3] * 2 * (r[2] + 2) * 4)),
+           "runs of " + std::to_string(r[1]) + " keys of " + std::to_string(r[0]) + " heads");
   std::printf("ok\n");
 }

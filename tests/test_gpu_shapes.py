@@ -29,8 +29,10 @@ def shifted(t, off):
 
 # rows x columns around a wave's, a 4-wave and a 16-wave team's shares (64, 512, 2048 and 8192
 # vectors), tails of every kind, and past the registers (65536 bf16, 32768 fp32)
-ROW_SHAPES = [(1, 1, 0), (3, 7, 1), (2050, 511, 1), (700, 4097, 0), (511, 4105, 3), (2, 16384, 1), (33, 16391, 0),
-              (5, 50257, 0), (3, 65529, 1), (2, 65551, 0), (2, 140003, 1)]
+ROW_SHAPES = [(1, 1, 0), (4, 7, 1), (2050, 511, 1), (700, 4097, 0), (511, 4105, 3), (2, 16384, 1), (33, 16391, 0),
+              (5, 50257, 0), (4, 65529, 1), (2, 65551, 0), (2, 140003, 1)]
+# one wave with 3 - 4 and 5 - 8 vectors per lane, four waves with 5 - 8 (softmax, LayerNorm), of either type
+ROW_SHAPES += [(2049, 601, 1), (2051, 1100, 0), (2051, 2043, 1), (2049, 4091, 1), (600, 6001, 1), (600, 12301, 0)]
 
 
 @pytest.mark.parametrize("rows,cols,off", ROW_SHAPES)
@@ -59,9 +61,8 @@ def test_row_kernels_any_width(K, rows, cols, off, dtype):
     np.testing.assert_array_equal(K.row_reduce(xd, "max").cpu().numpy().astype(np.float64), xf.max(-1))
 
     ok = slice(3, None) if rows > 2 else slice(None)  # the finite rows
-    xs, xf = shifted(x[ok], off) if x[ok].numel() else None, xf[ok]
-    if xs is None:
-        return
+    assert x[ok].numel() > 0
+    xs, xf = shifted(x[ok], off), xf[ok]
     # unit roundoff of the stored type: bf16 has 8 significant bits, so half an ulp is up to 2^-8 of the value
     eps, out = 16 * 2.0 ** -24 * np.sqrt(cols), 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -24
     got = K.row_reduce(xs, "sum").cpu().double().numpy()
@@ -138,8 +139,50 @@ def test_gemm_few_rows(K, M, N, K_, dtype, b_kc):
     assert bool((out[M] == 7).all()) and bool((out[:, N] == 7).all())
 
 
+# deep products of few rows: k cut over workgroups (the workspace function says so) and, where C's
+# rows are off the grid, in one launch whose waves run their pipelined loop; k's remainder owned by
+# the first and by later slices (281 steps of 32 in 16 slices of 8 or 16 waves: slice 1 or 3)
+@pytest.mark.parametrize("M,N,K_", [(1, 256, 4300), (16, 768, 9003), (17, 64, 4127), (33, 500, 6200), (64, 132, 12301),
+                                    (5, 2048, 16411)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("b_kc", [False, True])
+@pytest.mark.parametrize("sliced", [True, False])
+def test_gemm_few_rows_deep(K, M, N, K_, dtype, b_kc, sliced):
+    """relu(A B + bias) through gemm, and A B through gemm_splitk, against
+    float64, with NaN past every row end: fp32 sums within 8 * 2^-23 of the
+    magnitudes (at most 0.01 here; a lost element of k is worth 0.6 on
+    average) and one rounding to C."""
+    print(f"case: gemm {M}x{N}x{K_} {dtype} b_kc={b_kc} sliced={sliced}", flush=True)
+    g = torch.Generator().manual_seed(M + N + K_)
+    a, b = torch.randn(M, K_, generator=g).to(dtype), torch.randn(K_, N, generator=g).to(dtype)
+    bias = torch.randn(N, generator=g).to(dtype)
+    ad = torch.full((M, K_ + 3), float("nan"), dtype=dtype, device="cuda")[:, 1:K_ + 1]
+    ad.copy_(a)
+    rows, cols = (N, K_) if b_kc else (K_, N)
+    bd = torch.full((rows, cols + 5), float("nan"), dtype=dtype, device="cuda")[:, 2:cols + 2]
+    bd.copy_(b.t() if b_kc else b)
+    bd = bd.t() if b_kc else bd
+    need = K.lib().mk_gemm_few_rows_workspace_bytes(K.mk_dtype(dtype), M, N, K_, 1, *bd.stride())
+    assert need >= 2 * M * N * 4
+    want, mag = a.double() @ b.double(), a.double().abs() @ b.double().abs()
+    for out_dtype in (torch.float32, dtype):
+        u = 2.0 ** -8 if out_dtype == torch.bfloat16 else 2.0 ** -24
+        out = torch.full((M + 1, N + (4 if sliced else 1)), 7.0, dtype=out_dtype, device="cuda")
+        K.gemm(ad, bd, out_dtype=out_dtype, bias=bias.cuda().to(out_dtype), relu=True, out=out[:M, :N])
+        top = torch.relu(want + bias.double())
+        bound = 8 * 2.0 ** -23 * (mag + bias.double().abs()) + u * top
+        assert bool(((out[:M, :N].cpu().double() - top).abs() <= bound).all())
+        assert bool((out[M] == 7).all()) and bool((out[:, N:] == 7).all())
+        if sliced:
+            for splits in (3, 16):
+                got = K.gemm_splitk(ad, bd, splits, out_dtype=out_dtype)
+                assert bool(((got.cpu().double() - want).abs() <= 8 * 2.0 ** -23 * mag + u * want.abs()).all())
+                assert torch.equal(got, K.gemm_splitk(ad, bd, splits, out_dtype=out_dtype))
+
+
 def test_gemm_few_rows_batched_and_split(K):
-    """Batches with a broadcast B, and the split-K entry at few rows."""
+    """Batches with a broadcast B, and the split-K entry at few rows (too
+    shallow a k to be cut)."""
     g = torch.Generator().manual_seed(3)
     a, b = torch.randn(5, 7, 100, generator=g), torch.randn(100, 48, generator=g)
     got = K.gemm(a.cuda(), b.cuda())
@@ -155,6 +198,7 @@ def test_gemm_few_rows_batched_and_split(K):
 @pytest.mark.parametrize("B,H,Sq,Sk,D", [(1, 1, 1, 1, 128), (2, 3, 1, 31, 64), (1, 2, 7, 33, 128), (1, 2, 16, 129, 64),
                                          (2, 2, 1, 511, 128), (1, 2, 2, 513, 128), (1, 3, 16, 2049, 128),
                                          (3, 5, 4, 1000, 64), (1, 1, 1, 16391, 128), (32, 16, 1, 300, 64),
+                                         (3, 5, 4, 1025, 64), (1, 2, 2, 769, 128), (8, 16, 1, 2048, 128),
                                          (1, 2, 10, 64, 128), (2, 3, 11, 33, 128), (1, 2, 16, 64, 128),
                                          (1, 2, 16, 65, 128), (32, 16, 16, 64, 128), (16, 16, 12, 1, 128)])
 @pytest.mark.parametrize("slices", [True, False])
@@ -276,16 +320,29 @@ def test_gemm_splitk_slices_off_the_16_byte_grid(K, M, N, Kd, splits):
     """Slice counts that divide K into slices that are no multiple of 8, on
     the uneven slices (400 in 8: slices of 56 are too short for the tiled
     kernel; 36 and 1004: rows off the grid, the even form), each operand
-    k-contiguous in turn.  Bound: fp32 sums in another order, K ulps of the
-    sum of magnitudes at the most."""
+    k-contiguous in turn with NaN past K.  fp32 sums within 8 * 2^-23 of the
+    magnitudes, bit for bit the slices' own products added in order."""
     assert Kd % splits == 0 and Kd // splits % 8 != 0
     g = torch.Generator().manual_seed(Kd)
     a, b = torch.randn(M, Kd, generator=g).bfloat16(), torch.randn(Kd, N, generator=g).bfloat16()
     want, norm = a.double() @ b.double(), a.double().abs() @ b.double().abs()
-    for ad, bd in ((a.cuda(), b.cuda()), (a.cuda(), b.t().contiguous().cuda().t()),
-                   (a.t().contiguous().cuda().t(), b.t().contiguous().cuda().t())):
+
+    def k_rows(t):  # t's rows of K on the GPU, 8 NaN behind each
+        rows = torch.full((t.shape[0], Kd + 8), float("nan"), dtype=torch.bfloat16, device="cuda")[:, :Kd]
+        rows.copy_(t)
+        return rows
+
+    for ad, bd in ((k_rows(a), b.cuda()), (k_rows(a), k_rows(b.t()).t()), (a.t().contiguous().cuda().t(), k_rows(b.t()).t())):
         got = K.gemm_splitk(ad, bd, splits)
-        assert bool(((got.cpu().double() - want).abs() <= Kd * 2.0 ** -24 * norm).all())
+        assert bool(((got.cpu().double() - want).abs() <= 8 * 2.0 ** -23 * norm).all())
+        ks = ((Kd + splits - 1) // splits + 7) // 8 * 8
+        if ks < 64 or any(max(t.stride()) % 8 for t in (ad, bd)):
+            ks = Kd // splits
+        total = None
+        for k0 in range(0, Kd, ks):
+            part = K.gemm(ad[:, k0:k0 + ks], bd[k0:k0 + ks], out_dtype=torch.float32)
+            total = part if total is None else total + part
+        assert torch.equal(got, total)
         assert torch.equal(got, K.gemm_splitk(ad, bd, splits))
         low = K.gemm_splitk(ad, bd, splits, out_dtype=torch.bfloat16)
         assert torch.equal(low, got.bfloat16())

@@ -458,6 +458,8 @@ extern "C" int mk_gemm_splitk_typed(void* stream, int ab_type, int c_type, int64
   if ((N % 4) != 0 || (c_ms % 4) != 0 || (reinterpret_cast<uintptr_t>(C) & cal) ||
       (reinterpret_cast<uintptr_t>(workspace) & 15u))
     return fail(MK_ERR_UNSUPPORTED, "mk_gemm_splitk: N and c_ms multiples of 4, aligned C and workspace");
+  if (K % splits == 0 && splits >= 65536)
+    return fail(MK_ERR_UNSUPPORTED, "mk_gemm_splitk: even slices must be < 65536");
   // few rows: the kernel that takes them splits k inside the workgroup, and
   // over workgroups only where the columns alone leave the chip idle
   if (gemm_skinny_fits(M, N, K, a_ks, b_ks, b_ns)) {

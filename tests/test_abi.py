@@ -48,6 +48,18 @@ def test_kernel_library_loads_and_answers_without_gpu():
     assert lib.mk_scatter_add_workspace_bytes(50257, 65536) > 4 * 65536 * 4
 
 
+def test_splitk_refuses_too_many_even_slices():
+    """65536 even slices are more than one launch's batches, with few rows as
+    with many, before anything is launched."""
+    from mi355x_pjrt import _lib
+
+    lib = _lib.load_kernels()
+    for rows in (16, 64, 200):
+        rc = lib.mk_gemm_splitk_typed(None, 13, 11, rows, 64, 131072, 4096, 131072, 1, 4096, 64, 1, 4096, 64, 65536, 4096,
+                                      None, 0)
+        assert rc == 2 and b"65536" in lib.mk_last_error(), (rows, rc, lib.mk_last_error())
+
+
 def test_pjrt_plugin_exports_only_GetPjrtApi():
     so = os.path.join(LIB, "libpjrt_mi355x.so")
     if not os.path.exists(so):

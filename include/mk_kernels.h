@@ -105,7 +105,9 @@ int mk_gemm_gelu_bwd(void* stream, int ab_type, int64_t M, int64_t N, int64_t K,
  * axis is cut into `splits` equal slices; one batched mk_gemm writes the
  * slices' products to the workspace (splits x M x N fp32) and a second pass
  * adds them in slice order into C (deterministic: the result does not depend
- * on scheduling).  K % splits == 0; N and c_ms multiples of 4; C and
+ * on scheduling).  Equal slices that would start off the 16-byte grid of a
+ * k-contiguous bf16 operand are cut as mk_gemm_splitk_typed cuts uneven ones
+ * where the tiled kernel takes them.  K % splits == 0, splits < 65536; N and c_ms multiples of 4; C and
  * workspace 16-byte aligned; C is overwritten.  splits == 1 is a plain
  * mk_gemm call (no workspace).  Operand convention as mk_gemm.
  * Replaces, for these products: src/jam/ops/linalg.mm:98. */
@@ -198,9 +200,9 @@ int mk_sdpa_fwd(void* stream, int64_t B, int64_t H, int64_t Sq, int64_t Sk, int6
                 float scale, int causal, float* lse);
 
 /* mk_sdpa_fwd with a workspace of mk_sdpa_fwd_workspace_bytes (0 bytes: none
- * is used; NULL: mk_sdpa_fwd): with at most 16 queries, no causal mask and too
- * few heads to fill the chip, the keys are cut into runs whose partial
- * results are merged in order by a second launch. */
+ * is used; NULL: mk_sdpa_fwd): with at most 16 queries, no causal mask, at most
+ * 128 heads and many keys, the keys are cut into runs whose partial results
+ * are merged in order by a second launch. */
 size_t mk_sdpa_fwd_workspace_bytes(int64_t B, int64_t H, int64_t Sq, int64_t Sk, int64_t D, int causal);
 int mk_sdpa_fwd_ws(void* stream, int64_t B, int64_t H, int64_t Sq, int64_t Sk, int64_t D,
                    const void* q, int64_t q_bs, int64_t q_hs, int64_t q_ss,

@@ -34,8 +34,8 @@ the 50257 classes into a 8192 x 768 result) on mk_gemm_splitk_typed, 8
 slices.  No product goes to the library: rocBLAS runs the logits product on a
 stream-K kernel whose workgroups wait for each other through the handle's one
 workspace, which captured steps on several streams would share (two such
-kernels at once need never finish); the tiled kernel takes 667 us for it
-against about 600.  All parameters live in five flat buffers
+kernels at once need never finish); the tiled kernel takes 692 us for it in
+the step, the library 600 - 635.  All parameters live in five flat buffers
 (fp32 master, bf16 working copy, fp32 gradient, fp32 m, fp32 v), each
 parameter a 64-element-aligned slice, so the optimizer is a single launch and
 every gradient is written in place.  The

@@ -63,8 +63,9 @@ def _ptr(t):
 def _scratch(nbytes, device, stream):
     """A call's workspace on `stream` (None: the current one), from that
     stream's memory: freed when the call returns, it goes to later work of the
-    same stream only."""
-    if stream is None:
+    same stream only.  (A handle that is no torch stream has no such memory:
+    its caller passes a workspace, or waits before it frees anything.)"""
+    if stream is None or not isinstance(stream, torch.cuda.Stream) or stream.cuda_stream == _stream():
         return torch.empty(nbytes, dtype=torch.uint8, device=device)
     with torch.cuda.stream(stream):
         return torch.empty(nbytes, dtype=torch.uint8, device=device)

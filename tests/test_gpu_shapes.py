@@ -2,6 +2,8 @@
 tiles and teams, remainders, unaligned rows, the smallest and largest of each
 range.  References are the oracle, or torch on the CPU in float64."""
 
+import types
+
 import numpy as np
 import pytest
 import torch
@@ -252,6 +254,11 @@ def test_few_rows_and_queries_on_an_explicit_stream(K):
     blocks = [torch.empty(1 << 22, dtype=torch.uint8, device="cuda") for _ in range(4)]
     assert all(b.data_ptr() != held for b in blocks)
     assert K._scratch(1 << 22, x.device, s).data_ptr() == held
+    bare = types.SimpleNamespace(cuda_stream=s.cuda_stream)  # any object with a stream's handle
+    for ys, want in ((K.gemm(x, w, stream=bare), y), (K.gemm_splitk(x, w, 16, stream=bare, out_dtype=x.dtype), y),
+                     (K.sdpa_fwd(q, k, v, 0.1, causal=False, stream=bare), o)):
+        s.synchronize()
+        assert torch.equal(ys, want)
 
 
 def test_sdpa_few_queries_infinities(K):

@@ -81,6 +81,7 @@ struct TiledGemm {
   int c_mode;                 // 0 element stores, 1 4-column vector stores, 2 / 3 staged 16-bit rows
                               // stored as 16-byte chunks / element by element, 4 / 5 staged fp32 rows
                               // stored element by element / as 16-byte chunks
+  int stream_c;               // c_mode 2: C's whole chunks go out as non-temporal stores
 };
 
 // The copies one wave makes of one operand's tile: copy c is j = wave + W c
@@ -254,11 +255,12 @@ __device__ inline void finish4(const TiledGemm& p, int64_t n, float (&v)[4]) {
 // rows 2 apart share the bank offset).  Then the workgroup stores runs of consecutive
 // C rows: whole 16-byte chunks when C rows are 16-byte aligned (ROWS16),
 // else one element per thread, consecutive threads on consecutive columns.
-// The chunks are stored non-temporally: a round of workgroups writes as much
-// as an XCD's whole L2 holds (32 tiles of 96 or 128 KB), which evicted the
-// operand rows and columns its next round shares.  8192 x 50257 x 768 with
-// bf16 C: 775 -> 703 us on 256 x 256 tiles, 764 -> 668 us on 128 x 192.  fp32
-// C keeps ordinary stores (no gain, and split-K slices are read back at once).
+// A round of workgroups writes as much as an XCD's whole L2 holds (32 tiles of
+// 96 or 128 KB), which evicted the operand rows and columns its next round
+// shares, so chunks of a C too large to stay or not read soon are stored past
+// the caches (stream_c, set on the host: gemm_tiled_streams).  Any other C is
+// the next kernel's operand and keeps ordinary stores, as does the GELU side
+// output; fp32 C always does (no gain, and split-K slices are read back at once).
 template <int CT, bool ROWS16, int TM, int TN, int kW, int kWM, int kWN, int kI, int kJ>
 __device__ __attribute__((always_inline)) inline void store_staged(const TiledGemm& p,
                                                                    const f32x16_t (&acc)[kI][kJ], uint16_t* st,
@@ -313,49 +315,64 @@ __device__ __attribute__((always_inline)) inline void store_staged(const TiledGe
     return;
   }
   const bool gelu_bwd = (p.epilogue & kEpiGeluBwd) != 0;
+  auto chunks = [&](auto stream) __attribute__((always_inline)) {
 #pragma unroll
-  for (int it = 0; it < TM * kCpr / kThreads; ++it) {
-    const int e = it * kThreads + int(threadIdx.x);
-    const int row = e / kCpr, cn = e % kCpr;
-    u32x4_t v = *reinterpret_cast<const u32x4_t*>(st + row * TN + 8 * pos(row, cn));
-    const int64_t m = m0 + row, n = n0 + 8 * cn;
-    if (gelu_bwd) {
-      // v (the product as stored) times gelu'(pre), pre read only inside
-      // [M, N); the chunk is written back for the column pass (zeros
-      // outside [M, N))
-      u32x4_t pre = {0u, 0u, 0u, 0u};
+    for (int it = 0; it < TM * kCpr / kThreads; ++it) {
+      const int e = it * kThreads + int(threadIdx.x);
+      const int row = e / kCpr, cn = e % kCpr;
+      u32x4_t v = *reinterpret_cast<const u32x4_t*>(st + row * TN + 8 * pos(row, cn));
+      const int64_t m = m0 + row, n = n0 + 8 * cn;
+      if (gelu_bwd) {
+        // v (the product as stored) times gelu'(pre), pre read only inside
+        // [M, N); the chunk is written back for the column pass (zeros
+        // outside [M, N))
+        u32x4_t pre = {0u, 0u, 0u, 0u};
+        if (m < p.M && n + 8 <= p.N) {
+          pre = *reinterpret_cast<const u32x4_t*>(p.aux + m * p.ld_aux + n);
+        } else if (m < p.M && n < p.N) {
+#pragma unroll
+          for (int q = 0; q < 8; ++q)
+            if (n + q < p.N) pre[q / 2] |= uint32_t(p.aux[m * p.ld_aux + n + q]) << (16 * (q & 1));
+        }
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const bool in0 = m < p.M && n + 2 * q < p.N, in1 = m < p.M && n + 2 * q + 1 < p.N;
+          const float d0 = __builtin_bit_cast(float, v[q] << 16), d1 = __builtin_bit_cast(float, v[q] & 0xFFFF0000u);
+          const float x0 = __builtin_bit_cast(float, pre[q] << 16), x1 = __builtin_bit_cast(float, pre[q] & 0xFFFF0000u);
+          const uint32_t lo = in0 ? f32_to_bf16(d0 * gelu_tanh_grad_f32(x0)) : 0u;
+          const uint32_t hi = in1 ? f32_to_bf16(d1 * gelu_tanh_grad_f32(x1)) : 0u;
+          v[q] = lo | (hi << 16);
+        }
+        *reinterpret_cast<u32x4_t*>(st + row * TN + 8 * pos(row, cn)) = v;
+      }
       if (m < p.M && n + 8 <= p.N) {
-        pre = *reinterpret_cast<const u32x4_t*>(p.aux + m * p.ld_aux + n);
-      } else if (m < p.M && n < p.N) {
+        u32x4_t* const to = reinterpret_cast<u32x4_t*>(Cz + 2 * (m * p.ldc + n));
+        if constexpr (decltype(stream)::value) {
+          __builtin_nontemporal_store(v, to);
+        } else {
+          *to = v;
+        }
+        if (p.epilogue & kEpiGeluAux) *reinterpret_cast<u32x4_t*>(p.aux + m * p.ld_aux + n) = gelu8_bf16(v);
+      } else if (m < p.M && n < p.N) {  // the chunk that straddles N: its columns below N only
+        uint16_t* Ce = reinterpret_cast<uint16_t*>(Cz) + m * p.ldc + n;
+        const u32x4_t gv = gelu8_bf16(v);
 #pragma unroll
         for (int q = 0; q < 8; ++q)
-          if (n + q < p.N) pre[q / 2] |= uint32_t(p.aux[m * p.ld_aux + n + q]) << (16 * (q & 1));
+          if (n + q < p.N) {
+            Ce[q] = uint16_t(v[q / 2] >> (16 * (q & 1)));
+            if (p.epilogue & kEpiGeluAux) p.aux[m * p.ld_aux + n + q] = uint16_t(gv[q / 2] >> (16 * (q & 1)));
+          }
       }
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const bool in0 = m < p.M && n + 2 * q < p.N, in1 = m < p.M && n + 2 * q + 1 < p.N;
-        const float d0 = __builtin_bit_cast(float, v[q] << 16), d1 = __builtin_bit_cast(float, v[q] & 0xFFFF0000u);
-        const float x0 = __builtin_bit_cast(float, pre[q] << 16), x1 = __builtin_bit_cast(float, pre[q] & 0xFFFF0000u);
-        const uint32_t lo = in0 ? f32_to_bf16(d0 * gelu_tanh_grad_f32(x0)) : 0u;
-        const uint32_t hi = in1 ? f32_to_bf16(d1 * gelu_tanh_grad_f32(x1)) : 0u;
-        v[q] = lo | (hi << 16);
-      }
-      *reinterpret_cast<u32x4_t*>(st + row * TN + 8 * pos(row, cn)) = v;
     }
-    if (m < p.M && n + 8 <= p.N) {
-      __builtin_nontemporal_store(v, reinterpret_cast<u32x4_t*>(Cz + 2 * (m * p.ldc + n)));
-      if (p.epilogue & kEpiGeluAux)
-        __builtin_nontemporal_store(gelu8_bf16(v), reinterpret_cast<u32x4_t*>(p.aux + m * p.ld_aux + n));
-    } else if (m < p.M && n < p.N) {  // the chunk that straddles N: its columns below N only
-      uint16_t* Ce = reinterpret_cast<uint16_t*>(Cz) + m * p.ldc + n;
-      const u32x4_t gv = gelu8_bf16(v);
-#pragma unroll
-      for (int q = 0; q < 8; ++q)
-        if (n + q < p.N) {
-          Ce[q] = uint16_t(v[q / 2] >> (16 * (q & 1)));
-          if (p.epilogue & kEpiGeluAux) p.aux[m * p.ld_aux + n + q] = uint16_t(gv[q / 2] >> (16 * (q & 1)));
-        }
-    }
+  };
+  // one loop for each kind of store (8192 x 4096 x 1024 78 us, 81 with a branch
+  // at every store).  The empty statement keeps the loops' last stores apart,
+  // which the compiler would make one ordinary store of.
+  if (p.stream_c) {
+    chunks(std::true_type{});
+    asm volatile("");
+  } else {
+    chunks(std::false_type{});
   }
   if (gelu_bwd) {
     // column sums of the stored values, 128 rows at a time in row order,
@@ -753,6 +770,28 @@ int64_t cu_count() {
 
 }  // namespace
 
+// Where C goes past the caches.  us, ordinary stores / streamed, of the product
+// and of it with the product that reads its result (bf16, K 768 unless given):
+// - from 192 MiB on, three quarters of the last-level cache: 8192 x 50257 (823
+//   MB) 815 / 688; 2048 x 50304 (206 MB) 182 / 167 and 834 / 835; 32768 x 3072
+//   (201 MB) 163 / 166 and 320 / 313.  Below, the reader finds it in the caches:
+//   2300 x 40000 (184 MB) 154 / 153 and 555 / 672; 1024 x 50304 (103 MB) 95 / 94
+//   and 572 / 742; 8192 x 3072 (50 MB) 44 / 43 and 88 / 96; 4096 x 3072 60 / 69;
+// - with the GELU side output, which is the next operand (and stays ordinary:
+//   streamed as well, 8192 x 3072 and its reader take 117 for 110): C is read in
+//   the backward pass.  MLP forward and backward of 4096 x 1024 x 4096 363 / 354,
+//   32768 x 3072 274 / 246 and 428 / 385;
+// - a C of 4 MiB or more beside a contraction 4 times as deep as it is wide: A
+//   stays cached instead for its next reader, the weight gradient.  The MLP of
+//   4096 x 1024 x 4096 380 / 368, 2048 x 1024 x 4096 257 / 253, 8192 x 768 x 3072
+//   394 / 392.  With a LayerNorm and then a product reading 8192 x 768 (K 3072)
+//   96 / 95; a product reading it at once takes 90 / 92 .. 94.  At K = 2 N the
+//   LayerNorm's reader loses as well (77 / 80).
+bool gemm_tiled_streams(int64_t batch, int64_t M, int64_t N, int64_t K, bool side_output) {
+  const int64_t bytes = 2 * batch * M * N;
+  return side_output || bytes >= int64_t(192) << 20 || (bytes >= int64_t(4) << 20 && K >= 4 * N);
+}
+
 int gemm_tiled(hipStream_t s, int c_type, int64_t batch, int64_t M, int64_t N, int64_t K, const void* A,
                int64_t a_bs, int64_t a_ms, int64_t a_ks, const void* B, int64_t b_bs, int64_t b_ks,
                int64_t b_ns, void* C, int64_t c_bs, int64_t c_ms, const void* bias, int epilogue, int64_t k_rem,
@@ -762,6 +801,7 @@ int gemm_tiled(hipStream_t s, int c_type, int64_t batch, int64_t M, int64_t N, i
   if (!tiled_args(a, a_kc, b_kc, c_type, batch, M, N, K, A, a_bs, a_ms, a_ks, B, b_bs, b_ks, b_ns, C, c_bs, c_ms,
                   bias, epilogue, k_rem, Y, y_ms, colpart))
     return -1;
+  a.stream_c = gemm_tiled_streams(batch, M, N, K, (epilogue & kEpiGeluAux) != 0);
   // Kernel shape: the one with the least estimated time.  A round of
   // workgroups costs nk + e k tiles, each of its area over the shape's rate
   // per CU; e is the first loads and the epilogue in k tiles, for 16-bit C
@@ -772,11 +812,11 @@ int gemm_tiled(hipStream_t s, int c_type, int64_t batch, int64_t M, int64_t N, i
   // a full one's time, however few they are.  The constants are fitted to the
   // three shapes' times on 860 drawn products and the training step's
   // (profiles/gemm_tile_shapes.txt; 250 .. 50257 rows and columns, 64 .. 8192
-  // deep, both C types, unsplit, split and batched).  The choice costs 0.3% on
-  // average over always taking the fastest, 11% at the worst but for two
-  // products.  In the order below, us: 8192 x 50257 x 768, bf16 C 774 / 618 /
-  // 741; 3245 x 2112 x 1344, fp32 C 42 / 35 / 29; 8192 x 8192 x 4096 451 /
-  // 487 / 519; 8192 x 6144 x 2048 181 / 187 / 201.
+  // deep, both C types, unsplit, split and batched).  The choice costs 0.4% on
+  // average over always taking the fastest, 9% at the worst but for two
+  // products.  In the order below, us: 8192 x 50257 x 768, bf16 C 778 / 648 /
+  // 758; 3245 x 2112 x 1344, fp32 C 42 / 35 / 29; 8192 x 8192 x 4096 469 /
+  // 508 / 538; 8192 x 6144 x 2048 195 / 197 / 211.
   struct Option {
     int tm, tn, per_cu;
     double rate, e16, e32;

@@ -83,6 +83,8 @@ int gemm_tiled(hipStream_t s, int c_type, int64_t batch, int64_t M, int64_t N, i
                int64_t a_bs, int64_t a_ms, int64_t a_ks, const void* B, int64_t b_bs, int64_t b_ks,
                int64_t b_ns, void* C, int64_t c_bs, int64_t c_ms, const void* bias, int epilogue,
                int64_t k_rem = 0, void* Y = nullptr, int64_t y_ms = 0, float* colpart = nullptr);
+// whether its 16-bit C is stored past the caches
+bool gemm_tiled_streams(int64_t batch, int64_t M, int64_t N, int64_t K, bool side_output);
 
 // GEMM with at most 64 rows behind mk_gemm (gemm_skinny.hip), same operand
 // convention, A k-contiguous; returns -1 without launching when the shape or

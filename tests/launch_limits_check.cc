@@ -14,6 +14,10 @@
 
 #include "mk_kernels.h"
 
+namespace mk {
+bool gemm_tiled_streams(int64_t batch, int64_t M, int64_t N, int64_t K, bool side_output);  // gemm_tiled.hip
+}
+
 namespace {
 struct Launch {
   const void* kernel;       // its host stub
@@ -179,6 +183,16 @@ int main() {
            "the tile shape of " + std::to_string(t.M) + " x " + std::to_string(t.N) + " x " + std::to_string(t.K));
     g_launches.clear();
   }
+
+  // a 16-bit result that the next product reads is stored into the caches
+  struct { int64_t batch, M, N, K; bool side, streams; } results[] = {
+      {1, 2048, 4096, 1024, false, false},   {1, 256, 8192, 2048, false, false}, {1, 2300, 40000, 768, false, false},
+      {12, 1024, 1024, 64, false, false},    {1, 8192, 768, 1536, false, false}, {1, 1024, 768, 3072, false, false},
+      {1, 8192, 50264, 768, false, true},    {1, 2048, 4096, 1024, true, true},  {1, 8192, 768, 3072, false, true},
+      {64, 2048, 2048, 128, false, true}};
+  for (const auto& r : results)
+    expect(mk::gemm_tiled_streams(r.batch, r.M, r.N, r.K, r.side) == r.streams,
+           "the stores of " + std::to_string(r.M) + " x " + std::to_string(r.N) + " x " + std::to_string(r.K));
 
   // few queries, many of them beside few keys: the query-tile kernel of 17 queries
   auto kernel = [&](int64_t BH, int64_t Sq, int64_t Sk, int64_t D, int causal) {

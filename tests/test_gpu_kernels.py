@@ -812,6 +812,41 @@ def test_gemm_bias_gelu(K, out_dtype):
             assert torch.isnan(c[:, N:].float()).all() and torch.isnan(y[:, N:].float()).all()
 
 
+@pytest.mark.parametrize("M,N,Kd,gelu", [(4096, 24568, 64, False), (4096, 24576, 64, False), (4099, 24572, 64, False),
+                                         (2050, 4092, 64, True), (256, 252, 64, True), (4092, 512, 2048, False),
+                                         (4096, 512, 2048, False), (4100, 516, 2064, False)])
+def test_gemm_tiled_result_stores(K, M, N, Kd, gelu):
+    """bf16 results stored into the caches and past them (from 192 MiB on, with
+    the GELU side output, from 4 MiB on beside a deep contraction), ragged rows
+    and the chunk that straddles N included: bit for bit the fp32 product (its
+    stores are ordinary) rounded to bf16, the row padding untouched.  The next
+    product reads the result as its operand at once."""
+    wide = (N + 7) // 8 * 8
+    g = torch.Generator(device="cuda")
+    g.manual_seed(N)
+    print(f"case: gemm_tiled_result_stores M={M} N={N} K={Kd} gelu={gelu}", flush=True)
+    a = torch.randn(M, Kd, device="cuda", generator=g).bfloat16()
+    b = torch.randn(Kd, wide, device="cuda", generator=g).bfloat16()[:, :N]
+    d = torch.randn(wide, 128, device="cuda", generator=g).bfloat16()[:N]
+    c, y = (torch.full((M, wide), float("nan"), dtype=torch.bfloat16, device="cuda") for _ in range(2))
+    if gelu:
+        K.gemm_bias_gelu(a, b, torch.zeros(N, dtype=torch.bfloat16, device="cuda"), out=c[:, :N], y=y[:, :N])
+    else:
+        K.gemm(a, b, out=c[:, :N])
+    out = y if gelu else c
+    then = K.gemm(out[:, :N], d)
+    want = K.gemm(a, b, out_dtype=torch.float32).bfloat16()
+    assert torch.equal(c[:, :N], want)
+    if gelu:
+        want = K.gelu_tanh(want)
+        assert torch.equal(y[:, :N], want)
+    assert torch.isnan(c[:, N:]).all() and torch.isnan(out[:, N:]).all()
+    copy = torch.zeros(M, wide, dtype=torch.bfloat16, device="cuda")
+    copy[:, :N] = want
+    torch.cuda.synchronize()
+    assert torch.equal(then, K.gemm(copy[:, :N], d))
+
+
 def test_gemm_gelu_bwd(K):
     """mk_gemm_gelu_bwd: dx is mk_gelu_tanh_bwd(pre, mk_gemm's bf16 product)
     bit for bit, including the chunk that straddles N (rows padded to 1008)

@@ -8,6 +8,7 @@ if the library is missing the call raises.
 from __future__ import annotations
 
 import ctypes
+import functools
 
 import torch
 
@@ -108,6 +109,11 @@ def sdpa_fwd(q, k, v, scale: float, causal: bool = True, out=None, lse=None, str
 
 
 # ------------------------------------------------------------------ a4 GEMM
+@functools.lru_cache(maxsize=1024)
+def _few_rows_bytes(ab, M, N, K, a_ks, b_ks, b_ns):
+    return lib().mk_gemm_few_rows_workspace_bytes(ab, M, N, K, a_ks, b_ks, b_ns)
+
+
 def _gemm2(a, b, out_dtype, bias, relu, out, stream):
     """gemm of 2-D views."""
     M, K = a.shape
@@ -120,9 +126,13 @@ def _gemm2(a, b, out_dtype, bias, relu, out, stream):
     if bias is not None and bias.dtype == torch.float32 and out_dtype != torch.float32:
         epi |= 4  # an fp32 bias added before the narrowing store
     ab, ct, sa, sb, so = mk_dtype(a.dtype), mk_dtype(out_dtype), a.stride(), b.stride(), out.stride()
-    # few rows and columns: the contraction may be cut over workgroups
-    if 0 < M <= 64 and K >= 1024 and so[0] % 4 == 0 and out.data_ptr() % 16 == 0 and out_dtype != torch.float16:
-        nbytes = lib().mk_gemm_few_rows_workspace_bytes(ab, M, N, K, sa[1], sb[0], sb[1])
+    # few rows and columns: the contraction may be cut over workgroups.  Below
+    # 4096 bf16 deep a cut saves less on the GPU (4 x 3072 x 768: 2 us) than its
+    # workspace and second kernel cost in this call (an MLP of 4 x 768 x 3072
+    # called in a row: 19.4 us, 24.7 with the cut)
+    if 0 < M <= 64 and K * a.element_size() >= 8192 and so[0] % 4 == 0 and out.data_ptr() % 16 == 0 and \
+            out_dtype != torch.float16:
+        nbytes = _few_rows_bytes(ab, M, N, K, sa[1], sb[0], sb[1])
         if nbytes:
             ws = _scratch(nbytes, a.device, stream)
             rc = lib().mk_gemm_splitk_typed(_stream(stream), ab, ct, M, N, K, a.data_ptr(), sa[0], sa[1], b.data_ptr(),

@@ -182,6 +182,18 @@ def test_gemm_few_rows_deep(K, M, N, K_, dtype, b_kc, sliced):
                 assert torch.equal(got, K.gemm_splitk(ad, bd, splits, out_dtype=out_dtype))
 
 
+@pytest.mark.parametrize("dtype,depth", [(torch.bfloat16, 4096), (torch.float32, 2048)])
+def test_gemm_few_rows_cut_from_its_depth_on(K, dtype, depth, monkeypatch):
+    """A product too shallow to pay for a workspace and a second kernel takes
+    neither; from 4096 bf16 (2048 fp32) deep on it is cut."""
+    taken, scratch = [], K._scratch
+    monkeypatch.setattr(K, "_scratch", lambda n, *rest: (taken.append(n), scratch(n, *rest))[1])
+    for k in (depth - 8, depth):
+        x, w = torch.ones(4, k, dtype=dtype, device="cuda"), torch.ones(k, 768, dtype=dtype, device="cuda")
+        assert bool((K.gemm(x, w, out_dtype=torch.float32) == k).all())
+        assert len(taken) == (k >= depth), k
+
+
 def test_gemm_few_rows_batched_and_split(K):
     """Batches with a broadcast B, and the split-K entry at few rows (too
     shallow a k to be cut)."""

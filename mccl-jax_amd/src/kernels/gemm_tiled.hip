@@ -316,7 +316,7 @@ __device__ __attribute__((always_inline)) inline void store_staged(const TiledGe
   }
   const bool gelu_bwd = (p.epilogue & kEpiGeluBwd) != 0;
   auto chunks = [&](auto stream) __attribute__((always_inline)) {
-#pragma unroll
+#pragma unroll 2
     for (int it = 0; it < TM * kCpr / kThreads; ++it) {
       const int e = it * kThreads + int(threadIdx.x);
       const int row = e / kCpr, cn = e % kCpr;
@@ -365,9 +365,12 @@ __device__ __attribute__((always_inline)) inline void store_staged(const TiledGe
       }
     }
   };
-  // one loop for each kind of store (8192 x 4096 x 1024 78 us, 81 with a branch
-  // at every store).  The empty statement keeps the loops' last stores apart,
-  // which the compiler would make one ordinary store of.
+  // one loop for each kind of store (a branch at every store costs 3 us in 80),
+  // unrolled twice: whole, the loops' code (the straddling chunk's columns, the
+  // GELUs) is 3 MB of the library; 8192 x 4096 x 1024 78 -> 71 us, 8192 x 6144 x
+  // 2048 196 -> 180, 4096 x 4096 x 4096 122 -> 117, 128-row tiles the same.  The
+  // empty statement keeps the loops' last stores apart, which the compiler would
+  // make one ordinary store of.
   if (p.stream_c) {
     chunks(std::true_type{});
     asm volatile("");
